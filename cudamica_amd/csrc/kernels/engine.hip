@@ -562,25 +562,31 @@ int amica_engine_whiten(amica_engine* e, int do_sphere) {
     /* scratch of the covariance and sphering partials, and of the FP8 channel maxima */
     const size_t partn = std::max(std::max((size_t)nchunks * n * n, (size_t)nchunks * 2 * n),
                                   (size_t)nchunks * e->NP);
+    double* ns = nullptr;
     HIPCHK(hipMalloc((void**)&part, partn * sizeof(double)));
     HIPCHK(hipMalloc((void**)&C, (size_t)n * n * sizeof(double)));
     HIPCHK(hipMalloc((void**)&V, (size_t)n * n * sizeof(double)));
     HIPCHK(hipMalloc((void**)&d, (size_t)n * sizeof(double)));
+    if (do_sphere == 1) HIPCHK(hipMalloc((void**)&ns, inv_sqrt_doubles(n) * sizeof(double)));
     int rc = 0;
     do {
+        bool have_S = false;
         if (do_sphere == 1) {
             if (launch_cov(e->xraw, e->mean, T, n, part, nchunks, C, e->st)) { rc = -1; break; }
-            if (launch_eigh(C, V, d, n, nullptr, e->st)) { rc = -1; break; }
+            const int conv = launch_inv_sqrt(C, n, e->S, e->ldetS_d, ns, e->st);
+            if (conv < 0) { rc = -1; break; }
+            have_S = conv == 0;
+            if (!have_S && launch_eigh(C, V, d, n, nullptr, e->st)) { rc = -1; break; }
         }
-        if (launch_sphere_matrix(V, d, C, n, e->xraw, e->mean, T, do_sphere, e->S, e->ldetS_d,
-                                 part, nchunks, e->st)) { rc = -1; break; }
+        if (!have_S && launch_sphere_matrix(V, d, C, n, e->xraw, e->mean, T, do_sphere, e->S, e->ldetS_d,
+                                            part, nchunks, e->st)) { rc = -1; break; }
         if (launch_whiten(e->xraw, e->mean, e->S, T, n, e->NP, e->xw, e->xw64, e->xbf, e->st)) { rc = -1; break; }
         if (e->x8 && !e->fp8 && launch_pack8(e->xbf, T, e->NP, e->x8, e->st)) { rc = -1; break; }
         if (e->fp8 && launch_quantize_fp8(e->xw, T, e->NP, e->xscale, e->xq, e->x8, (float*)part,
                                           nchunks, e->st)) { rc = -1; break; }
     } while (0);
     const hipError_t se = hipStreamSynchronize(e->st);
-    (void)hipFree(part); (void)hipFree(C); (void)hipFree(V); (void)hipFree(d);
+    (void)hipFree(part); (void)hipFree(C); (void)hipFree(V); (void)hipFree(d); (void)hipFree(ns);
     if (rc) return fail(AMICA_E_DEVICE, std::string("sphering launch failed: ") + hipGetErrorString(hipGetLastError()));
     if (se != hipSuccess) return fail(AMICA_E_DEVICE, std::string("sphering: ") + hipGetErrorString(se));
     HIPCHK(hipMemcpy(&e->ldetS, e->ldetS_d, sizeof(double), hipMemcpyDeviceToHost));

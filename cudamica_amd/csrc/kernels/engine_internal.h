@@ -231,6 +231,11 @@ int launch_colmean(const float* x, long T, int n, double* part, int nchunks, dou
                    hipStream_t st);
 int launch_cov(const float* x, const double* mean, long T, int n, double* part, int nchunks,
                double* C, hipStream_t st);
+/* S = 2 C^-1/2 and ldetS = -log|det S| by Newton-Schulz products; ws holds
+ * inv_sqrt_doubles(n) doubles.  Synchronises st to read the convergence; 1
+ * where C is too ill-conditioned for it (S is then not written). */
+size_t inv_sqrt_doubles(int n);
+int launch_inv_sqrt(const double* C, int n, double* S, double* ldetS, double* ws, hipStream_t st);
 int launch_eigh(double* C, double* V, double* d, int n, double* work, hipStream_t st);
 int launch_sphere_matrix(const double* V, const double* d, const double* C, int n,
                          const float* x, const double* mean, long T, int do_sphere,
