@@ -530,10 +530,9 @@ int amica_engine_center(amica_engine* e) {
     HIPCHK(hipSetDevice(e->o.device));
     const int n = e->o.n;
     const long T = e->o.T;
-    const int nchunks = (int)std::max(1L, std::min((long)e->cus * 2, T / 64 + 1));
     double* part = nullptr;
-    HIPCHK(hipMalloc((void**)&part, (size_t)nchunks * n * sizeof(double)));
-    const int rc = launch_colmean(e->xraw, T, n, part, nchunks, e->mean, e->st);
+    HIPCHK(hipMalloc((void**)&part, sphere_part_doubles(T, n, e->cus) * sizeof(double)));
+    const int rc = launch_colmean(e->xraw, T, n, part, e->cus, e->mean, e->st);
     const hipError_t se = hipStreamSynchronize(e->st);
     (void)hipFree(part);
     if (rc) return fail(AMICA_E_DEVICE, "centering launch failed");
@@ -560,7 +559,7 @@ int amica_engine_whiten(amica_engine* e, int do_sphere) {
     const int nchunks = (int)std::max(1L, std::min((long)e->cus * 2, T / 64 + 1));
     double *part = nullptr, *C = nullptr, *V = nullptr, *d = nullptr;
     /* scratch of the covariance and sphering partials, and of the FP8 channel maxima */
-    const size_t partn = std::max(std::max((size_t)nchunks * n * n, (size_t)nchunks * 2 * n),
+    const size_t partn = std::max(std::max(sphere_part_doubles(T, n, e->cus), (size_t)nchunks * 2 * n),
                                   (size_t)nchunks * e->NP);
     double* ns = nullptr;
     HIPCHK(hipMalloc((void**)&part, partn * sizeof(double)));
@@ -572,7 +571,7 @@ int amica_engine_whiten(amica_engine* e, int do_sphere) {
     do {
         bool have_S = false;
         if (do_sphere == 1) {
-            if (launch_cov(e->xraw, e->mean, T, n, part, nchunks, C, e->st)) { rc = -1; break; }
+            if (launch_cov(e->xraw, e->mean, T, n, part, e->cus, C, e->st)) { rc = -1; break; }
             const int conv = launch_inv_sqrt(C, n, e->S, e->ldetS_d, ns, e->st);
             if (conv < 0) { rc = -1; break; }
             have_S = conv == 0;
@@ -580,8 +579,8 @@ int amica_engine_whiten(amica_engine* e, int do_sphere) {
         }
         if (!have_S && launch_sphere_matrix(V, d, C, n, e->xraw, e->mean, T, do_sphere, e->S, e->ldetS_d,
                                             part, nchunks, e->st)) { rc = -1; break; }
-        if (launch_whiten(e->xraw, e->mean, e->S, T, n, e->NP, e->xw, e->xw64, e->xbf, e->st)) { rc = -1; break; }
-        if (e->x8 && !e->fp8 && launch_pack8(e->xbf, T, e->NP, e->x8, e->st)) { rc = -1; break; }
+        if (launch_whiten(e->xraw, e->mean, e->S, T, n, e->NP, e->xw, e->xw64, e->xbf, e->fp8 ? nullptr : e->x8,
+                          e->st)) { rc = -1; break; }
         if (e->fp8 && launch_quantize_fp8(e->xw, T, e->NP, e->xscale, e->xq, e->x8, (float*)part,
                                           nchunks, e->st)) { rc = -1; break; }
     } while (0);

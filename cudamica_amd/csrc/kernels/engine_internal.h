@@ -227,10 +227,11 @@ int launch_gj_inverse(const double* A, double* Ainv, double* ldet_inv, int n, in
                       hipStream_t st);
 
 /* Preprocessing -------------------------------------------------------------- */
-int launch_colmean(const float* x, long T, int n, double* part, int nchunks, double* mean,
-                   hipStream_t st);
-int launch_cov(const float* x, const double* mean, long T, int n, double* part, int nchunks,
-               double* C, hipStream_t st);
+/* doubles of scratch (part) the column means and the covariance use */
+size_t sphere_part_doubles(long T, int n, int cus);
+int launch_colmean(const float* x, long T, int n, double* part, int cus, double* mean, hipStream_t st);
+int launch_cov(const float* x, const double* mean, long T, int n, double* part, int cus, double* C,
+               hipStream_t st);
 /* S = 2 C^-1/2 and ldetS = -log|det S| by Newton-Schulz products; ws holds
  * inv_sqrt_doubles(n) doubles.  Synchronises st to read the convergence; 1
  * where C is too ill-conditioned for it (S is then not written). */
@@ -241,10 +242,11 @@ int launch_sphere_matrix(const double* V, const double* d, const double* C, int 
                          const float* x, const double* mean, long T, int do_sphere,
                          double* S, double* ldetS_out, double* part, int nchunks,
                          hipStream_t st);
-/* x_white = S (x - mean): float32 copy xw, optional FP64 copy xw64 and bf16
- * copy xbf, all [T][NP] with zero padding. */
+/* x_white = S (x - mean): float32 copy xw, optional FP64 copy xw64 and split
+ * bf16 copy xbf, all [T][NP] with zero padding, and optional x8, the bf16 hi
+ * part packed as by launch_pack8. */
 int launch_whiten(const float* x, const double* mean, const double* S, long T, int n, int NP,
-                  float* xw, double* xw64, uint16_t* xbf, hipStream_t st);
+                  float* xw, double* xw64, uint16_t* xbf, uint16_t* x8, hipStream_t st);
 int launch_white_from_f64(const double* xin, long T, int n, int NP, float* xw, double* xw64,
                           uint16_t* xbf, hipStream_t st);
 int launch_bf16_from_f32(const float* x, size_t count, uint16_t* out, hipStream_t st);

@@ -23,86 +23,180 @@ namespace amica {
 
 namespace {
 
-/* per-chunk FP64 column sums of x (T x n float32) */
+/* per-chunk FP64 column sums of x (T x n float32), 256 columns per
+ * blockIdx.y: the workgroup's threads cover as many whole rows at once as fit
+ * (consecutive addresses), kRowUnroll passes of loads in flight, and the rows'
+ * sums meet in LDS in a fixed order.  Bound by the read of x: 0.13 ms at
+ * 128 ch x 1M, 4.0 TB/s (0.82 ms with one thread per column, which left half
+ * the workgroup idle and one load in flight). */
+constexpr int kRowUnroll = 8;
+
 __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ x, long T, int n,
                                                      long chunk, double* __restrict__ part) {
+    __shared__ double red[256];
     const long ts = (long)blockIdx.x * chunk, te = min(T, ts + chunk);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        double s = 0.0;
-        for (long t = ts; t < te; ++t) s += (double)x[(size_t)t * n + i];
+    const int c0 = blockIdx.y * 256, cols = min(256, n - c0), rows = 256 / cols;
+    const int tid = threadIdx.x, r = tid / cols, i = c0 + tid - r * cols;
+    double s = 0.0;
+    if (r < rows) {
+        long t = ts + r;
+        for (; t + (long)(kRowUnroll - 1) * rows < te; t += (long)kRowUnroll * rows) {
+            float v[kRowUnroll];
+#pragma unroll
+            for (int u = 0; u < kRowUnroll; ++u) v[u] = x[(size_t)(t + (long)u * rows) * n + i];
+#pragma unroll
+            for (int u = 0; u < kRowUnroll; ++u) s += (double)v[u];
+        }
+        for (; t < te; t += rows) s += (double)x[(size_t)t * n + i];
+    }
+    red[tid] = s;
+    __syncthreads();
+    if (tid < cols) {
+        for (int q = 1; q < rows; ++q) s += red[q * cols + tid];
         part[(size_t)blockIdx.x * n + i] = s;
     }
 }
 
-__global__ void finish_mean_kernel(const double* __restrict__ part, int nchunks, int n, long T,
-                                   double* __restrict__ mean) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+/* Fixed-order totals of per-chunk partials: 64 entries (lanes) per workgroup,
+ * wave w takes the chunks w, w + 16, ..., the waves' sums are added in order. */
+__device__ __forceinline__ double chunk_total(const double* __restrict__ part, int nchunks, size_t stride,
+                                              size_t e, bool valid) {
+    __shared__ double red[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     double s = 0.0;
-    for (int c = 0; c < nchunks; ++c) s += part[(size_t)c * n + i];
-    mean[i] = s / (double)T;
+    if (valid) {
+#pragma unroll 4
+        for (int c = w; c < nchunks; c += 16) s += part[(size_t)c * stride + e];
+    }
+    red[w][lane] = s;
+    __syncthreads();
+    double t = 0.0;
+    if (w == 0)
+        for (int q = 0; q < 16; ++q) t += red[q][lane];
+    return t;
 }
 
-/* C tile [ib, ib+64) x [kb, kb+64) summed over one chunk of samples.  Each
- * of the 256 threads owns a 4 x 4 block of the tile; 32 centred samples are
- * staged in LDS per step. */
-__global__ __launch_bounds__(256) void cov_kernel(const float* __restrict__ x,
+__global__ __launch_bounds__(1024) void finish_mean_kernel(const double* __restrict__ part, int nchunks, int n,
+                                                           long T, double* __restrict__ mean) {
+    const int i = blockIdx.x * 64 + (threadIdx.x & 63);
+    const double s = chunk_total(part, nchunks, n, i, i < n);
+    if (threadIdx.x < 64 && i < n) mean[i] = s / (double)T;
+}
+
+/* Upper triangle of the covariance over one chunk of samples: blockIdx.y is
+ * the pair (bi <= bk) of 16 TI-channel blocks, each of the four waves takes
+ * every fourth group of kU 4-sample steps, TI x TI FP64 MFMA tiles; their sums
+ * meet in LDS in wave order.  Fragments are loaded straight from x (lane
+ * (i, k) = channel l % 16, sample l / 16: 64-byte runs), kU steps ahead of
+ * their use, and centred in registers, so that nothing but the sums goes
+ * through LDS.  Bound by the FP64 MFMA rate (64 cycles per 1024 FMAs), and
+ * only one triangle is formed: 0.57 ms at 128 ch x 1M, 1.86 ms at 256 ch (44
+ * TFLOP/s of 73; 1.31 ms for both triangles by FMAs from LDS at 128 ch). */
+template <int TI>
+__global__ __launch_bounds__(256, 2) void cov_kernel(const float* __restrict__ x,
                                                   const double* __restrict__ mean, long T, int n,
-                                                  long chunk, double* __restrict__ part) {
-    __shared__ double xa[32][64];
-    __shared__ double xb[32][64];
-    const int tid = threadIdx.x;
-    const int ib = blockIdx.y * 64, kb = blockIdx.z * 64;
+                                                  long chunk, int nblk, double* __restrict__ part) {
+    constexpr int W = 16 * TI, kU = TI == 4 ? 2 : 4;
+    __shared__ double sum[TI * TI][256];
+    int bi = 0, bk = (int)blockIdx.y;
+    while (bk >= nblk - bi) { bk -= nblk - bi; ++bi; }
+    bk += bi;
+    const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, kq = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool diag = bi == bk;                          /* block-uniform */
     const long ts = (long)blockIdx.x * chunk, te = min(T, ts + chunk);
-    const int ti = (tid & 15) * 4, tk = (tid >> 4) * 4;
-    double acc[4][4];
+    int ci[TI], ck[TI];
+    double mi[TI], mk[TI];
+    bool vi[TI], vk[TI];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int p = 0; p < TI; ++p) {
+        const int i = bi * W + 16 * p + l15, k = bk * W + 16 * p + l15;
+        vi[p] = i < n;
+        vk[p] = k < n;
+        ci[p] = vi[p] ? i : n - 1;
+        ck[p] = vk[p] ? k : n - 1;
+        mi[p] = mean[ci[p]];
+        mk[p] = mean[ck[p]];
+    }
+    f64x4 acc[TI][TI];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-    for (long t0 = ts; t0 < te; t0 += 32) {
-        for (int q = tid; q < 32 * 64; q += 256) {
-            const int s = q >> 6, c = q & 63;
-            const long t = t0 + s;
-            double va = 0.0, vb = 0.0;
-            if (t < te) {
-                if (ib + c < n) va = (double)x[(size_t)t * n + ib + c] - mean[ib + c];
-                if (kb + c < n) vb = (double)x[(size_t)t * n + kb + c] - mean[kb + c];
+    for (int p = 0; p < TI; ++p)
+#pragma unroll
+        for (int q = 0; q < TI; ++q) acc[p][q] = (f64x4){0.0, 0.0, 0.0, 0.0};
+    float fa[kU][TI], fb[kU][TI];
+    auto load = [&](long t0) {
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const long t = t0 + 4 * u + kq;
+            const float* row = x + (size_t)(t < te ? t : te - 1) * n;
+#pragma unroll
+            for (int p = 0; p < TI; ++p) {
+                fa[u][p] = row[ci[p]];
+                if (!diag) fb[u][p] = row[ck[p]];
             }
-            xa[s][c] = va;
-            xb[s][c] = vb;
         }
-        __syncthreads();
-        for (int s = 0; s < 32; ++s) {
-            double av[4], bv[4];
+    };
+    const long step = 4 * 4 * kU;
+    long t0 = ts + (long)w * 4 * kU;
+    if (t0 < te) load(t0);
+    for (; t0 < te; t0 += step) {
+        double a[kU][TI], b[kU][TI];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) av[a] = xa[s][ti + a];
+        for (int u = 0; u < kU; ++u) {
+            const bool ok = t0 + 4 * u + kq < te;
 #pragma unroll
-            for (int b = 0; b < 4; ++b) bv[b] = xb[s][tk + b];
+            for (int p = 0; p < TI; ++p) {
+                a[u][p] = ok && vi[p] ? (double)fa[u][p] - mi[p] : 0.0;
+                b[u][p] = diag ? a[u][p] : (ok && vk[p] ? (double)fb[u][p] - mk[p] : 0.0);
+            }
+        }
+        if (t0 + step < te) load(t0 + step);
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+        for (int u = 0; u < kU; ++u)
 #pragma unroll
-                for (int b = 0; b < 4; ++b) acc[a][b] = fma(av[a], bv[b], acc[a][b]);
+            for (int p = 0; p < TI; ++p)
+#pragma unroll
+                for (int q = 0; q < TI; ++q)
+                    acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][p], b[u][q], acc[p][q], 0, 0, 0);
+    }
+    /* register r of lane l: row l / 16 + 4 r, column l % 16 */
+    for (int v = 0; v < 4; ++v) {
+        if (v == w) {
+#pragma unroll
+            for (int p = 0; p < TI; ++p)
+#pragma unroll
+                for (int q = 0; q < TI; ++q)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        double* s = &sum[p * TI + q][l15 * 16 + kq + 4 * r];
+                        *s = v == 0 ? acc[p][q][r] : *s + acc[p][q][r];
+                    }
         }
         __syncthreads();
     }
-    double* out = part + (size_t)blockIdx.x * n * n;
+    double* out = part + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * (W * W);
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int i = ib + ti + a, k = kb + tk + b;
-            if (i < n && k < n) out[i + (size_t)k * n] = acc[a][b];
-        }
+    for (int t = 0; t < TI * TI; ++t) out[t * 256 + tid] = sum[t][tid];
 }
 
-__global__ void finish_cov_kernel(const double* __restrict__ part, int nchunks, int n, long T,
-                                  double* __restrict__ C) {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)n * n) return;
-    double s = 0.0;
-    for (int c = 0; c < nchunks; ++c) s += part[(size_t)c * n * n + e];
-    C[e] = s / (double)T;
+/* C from the chunks' block pairs, mirrored: entry e = (pair, tile, row and
+ * column) of the layout above */
+__global__ __launch_bounds__(1024) void finish_cov_kernel(const double* __restrict__ part, int nchunks, int n,
+                                                          int TI, int nblk, int npairs, long T,
+                                                          double* __restrict__ C) {
+    const int W = 16 * TI;
+    const size_t len = (size_t)npairs * W * W, e = (size_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    const double s = chunk_total(part, nchunks, len, e, e < len);
+    if (threadIdx.x >= 64 || e >= len) return;
+    int bk = (int)(e / (W * W)), bi = 0;
+    const int f = (int)(e % (W * W));
+    while (bk >= nblk - bi) { bk -= nblk - bi; ++bi; }
+    bk += bi;
+    const int t = f >> 8, g = f & 255;
+    const int i = bi * W + (t / TI) * 16 + (g & 15), k = bk * W + (t % TI) * 16 + (g >> 4);
+    if (i >= n || k >= n) return;
+    C[i + (size_t)k * n] = s / (double)T;
+    if (bi != bk) C[k + (size_t)i * n] = s / (double)T;
 }
 
 /* Parallel cyclic Jacobi (Brent-Luk round-robin ordering): each round
@@ -199,8 +293,9 @@ __global__ __launch_bounds__(256) void eigh_kernel(double* __restrict__ A, doubl
  * Z Y^T it is not: the skew part of the rounding errors grows).  Against
  * 80-bit results its error is 0.2 .. 0.8 of the Jacobi eigensolver's for
  * condition numbers of C from 1e2 to 1e8.  Bound by the latency of its
- * dependent products: 16 iterations of two launches replace ~9 sweeps of
- * n - 1 barrier-separated rounds in one workgroup. */
+ * dependent products: 14 to 19 iterations of two 5 us launches (7 + 11 us at
+ * 256 channels) replace ~9 sweeps of n - 1 barrier-separated rounds in one
+ * workgroup: 46 ms -> 0.2 ms at 128 channels, 356 ms -> 0.5 ms at 260. */
 
 /* scal[0] = |C|_F (one workgroup) and the residual slots cleared */
 constexpr int kNsSlots = 32;
@@ -400,31 +495,143 @@ __device__ __forceinline__ void store_split_bf16(uint16_t* xbf, size_t lo_ofs, s
     xbf[lo_ofs + e] = f32_to_bf16_bits(f - bf16_bits_to_f32(hi));
 }
 
-__global__ __launch_bounds__(256) void whiten_kernel(const float* __restrict__ x,
-                                                     const double* __restrict__ mean,
-                                                     const double* __restrict__ S, long T, int n,
-                                                     int NP, int TS, float* __restrict__ xw,
-                                                     double* __restrict__ xw64,
-                                                     uint16_t* __restrict__ xbf) {
-    extern __shared__ double xc[];
+/* A workgroup takes 16 RT WR samples x all channels: x is staged in LDS as it
+ * is (float32, rows of stride = 4 mod 64 words: the 64 lanes of an A fragment
+ * hit 64 banks), centred in FP64 as the fragments are read, and multiplied by
+ * S from L2 on the FP64 MFMA units; wave (wr, wc) forms the 16 RT samples wr x
+ * the 64-channel groups wc, wc + WC, ...  A wave's results pass through its
+ * own LDS tile of 16 samples so that every copy -- float32, split bf16, bf16
+ * packed by 8 samples -- leaves in 16-byte stores and the packed copy needs no
+ * pass of its own.  Bound by the FP64 MFMA rate (2 n per value) and its
+ * stores: 1.12 ms at 128 ch x 1M, 3.0 ms at 256 ch (44 TFLOP/s; 7.6 and 27 ms
+ * with one thread per value, S from L2, and 0.18 ms more for the packing). */
+struct WhitenArgs {
+    const float* x;
+    const double* mean;
+    const double* S;
+    long T;
+    int n, NP, WR, WC;
+    float* xw;
+    double* xw64;
+    uint16_t* xbf;
+    uint16_t* x8;
+};
+
+constexpr int kWhitenRow = 68;                 /* floats per row of a wave's LDS tile */
+constexpr int kWhitenRT = 2;                   /* 16-sample tiles per wave: 4 leave one workgroup per CU */
+
+__global__ __launch_bounds__(512) void whiten_kernel(WhitenArgs a) {
+    constexpr int RT = kWhitenRT;
+    extern __shared__ __align__(16) float wlds[];
+    const int n = a.n, NP = a.NP, stride = NP + 4, K4 = (n + 3) / 4;
+    const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, kq = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
+    const int wr = w / a.WC, wc = w - wr * a.WC;
+    const int TS = 16 * RT * a.WR;
+    float* xs = wlds;                                              /* [TS][stride] */
+    double* ms = (double*)(wlds + (size_t)TS * stride);            /* [NP] */
+    float* tile = (float*)(ms + NP) + w * 16 * kWhitenRow;         /* [16][kWhitenRow] */
     const long t0 = (long)blockIdx.x * TS;
-    for (int q = threadIdx.x; q < TS * n; q += blockDim.x) {
-        const int s = q / n, k = q % n;
-        const long t = t0 + s;
-        xc[q] = (t < T) ? (double)x[(size_t)t * n + k] - mean[k] : 0.0;
-    }
+    for (int s = w; s < TS; s += nw)
+        for (int k = lane; k < 4 * K4; k += 64)
+            xs[s * stride + k] = (t0 + s < a.T && k < n) ? a.x[(size_t)(t0 + s) * n + k] : 0.f;
+    for (int k = tid; k < NP; k += blockDim.x) ms[k] = k < n ? a.mean[k] : 0.0;
     __syncthreads();
-    for (int q = threadIdx.x; q < TS * NP; q += blockDim.x) {
-        const int s = q / NP, i = q % NP;
-        const long t = t0 + s;
-        if (t >= T) continue;
-        double v = 0.0;
-        if (i < n)
-            for (int k = 0; k < n; ++k) v += S[i + (long)k * n] * xc[s * n + k];
-        const float f = (float)v;
-        xw[(size_t)t * NP + i] = f;
-        if (xw64) xw64[(size_t)t * NP + i] = v;
-        if (xbf) store_split_bf16(xbf, (size_t)T * NP, (size_t)t * NP + i, f);
+    const long tw = t0 + (long)wr * 16 * RT;
+    const float* xa = xs + (wr * 16 * RT + l15) * stride + kq;
+    for (int cg = wc; cg < NP / 64; cg += a.WC) {
+        f64x4 acc[RT][4];
+#pragma unroll
+        for (int p = 0; p < RT; ++p)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[p][q] = (f64x4){0.0, 0.0, 0.0, 0.0};
+        /* past the last row and column the loads repeat it: x - mean is 0
+         * there, and the padding channels are cleared on the way out */
+        const double* Sc[4];
+        bool vc[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int c = cg * 64 + 16 * q + l15;
+            vc[q] = c < n;
+            Sc[q] = a.S + min(c, n - 1);
+        }
+        double bn[4];
+        auto loadS = [&](int s) {
+            const size_t k = (size_t)min(4 * s + kq, n - 1) * n;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) bn[q] = Sc[q][k];
+        };
+        loadS(0);
+#pragma unroll 2
+        for (int s = 0; s < K4; ++s) {
+            double bc[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) bc[q] = bn[q];
+            loadS(s + 1);                      /* past the end: the last row again */
+            const double mk = ms[4 * s + kq];
+#pragma unroll
+            for (int p = 0; p < RT; ++p) {
+                const double av = (double)xa[p * 16 * stride + 4 * s] - mk;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bc[q], acc[p][q], 0, 0, 0);
+            }
+        }
+        /* register r of lane l: sample l / 16 + 4 r, channel l % 16 */
+#pragma unroll
+        for (int p = 0; p < RT; ++p) {
+            const long tp = tw + 16 * p;
+            if (tp >= a.T) continue;                               /* wave-uniform */
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int s = kq + 4 * r;
+                    const double v = vc[q] ? acc[p][q][r] : 0.0;
+                    if (a.xw64 && tp + s < a.T)
+                        a.xw64[(size_t)(tp + s) * NP + cg * 64 + 16 * q + l15] = v;
+                    tile[s * kWhitenRow + 16 * q + l15] = tp + s < a.T ? (float)v : 0.f;
+                }
+            __builtin_amdgcn_wave_barrier();
+            {
+                const int s = lane >> 2, c = (lane & 3) * 16;      /* 16 channels of one sample */
+                const float4* src = (const float4*)(tile + s * kWhitenRow + c);
+                if (tp + s < a.T) {
+                    float4* dst = (float4*)(a.xw + (size_t)(tp + s) * NP + cg * 64 + c);
+                    float f[16];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const float4 v = src[u];
+                        dst[u] = v;
+                        f[4 * u] = v.x; f[4 * u + 1] = v.y; f[4 * u + 2] = v.z; f[4 * u + 3] = v.w;
+                    }
+                    if (a.xbf) {
+                        __align__(16) uint16_t hi[16], lo[16];
+#pragma unroll
+                        for (int u = 0; u < 16; ++u) {
+                            hi[u] = f32_to_bf16_bits(f[u]);
+                            lo[u] = f32_to_bf16_bits(f[u] - bf16_bits_to_f32(hi[u]));
+                        }
+                        const size_t e = (size_t)(tp + s) * NP + cg * 64 + c;
+                        uint4* dh = (uint4*)(a.xbf + e);
+                        uint4* dl = (uint4*)(a.xbf + (size_t)a.T * NP + e);
+                        dh[0] = ((const uint4*)hi)[0]; dh[1] = ((const uint4*)hi)[1];
+                        dl[0] = ((const uint4*)lo)[0]; dl[1] = ((const uint4*)lo)[1];
+                    }
+                }
+            }
+            if (a.x8) {                                            /* lane = channel */
+#pragma unroll
+                for (int gr = 0; gr < 2; ++gr) {
+                    if (tp + 8 * gr >= a.T) continue;              /* wave-uniform */
+                    __align__(16) uint16_t h[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) h[u] = f32_to_bf16_bits(tile[(8 * gr + u) * kWhitenRow + lane]);
+                    *(uint4*)(a.x8 + ((size_t)((tp >> 3) + gr) * NP + cg * 64 + lane) * 8) = *(const uint4*)h;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
     }
 }
 
@@ -529,23 +736,47 @@ long chunk_of(long T, int nchunks) { return (T + nchunks - 1) / nchunks; }
 
 }  // namespace
 
-int launch_colmean(const float* x, long T, int n, double* part, int nchunks, double* mean,
-                   hipStream_t st) {
-    hipLaunchKernelGGL(colsum_kernel, dim3(nchunks), dim3(256), 0, st, x, T, n,
-                       chunk_of(T, nchunks), part);
-    hipLaunchKernelGGL(finish_mean_kernel, dim3((n + 255) / 256), dim3(256), 0, st, part, nchunks,
-                       n, T, mean);
+/* chunks of the column sums: about eight workgroups per CU, at least 256 samples each */
+static int mean_chunks(long T, int cus) { return (int)std::max(1L, std::min(8L * cus, T / 256)); }
+
+/* channel blocks of 16 TI, their pairs, and chunks for about two workgroups
+ * per CU in all (each wave holds one SIMD's MFMA pipe busy), at least 256 samples each */
+static void cov_shape(long T, int n, int cus, int* TI, int* nblk, int* npairs, int* nchunks) {
+    *TI = std::min(4, (n + 15) / 16);
+    if (*TI == 3) *TI = 4;
+    *nblk = (n + 16 * *TI - 1) / (16 * *TI);
+    *npairs = *nblk * (*nblk + 1) / 2;
+    *nchunks = (int)std::max(1L, std::min(2L * cus / *npairs, T / 256));
+}
+
+size_t sphere_part_doubles(long T, int n, int cus) {
+    int TI, nblk, npairs, nchunks;
+    cov_shape(T, n, cus, &TI, &nblk, &npairs, &nchunks);
+    return std::max((size_t)nchunks * npairs * 256 * TI * TI, (size_t)mean_chunks(T, cus) * n);
+}
+
+int launch_colmean(const float* x, long T, int n, double* part, int cus, double* mean, hipStream_t st) {
+    const int nc = mean_chunks(T, cus);
+    const long chunk = chunk_of(T, nc);
+    const int used = (int)((T + chunk - 1) / chunk);
+    hipLaunchKernelGGL(colsum_kernel, dim3(used, (n + 255) / 256), dim3(256), 0, st, x, T, n, chunk, part);
+    hipLaunchKernelGGL(finish_mean_kernel, dim3((n + 63) / 64), dim3(1024), 0, st, part, used, n, T, mean);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int launch_cov(const float* x, const double* mean, long T, int n, double* part, int nchunks,
-               double* C, hipStream_t st) {
-    const int nt = (n + 63) / 64;
-    hipLaunchKernelGGL(cov_kernel, dim3(nchunks, nt, nt), dim3(256), 0, st, x, mean, T, n,
-                       chunk_of(T, nchunks), part);
-    const size_t nn = (size_t)n * n;
-    hipLaunchKernelGGL(finish_cov_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st,
-                       part, nchunks, n, T, C);
+int launch_cov(const float* x, const double* mean, long T, int n, double* part, int cus, double* C,
+               hipStream_t st) {
+    int TI, nblk, npairs, nchunks;
+    cov_shape(T, n, cus, &TI, &nblk, &npairs, &nchunks);
+    const long chunk = chunk_of(T, nchunks);
+    nchunks = (int)((T + chunk - 1) / chunk);
+    const dim3 grid(nchunks, npairs), blk(256);
+    if (TI == 1) hipLaunchKernelGGL(cov_kernel<1>, grid, blk, 0, st, x, mean, T, n, chunk, nblk, part);
+    else if (TI == 2) hipLaunchKernelGGL(cov_kernel<2>, grid, blk, 0, st, x, mean, T, n, chunk, nblk, part);
+    else hipLaunchKernelGGL(cov_kernel<4>, grid, blk, 0, st, x, mean, T, n, chunk, nblk, part);
+    const size_t len = (size_t)npairs * 256 * TI * TI;
+    hipLaunchKernelGGL(finish_cov_kernel, dim3((unsigned)((len + 63) / 64)), dim3(1024), 0, st, part, nchunks, n,
+                       TI, nblk, npairs, T, C);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -633,12 +864,17 @@ int launch_sphere_matrix(const double* V, const double* d, const double* C, int 
 }
 
 int launch_whiten(const float* x, const double* mean, const double* S, long T, int n, int NP,
-                  float* xw, double* xw64, uint16_t* xbf, hipStream_t st) {
-    int TS = 4096 / n;
-    if (TS < 1) TS = 1;
-    const size_t shm = (size_t)TS * n * sizeof(double);
-    hipLaunchKernelGGL(whiten_kernel, dim3((unsigned)((T + TS - 1) / TS)), dim3(256), shm, st, x,
-                       mean, S, T, n, NP, TS, xw, xw64, xbf);
+                  float* xw, double* xw64, uint16_t* xbf, uint16_t* x8, hipStream_t st) {
+    /* one wave per 64-channel group up to eight (four where the LDS tiles of
+     * eight would not fit beside the rows), four waves at least */
+    const int WC = NP <= 768 ? std::min(NP / 64, 8) : 4, WR = std::max(1, 4 / WC);
+    const int TS = 16 * kWhitenRT * WR;
+    const size_t shm = (size_t)TS * (NP + 4) * sizeof(float) + NP * sizeof(double) +
+                       (size_t)WR * WC * 16 * kWhitenRow * sizeof(float);
+    const WhitenArgs a = {x, mean, S, T, n, NP, WR, WC, xw, xw64, xbf, x8};
+    if (hipFuncSetAttribute((const void*)whiten_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm) != hipSuccess) return -1;
+    const dim3 grid((unsigned)((T + TS - 1) / TS)), blk(64 * WR * WC);
+    hipLaunchKernelGGL(whiten_kernel, grid, blk, shm, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

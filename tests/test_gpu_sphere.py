@@ -25,7 +25,7 @@ def _recording(n, T, cond, seed):
 @pytest.mark.parametrize("n,T,cond", [(1, 50, 1.0), (2, 64, 10.0), (15, 1000, 1e2), (16, 1025, 1e3),
                                       (17, 2049, 1e4), (63, 3001, 1e4), (64, 4096, 1e6), (65, 4099, 1e2),
                                       (130, 5003, 1e4), (192, 6000, 1e2), (193, 6007, 1e3), (260, 9001, 1e4),
-                                      (300, 9000, 1e2), (32, 4000, 1e11)])
+                                      (300, 9000, 1e2), (704, 3000, 1e2), (1024, 4100, 1e1), (32, 4000, 1e11)])
 def test_sphering_against_numpy(built, n, T, cond):
     print(f"[sphere] n={n} T={T} cond={cond:g}", flush=True)
     x = _recording(n, T, cond, 17 * n + T)
