@@ -834,18 +834,18 @@ int amica_engine_output(amica_engine* e, double* A_out, double* c_out) {
     HIPCHK(hipSetDevice(e->o.device));
     const int n = e->o.n, M = e->o.M;
     const size_t nn = (size_t)n * n;
-    double *lu = nullptr, *Sinv = nullptr, *Ao = nullptr, *co = nullptr;
-    HIPCHK(hipMalloc((void**)&lu, 2 * nn * sizeof(double)));
+    double *work = nullptr, *Sinv = nullptr, *Ao = nullptr, *co = nullptr;
+    HIPCHK(hipMalloc((void**)&work, (16 + nn + inverse_work_doubles(n, 1)) * sizeof(double)));
     HIPCHK(hipMalloc((void**)&Sinv, nn * sizeof(double)));
     HIPCHK(hipMalloc((void**)&Ao, M * nn * sizeof(double)));
     HIPCHK(hipMalloc((void**)&co, (size_t)M * n * sizeof(double)));
-    int rc = launch_output_transform(e->S, e->mean, e->A, e->c, n, M, lu, Sinv, Ao, co, e->st);
+    int rc = launch_output_transform(e->S, e->mean, e->A, e->c, n, M, work, Sinv, Ao, co, e->st);
     hipError_t se = hipStreamSynchronize(e->st);
     if (!rc && se == hipSuccess) {
         se = hipMemcpy(A_out, Ao, M * nn * sizeof(double), hipMemcpyDeviceToHost);
         if (se == hipSuccess) se = hipMemcpy(c_out, co, (size_t)M * n * sizeof(double), hipMemcpyDeviceToHost);
     }
-    (void)hipFree(lu); (void)hipFree(Sinv); (void)hipFree(Ao); (void)hipFree(co);
+    (void)hipFree(work); (void)hipFree(Sinv); (void)hipFree(Ao); (void)hipFree(co);
     if (rc || se != hipSuccess) return fail(AMICA_E_DEVICE, "output transform failed");
     return 0;
 }

@@ -255,9 +255,10 @@ int launch_bf16_from_f32(const float* x, size_t count, uint16_t* out, hipStream_
  * packed 8 samples per channel. */
 int launch_quantize_fp8(float* xw, long T, int NP, float* scale, uint8_t* xq, uint16_t* x8,
                         float* part, int nchunks, hipStream_t st);
-/* Sinv = S^-1 (LU), A_out = colnorm(Sinv A_h), c_out = Sinv c_h + mean. */
+/* Sinv = S^-1, A_out = colnorm(Sinv A_h), c_out = Sinv c_h + mean; work holds
+ * 16 + n n + inverse_work_doubles(n, 1) doubles. */
 int launch_output_transform(const double* S, const double* mean, const double* A,
-                            const double* c, int n, int M, double* lu, double* Sinv,
+                            const double* c, int n, int M, double* work, double* Sinv,
                             double* A_out, double* c_out, hipStream_t st);
 
 }  // namespace amica

@@ -50,3 +50,27 @@ def test_sphering_against_numpy(built, n, T, cond):
     # whitened data: FP64 products rounded to float32 once
     ref = (xd - mean) @ Sg.T
     np.testing.assert_allclose(w, ref, rtol=2e-7, atol=1e-12 * np.abs(ref).max() + 1e-30)
+
+
+@pytest.mark.parametrize("n,M", [(1, 1), (16, 2), (17, 3), (65, 1), (193, 2), (260, 5)])
+def test_output_transform_against_numpy(built, n, M):
+    print(f"[output] n={n} M={M}", flush=True)
+    T = 20 * n + 50
+    x = _recording(n, T, 1e2, 31 * n + M)
+    st = ca.synth_init(n, M, 2, n + M)
+    with ca.Engine(ca.options(n, T, M, 2)) as eng:
+        eng.load_raw(x)
+        eng.preprocess(1)
+        eng.set_state(st)
+        S, mean, _ = eng.sphere()
+        A, c = eng.output()
+    Sinv = np.linalg.inv(S.reshape(n, n).T)
+    # two inverses of S, each off by at most ~n eps cond(S)
+    tol = 8.0 * n * EPS * np.linalg.cond(S.reshape(n, n)) + 1e-14
+    for h in range(M):
+        ref = Sinv @ st["A"].reshape(M, n, n)[h].T
+        ref /= np.linalg.norm(ref, axis=0)
+        got = A.reshape(M, n, n)[h].T
+        assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref)
+        ref = Sinv @ st["c"].reshape(M, n)[h] + mean
+        assert np.linalg.norm(c.reshape(M, n)[h] - ref) <= tol * (np.linalg.norm(Sinv) * np.sqrt(n) + np.linalg.norm(ref))
