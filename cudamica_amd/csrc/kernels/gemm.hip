@@ -694,7 +694,10 @@ __global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restric
     const int S = ldb < 512 ? max(1, (int)(blockDim.x >> 6) / rw) : 1;
     const int sr = w / rw, wr = w - sr * rw;
     const int r0 = blockIdx.z * 512 + wr * 64;     /* grid.z: groups of 512 g columns */
-    if (S == 1 && r0 >= ldb) return;                /* no barriers below when S = 1 */
+    /* the last group of 512 columns may have fewer rows than the workgroup has
+     * waves: the others would write zeros over its partial (no barriers below
+     * when S = 1) */
+    if (S == 1 && w >= rw) return;
     const int k0 = blockIdx.y * 16 * CT;
     long ts = (long)blockIdx.x * chunk;
     long te = min(T, ts + chunk);
@@ -826,7 +829,10 @@ __device__ __forceinline__ void gx_bf16_packed_body(const uint16_t* __restrict__
     const int S = ldb < 512 ? max(1, (int)(blockDim.x >> 6) / rw) : 1;
     const int sr = w / rw, wr = w - sr * rw;
     const int r0 = blockIdx.z * 512 + wr * 64;     /* grid.z: groups of 512 g columns */
-    if (S == 1 && r0 >= ldb) return;                /* no barriers below when S = 1 */
+    /* the last group of 512 columns may have fewer rows than the workgroup has
+     * waves: the others would write zeros over its partial (no barriers below
+     * when S = 1) */
+    if (S == 1 && w >= rw) return;
     {
         const long sub = (b1 - b0 + S - 1) / S;     /* this wave's sub-range */
         const long s0 = min(b1, b0 + sr * sub);
