@@ -675,18 +675,21 @@ __global__ __launch_bounds__(256) void unmix_f32_kernel(const float* __restrict_
  * stays short); wave w owns g rows [64w, 64w+64) x the 16 CT x columns of
  * slab blockIdx.y, 4 CT accumulators of v_mfma_f32_16x16x4f32; every g
  * element is read once per slab, x once per workgroup (the other waves hit
- * the caches), each lane's operands of one sample in 16-byte loads (164
- * VGPRs at CT = 8, 3 waves per SIMD: 3.10 -> 2.94 ms at 128 ch x 2M x 4
- * models against 4-byte loads).  FP64 partial per chunk.  Where g has
- * fewer than 512 columns (rw = ldb/64 row waves), a workgroup of 8 waves
- * runs S = 8 / rw sub-ranges of its chunk side by side (each as long as a
- * chunk of the one-wave-per-row layout) and adds their totals in FP64
- * through LDS in a fixed order before the one partial is written. */
+ * the caches), each lane's operands of one sample in 16-byte loads, two
+ * steps in flight (128 ch x 2M x 4 models: 2.97 -> 2.83 ms against one,
+ * 3.5 ms with three; bound by the FP32 MFMA rate, 62 % of 157 TFLOP/s).  FP64
+ * partial per chunk.  Where g has fewer than 512 columns (rw = ldb/64 row
+ * waves), a workgroup of 8 waves runs S = 8 / rw sub-ranges of its chunk
+ * side by side and adds their totals in FP64 through LDS in a fixed order, a
+ * quarter of the tile at a time so that every width fits the LDS, before the
+ * one partial is written (128 ch x 500k x 2 models: 438 -> 403 us and, with
+ * half the partials, reductions 123 -> 91 us). */
 template <int CT>
 __global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restrict__ g,
                                                           const float* __restrict__ x,
                                                           double* __restrict__ part, long T,
                                                           int NP, int ldb, long chunk) {
+    constexpr int D = 2;                            /* 4-sample steps in flight */
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int rw = min(ldb - (int)blockIdx.z * 512, 512) / 64;   /* row waves */
     /* sample sub-ranges: only below 512 columns, where the launch gives 8
@@ -714,32 +717,37 @@ __global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restric
     /* MFMA (rt, ct) row i and column j stand for g row r0 + 4 i + rt and x
      * column k0 + CT j + ct, so that a lane's 4 A values and CT B values of
      * one sample are consecutive in memory (16-byte loads) */
-    f32x4 A;
-    float B[CT];
-    auto load = [&](long t4) {
+    f32x4 A[D];
+    float B[D][CT];
+    auto load = [&](int d, long t4) {
         const long t = t4 + (lane >> 4);
         const bool ok = t < te;
-        A = ok ? *(const f32x4*)(g + (size_t)t * ldb + r0 + 4 * (lane & 15)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+        A[d] = ok ? *(const f32x4*)(g + (size_t)t * ldb + r0 + 4 * (lane & 15)) : (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c4 = 0; c4 < CT; c4 += 4) {
             const f32x4 v = ok ? *(const f32x4*)(x + (size_t)t * NP + k0 + CT * (lane & 15) + c4)
                                : (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) B[c4 + e] = v[e];
+            for (int e = 0; e < 4; ++e) B[d][c4 + e] = v[e];
         }
     };
-    load(ts);
-    for (long t4 = ts; t4 < te; t4 += 4) {
-        const f32x4 Ac = A;
-        float Bc[CT];
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) Bc[ct] = B[ct];
-        load(t4 + 4);
+    for (int d = 0; d < D; ++d) load(d, ts + 4 * d);
+    /* D steps per pass, whose last ones may lie past the range (zeros) */
+    for (long t4 = ts; t4 < te; t4 += 4 * D) {
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int d = 0; d < D; ++d) {
+            const f32x4 Ac = A[d];
+            float Bc[CT];
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-                acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ac[rt], Bc[ct], acc[rt][ct], 0, 0, 0);
+            for (int ct = 0; ct < CT; ++ct) Bc[ct] = B[d][ct];
+            load(d, t4 + 4 * (d + D));
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ac[rt], Bc[ct], acc[rt][ct], 0, 0, 0);
+        }
     }
     /* register r of MFMA (rt, ct) in lane l: row r0 + 4 (4 (l / 16) + r) + rt,
      * column k0 + CT (l % 16) + ct: a lane writes CT consecutive columns */
@@ -757,42 +765,44 @@ __global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restric
             }
         return;
     }
-    /* sub-ranges S-1 .. 0 add their totals in FP64 into the LDS tile of
-     * their row wave (register layout: lane-consecutive doubles), in that
-     * order; sub-range 0 then writes the partial from the tile */
+    /* a quarter of the tile (one rt) at a time: sub-ranges S-1 .. 0 add their
+     * totals in FP64 into the LDS of their row wave (register layout:
+     * lane-consecutive doubles), in that order; sub-range 0 then writes the
+     * partial from it */
     extern __shared__ double red64[];
-    double* const tile = red64 + (size_t)wr * 16 * CT * 64;
-    for (int q = S - 1; q >= 0; --q) {
-        if (sr == q) {
+    double* const tile = red64 + (size_t)wr * 4 * CT * 64;
 #pragma unroll
-            for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < 4; ++rt) {
+        for (int q = S - 1; q >= 0; --q) {
+            if (sr == q) {
 #pragma unroll
                 for (int ct = 0; ct < CT; ++ct) {
                     /* converted here, in this wave's turn (not hoisted out
-                     * of the q loop: 16 CT doubles beside the accumulators
+                     * of the q loop: the doubles beside the accumulators
                      * would not fit the registers) */
                     __asm__ volatile("" : "+v"(acc[rt][ct]));
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        double& d = tile[((rt * CT + ct) * 4 + r) * 64 + lane];
+                        double& d = tile[(ct * 4 + r) * 64 + lane];
                         d = q == S - 1 ? (double)acc[rt][ct][r] : d + (double)acc[rt][ct][r];
                     }
                 }
+            }
+            __syncthreads();
         }
-        __syncthreads();
+        if (sr == 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = r0 + 16 * (lane >> 4) + 4 * r + rt;
+                double* o = out + (size_t)row * NP + k0 + CT * (lane & 15);
+#pragma unroll
+                for (int ct = 0; ct < CT; ct += 2)
+                    *(double2*)(o + ct) = make_double2(tile[(ct * 4 + r) * 64 + lane],
+                                                       tile[((ct + 1) * 4 + r) * 64 + lane]);
+            }
+        }
+        __syncthreads();                            /* read before the next quarter */
     }
-    if (sr != 0) return;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = r0 + 16 * (lane >> 4) + 4 * r + rt;
-            double* o = out + (size_t)row * NP + k0 + CT * (lane & 15);
-#pragma unroll
-            for (int ct = 0; ct < CT; ct += 2)
-                *(double2*)(o + ct) = make_double2(tile[((rt * CT + ct) * 4 + r) * 64 + lane],
-                                                   tile[((rt * CT + ct + 1) * 4 + r) * 64 + lane]);
-        }
 }
 
 /* ---------------- statistic GEMM G = g^T x, BF16 --------------------- */
@@ -1138,25 +1148,28 @@ static long gx_chunk(long T, int nchunks, int mult) {
 static int gx_f32_ct(int NP) { return NP % 128 == 0 ? 8 : 4; }
 
 /* workgroups of 8 waves that split their chunk's samples (g narrower than
- * 512 columns, the FP64 LDS tile within 64 KB) */
+ * 512 columns): a quarter of the FP64 tile in LDS */
 static size_t gx_f32_split_lds(int NP, int ldb) {
-    return (size_t)(ldb / 64) * 16 * gx_f32_ct(NP) * 64 * sizeof(double);
+    return (size_t)(ldb / 64) * 4 * gx_f32_ct(NP) * 64 * sizeof(double);
 }
 
-static bool gx_f32_split(int NP, int ldb) {
-    return ldb < 512 && 8 % (ldb / 64) == 0 && gx_f32_split_lds(NP, ldb) <= 65536;
-}
+static bool gx_f32_split(int ldb) { return ldb < 512 && 8 % (ldb / 64) == 0; }
 
 int gx_f32_chunks(long T, int NP, int ldb, int cus) {
-    /* chunks of >= 512 samples (>= 256 per wave where S waves split a
-     * chunk: twice the waves in flight for the same partial count), at
-     * most 256 MB of partials, and at least one per CU of the budget where
-     * T allows */
-    const long per = gx_f32_split(NP, ldb) ? 256L * (8 / (ldb / 64)) : 512L;
-    const long by_len = (T + per - 1) / per;
-    const long by_mem = std::max(1L, (256L << 20) / ((long)ldb * NP * 8));
-    const int slabs = NP / (16 * gx_f32_ct(NP));
+    /* per wave (S of them split a chunk where g has fewer than 512 columns)
+     * 512 samples, 256 below 256 columns of 64 inputs, fewer -- down to 32 --
+     * where the launch would otherwise have less than one workgroup of 8 waves
+     * per CU; at most 256 MB of partials, which are written and read back
+     * once.  A wave's samples are a serial chain of loads and MFMAs: 16 ch x
+     * 20k samples took 62 us with 10 workgroups of 256 samples per wave, 21 us
+     * with 79; two workgroups per CU measured slower (71 ch x 200k, M = 2: 188
+     * instead of 165 us, the partials written twice as often) */
+    const int S = gx_f32_split(ldb) ? 8 / (ldb / 64) : 1;
+    const long len = (NP == 64 && ldb <= 128 ? 256L : 512L) * S;
+    const int slabs = NP / (16 * gx_f32_ct(NP)) * ((ldb + 511) / 512);
     const long want = std::max(1L, (long)cus / slabs);
+    const long by_len = std::max((T + len - 1) / len, std::min(want, (T + 32L * S - 1) / (32L * S)));
+    const long by_mem = std::max(1L, (256L << 20) / ((long)ldb * NP * 8));
     return (int)std::max(1L, std::min(by_len, std::max(want, by_mem)));
 }
 
@@ -1166,7 +1179,7 @@ int launch_gx_f32(const float* g, const float* x, double* part, long T, int NP, 
     const int CT = gx_f32_ct(NP);
     dim3 grid(nchunks, NP / (16 * CT), (ldb + 511) / 512), block(std::min(ldb, 512));
     const long chunk = gx_chunk(T, nchunks, 4);
-    const bool split = gx_f32_split(NP, ldb);
+    const bool split = gx_f32_split(ldb);
     if (split) block = dim3(512);
     const size_t shm = split ? gx_f32_split_lds(NP, ldb) : 0;
     if (CT == 8)

@@ -41,3 +41,16 @@ def test_last_column_group_of_the_statistic_gemm(built, prec, n, M, T):
     # products at a time
     bound = (1024 / 4 + 8) * 2.0 ** -24 * (np.abs(g).T @ np.abs(x))
     assert np.all(np.abs(G - g.T @ x) <= bound + 1e-300)
+
+
+@pytest.mark.parametrize("n,M,T", [(16, 1, 33), (16, 1, 20_000), (64, 2, 1000), (64, 2, 4099), (64, 3, 2050),
+                                   (64, 4, 5001), (100, 1, 3001), (100, 2, 3002), (128, 4, 4003), (200, 1, 2047),
+                                   (200, 2, 1029)])
+def test_fp32_statistic_gemm_sample_splits(built, n, M, T):
+    """Sample counts that end inside a 4-sample step, a wave's range and a
+    workgroup's range, for every width of g (waves that split a chunk's samples
+    or not) and both column tilings of x."""
+    print(f"[statgemm] n={n} M={M} T={T}", flush=True)
+    g, x, G = _operands(ca.PREC_FP32, n, M, T, T)
+    bound = (512 / 4 + 8) * 2.0 ** -24 * (np.abs(g).T @ np.abs(x))
+    assert np.all(np.abs(G - g.T @ x) <= bound + 1e-300)
