@@ -128,8 +128,7 @@ struct amica_engine {
     double* cst64 = nullptr;
     double* stats = nullptr;
     long stride = 0;
-    double *sigma2 = nullptr, *cnew = nullptr, *phis = nullptr, *kappa = nullptr,
-           *lambda = nullptr, *Bm = nullptr, *work = nullptr, *lu = nullptr;
+    double *sigma2 = nullptr, *dc = nullptr, *kappa = nullptr, *lambda = nullptr, *work = nullptr;
     int *bflag = nullptr, *newton = nullptr;
     DevState* ds = nullptr;
     double *log_ll = nullptr, *log_lrate = nullptr, *log_vsum = nullptr;
@@ -199,8 +198,7 @@ struct amica_engine {
         a.xscale = fp8 ? xscale : nullptr;
         a.cst = cst; a.cst64 = cst64;
         a.stats = stats; a.stride = stride;
-        a.sigma2 = sigma2; a.cnew = cnew; a.phis = phis; a.kappa = kappa; a.lambda = lambda;
-        a.B = Bm; a.work = work; a.lu = lu;
+        a.sigma2 = sigma2; a.dc = dc; a.kappa = kappa; a.lambda = lambda; a.work = work;
         a.bflag = bflag; a.newton = newton; a.ds = ds;
         a.log_ll = log_ll; a.log_lrate = log_lrate; a.log_bflag = log_bflag;
         a.log_newton = log_newton; a.log_lldec = log_lldec; a.log_vsum = log_vsum;
@@ -226,14 +224,16 @@ struct amica_engine {
     }
 
     /* the per-recording E-step partials (nparts slots) and statistic-GEMM
-     * partials (nch slots) into the canonical statistics */
-    int enqueue_reduce(int nparts, int nch) {
-        LCHK(launch_reduce(part, nparts, pstride, gxpart, nch, raw, gxtot, sumtmp, margs(), st));
+     * partials (nch slots) into the canonical statistics, with mstep on to
+     * the densities' M-step */
+    int enqueue_reduce(int nparts, int nch, bool mstep) {
+        LCHK(launch_reduce(part, nparts, pstride, gxpart, nch, raw, gxtot, sumtmp, margs(), mstep, st));
         return 0;
     }
 
-    /* prepare, unmixing GEMM, E-step, statistic GEMM, reductions */
-    int enqueue_estep(bool with_timing) {
+    /* prepare, unmixing GEMM, E-step, statistic GEMM, reductions (and with
+     * mstep the densities' M-step, which shares the last launch) */
+    int enqueue_estep(bool with_timing, bool mstep) {
         if (with_timing) HIPCHK(hipEventRecord(ev[0], st));
         int rc;
         {
@@ -269,7 +269,7 @@ struct amica_engine {
         }
         if (with_timing) HIPCHK(hipEventRecord(ev[4], st));
         StageRange r("amica: reductions");
-        return enqueue_reduce(nblocks, nchunks);
+        return enqueue_reduce(nblocks, nchunks, mstep);
     }
 
     /* The batch's launches over many recordings cover the BF16 single-model
@@ -287,7 +287,7 @@ struct amica_engine {
 
     int enqueue_iteration(bool with_timing) {
         StageRange r("amica: EM iteration");
-        int rc = enqueue_estep(with_timing);
+        int rc = enqueue_estep(with_timing, true);
         if (rc) return rc;
         rc = enqueue_mstep();
         if (rc) return rc;
@@ -428,7 +428,7 @@ int amica_engine_create(const amica_options* opts, amica_engine** out) {
     ALLOC(e->part, (size_t)e->nblocks_cap * e->pstride * sizeof(double));
     ALLOC(e->gxpart, (size_t)e->nchunks_cap * e->ldb * NP * sizeof(double));
     ALLOC(e->raw, e->pstride * sizeof(double));
-    ALLOC(e->sumtmp, (size_t)kSumGroups * std::max(e->pstride, (size_t)e->ldb * NP) * sizeof(double));
+    ALLOC(e->sumtmp, (size_t)kSumGroups * (e->pstride + (size_t)e->ldb * NP) * sizeof(double));
     ALLOC(e->gxtot, (size_t)e->ldb * NP * sizeof(double));
     const size_t nn = (size_t)n * n, nm = (size_t)n * m;
     ALLOC(e->A, M * nn * sizeof(double));
@@ -456,13 +456,10 @@ int amica_engine_create(const amica_options* opts, amica_engine** out) {
     e->stride = canonical_stride(n, m);
     ALLOC(e->stats, ((size_t)M * e->stride + 1) * sizeof(double));
     ALLOC(e->sigma2, M * (size_t)n * sizeof(double));
-    ALLOC(e->cnew, M * (size_t)n * sizeof(double));
-    ALLOC(e->phis, M * nn * sizeof(double));
+    ALLOC(e->dc, M * (size_t)n * sizeof(double));
     ALLOC(e->kappa, M * (size_t)n * sizeof(double));
     ALLOC(e->lambda, M * (size_t)n * sizeof(double));
-    ALLOC(e->Bm, M * nn * sizeof(double));
     ALLOC(e->work, (8 + M * nn + inverse_work_doubles(n, M)) * sizeof(double));
-    ALLOC(e->lu, std::max((size_t)M, (size_t)2) * nn * sizeof(double));
     ALLOC(e->bflag, M * sizeof(int));
     ALLOC(e->newton, M * sizeof(int));
     ALLOC(e->ds, sizeof(DevState));
@@ -490,8 +487,8 @@ int amica_engine_destroy(amica_engine* e) {
     void* ptrs[] = {e->xraw, e->xw, e->xw64, e->xbf, e->x8, e->xq, e->xscale, e->b, e->b64, e->g, e->part, e->gxpart,
                     e->raw, e->sumtmp, e->gxtot, e->A, e->c, e->alpha, e->mu, e->beta, e->rho, e->gm, e->W,
                     e->ldet, e->lconst, e->Wg64, e->Wg32, e->wc64, e->Whi, e->Wlo, e->wc, e->cst,
-                    e->cst64, e->stats, e->sigma2, e->cnew, e->phis,
-                    e->kappa, e->lambda, e->Bm, e->work, e->lu, e->bflag, e->newton, e->ds,
+                    e->cst64, e->stats, e->sigma2, e->dc,
+                    e->kappa, e->lambda, e->work, e->bflag, e->newton, e->ds,
                     e->log_ll, e->log_lrate, e->log_vsum, e->log_bflag, e->log_newton,
                     e->log_lldec, e->ltall, e->S, e->mean, e->ldetS_d, e->lq, e->vq};
     for (void* p : ptrs)
@@ -784,7 +781,7 @@ int amica_engine_estep_stats(amica_engine* e, double* stats) {
     int rc = check_ready(e);
     if (rc) return rc;
     HIPCHK(hipSetDevice(e->o.device));
-    rc = e->enqueue_estep(false);
+    rc = e->enqueue_estep(false, false);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(e->st));
     if (stats)
@@ -1080,7 +1077,7 @@ struct amica_batch {
                 continue;
             }
             if (hipStreamWaitEvent(e->st, fork2, 0) != hipSuccess) { rc = AMICA_E_DEVICE; break; }
-            rc = e->enqueue_reduce(gr_nparts[r], gr_nch[r]);
+            rc = e->enqueue_reduce(gr_nparts[r], gr_nch[r], true);
             if (!rc) rc = e->enqueue_mstep();
             if (rc) break;
             if (hipEventRecord(join2[r], e->st) != hipSuccess ||

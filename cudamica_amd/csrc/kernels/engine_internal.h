@@ -196,7 +196,8 @@ struct MstepArgs {
     double* stats;         /* canonical, M*stride + 1 */
     long stride;
     /* work */
-    double *sigma2, *cnew, *phis, *kappa, *lambda, *B, *work, *lu;
+    double *sigma2, *kappa, *lambda, *work;
+    double* dc;            /* step of c in this iteration's M-step */
     int* bflag;            /* [M] */
     int* newton;           /* [M] */
     DevState* ds;
@@ -206,13 +207,16 @@ struct MstepArgs {
 };
 
 /* Sum E-step partials and the statistic-GEMM partials, then write the
- * canonical statistics (including phi through the unmixing identity). */
-/* Partials are summed in up to kSumGroups groups first: tmp holds
- * kSumGroups * max(pstride, ldb NP) doubles. */
+ * canonical statistics (including phi through the unmixing identity) and, with
+ * mstep, take the part of the M-step that needs no phi (launch_mstep is the
+ * rest).  Partials are summed in up to kSumGroups groups first: tmp holds
+ * kSumGroups * (pstride + ldb NP) doubles. */
 constexpr int kSumGroups = 64;
 int launch_reduce(const double* part, int nparts, size_t pstride, const double* gxpart,
-                  int nchunks, double* raw, double* gxtot, double* tmp, const MstepArgs& ma,
+                  int nchunks, double* raw, double* gxtot, double* tmp, const MstepArgs& ma, bool mstep,
                   hipStream_t st);
+/* The M-step after launch_reduce with mstep set: LL and lrate, the A update,
+ * reparameterisation. */
 int launch_mstep(const MstepArgs& ma, hipStream_t st);
 /* W = A^-1, ldet, GEMM-precision W, W c, E-step constants. */
 int launch_prepare(const MstepArgs& ma, hipStream_t st);

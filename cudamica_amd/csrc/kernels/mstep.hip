@@ -64,38 +64,52 @@ __device__ double block_sum(double v, double* sh) {
 /* reductions                                                                 */
 /* ------------------------------------------------------------------------ */
 
-/* out[y][e] = sum of part[p][e] over the partials p of group y = blockIdx.y
- * ([y PG, (y + 1) PG)).  A workgroup covers 64 elements (lanes); its
- * kSumWaves waves take the group's partials p = w, w + kSumWaves, ... and
- * their totals are added in wave order, so the result does not depend on
- * timing. */
+/* One set of partials to sum: out[y][e] = sum of part[p][e] over the partials
+ * p of group y ([y PG, (y + 1) PG)), e < len, by xb workgroups of 64 elements
+ * (lanes) per group, G groups. */
+struct SumSeg {
+    const double* part;
+    double* out;
+    size_t stride, len;
+    int nparts, PG, xb, G;
+};
+
+/* Two sets in one launch (the E-step's partials and the statistic GEMM's):
+ * the first a.xb a.G workgroups take set a.  A workgroup's kSumWaves waves
+ * take its group's partials p = w, w + kSumWaves, ... and their totals are
+ * added in wave order, so the result does not depend on timing. */
 constexpr int kSumWaves = 16;
 
-__global__ __launch_bounds__(64 * kSumWaves) void sum_parts_kernel(const double* __restrict__ part,
-                                                                    int nparts, size_t pstride,
-                                                                    size_t len, int PG,
-                                                                    double* __restrict__ out) {
+__global__ __launch_bounds__(64 * kSumWaves) void sum_parts_kernel(SumSeg a, SumSeg b) {
     __shared__ double acc[kSumWaves][64];
+    const bool second = (int)blockIdx.x >= a.xb * a.G;              /* block-uniform */
+    const SumSeg s = second ? b : a;
+    const int blk = (int)blockIdx.x - (second ? a.xb * a.G : 0);
+    const int y = blk / s.xb, xq = blk - y * s.xb;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const size_t e = (size_t)blockIdx.x * 64 + lane;
-    const int p0 = (int)blockIdx.y * PG, p1 = min(nparts, p0 + PG);
-    double s = 0.0;
-    if (e < len) {
+    const size_t e = (size_t)xq * 64 + lane;
+    const int p0 = y * s.PG, p1 = min(s.nparts, p0 + s.PG);
+    double v = 0.0;
+    if (e < s.len) {
 #pragma unroll 4
-        for (int p = p0 + w; p < p1; p += kSumWaves) s += part[(size_t)p * pstride + e];
+        for (int p = p0 + w; p < p1; p += kSumWaves) v += s.part[(size_t)p * s.stride + e];
     }
-    acc[w][lane] = s;
+    acc[w][lane] = v;
     __syncthreads();
-    if (w == 0 && e < len) {
+    if (w == 0 && e < s.len) {
         double t = 0.0;
         for (int q = 0; q < kSumWaves; ++q) t += acc[q][lane];
-        out[(size_t)blockIdx.y * len + e] = t;
+        s.out[(size_t)y * s.len + e] = t;
     }
 }
 
+__device__ void mstep_a(const MstepArgs& a, int h);
+
 /* Canonical statistics of model blockIdx.x (layout of the oracle, see the
- * engine header), by the workgroups of blockIdx.y = 0; blockIdx.y is the
- * 16 x 16 tile of phi. */
+ * engine header), by the workgroups of blockIdx.y = 0, which with MSTEP go on
+ * to the M-step of the model's densities from them, beside the other
+ * workgroups: blockIdx.y - 1 is their 16 x 16 tile of phi. */
+template <bool MSTEP>
 __global__ __launch_bounds__(kBlk) void finalize_kernel(const double* __restrict__ raw,
                                                         const double* __restrict__ gx,
                                                         MstepArgs a) {
@@ -140,6 +154,11 @@ __global__ __launch_bounds__(kBlk) void finalize_kernel(const double* __restrict
                 a.work[0] = c0;   /* offset of the ltall record */
             }
         }
+        if constexpr (MSTEP) {
+            __syncthreads();      /* the statistics above, read by other threads */
+            mstep_a(a, h);
+        }
+        return;
     }
     /* phi_h[i][k] = sum_l G[h*NP+i][l] W~_h[k][l] - gsum_h[i] wc_h[k]: one
      * 16 x 16 (i, k) tile per workgroup (blockIdx.y), the l sum through
@@ -148,7 +167,7 @@ __global__ __launch_bounds__(kBlk) void finalize_kernel(const double* __restrict
      * increasing l */
     const double* gsum_base = rh + kStatsPerJ * m + kRawGsum;
     const int ntk = (n + 15) / 16;
-    const int tib = (int)blockIdx.y / ntk, tkb = (int)blockIdx.y - tib * ntk;
+    const int tib = ((int)blockIdx.y - 1) / ntk, tkb = (int)blockIdx.y - 1 - tib * ntk;
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
     __shared__ double Gs[16][17];                  /* [i][l] */
     __shared__ double Ws[16][17];                  /* [k][l] */
@@ -181,13 +200,13 @@ __global__ __launch_bounds__(kBlk) void finalize_kernel(const double* __restrict
 /* M-step                                                                     */
 /* ------------------------------------------------------------------------ */
 
-/* Per model: gm, alpha, sigma2, cnew, phi/vsum, kappa, lambda, mu, beta,
- * rho, the Newton test and the matrix B.  (Flat indices below n n <= 2^20
+/* Per model, by one workgroup: gm, alpha, sigma2, c (and its step), kappa,
+ * lambda, mu, beta, rho and the Newton test.  (Flat indices below n n <= 2^20
  * are split with 32-bit division, here and in the kernels below.) */
-__global__ __launch_bounds__(kBlk) void mstep_a_kernel(MstepArgs a) {
+__device__ void mstep_a(const MstepArgs& a, int h) {
     __shared__ double sh[16];
     __shared__ double ks[kInvMax];          /* kappa_i sigma2_i */
-    const int h = blockIdx.x, n = a.n, m = a.m;
+    const int n = a.n, m = a.m;
     const long nm = (long)n * m;
     const COff o(n, m);
     const double* st = a.stats + (size_t)h * a.stride;
@@ -198,7 +217,8 @@ __global__ __launch_bounds__(kBlk) void mstep_a_kernel(MstepArgs a) {
     double* beta = a.beta + (size_t)h * nm;
     double* rho = a.rho + (size_t)h * nm;
     double* sig = a.sigma2 + (size_t)h * n;
-    double* cnw = a.cnew + (size_t)h * n;
+    double* c = a.c + (size_t)h * n;
+    double* dc = a.dc + (size_t)h * n;
     double* kap = a.kappa + (size_t)h * n;
     double* lam = a.lambda + (size_t)h * n;
 
@@ -210,7 +230,9 @@ __global__ __launch_bounds__(kBlk) void mstep_a_kernel(MstepArgs a) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         const double sg = st[o.s2 + i] / vsum;
         sig[i] = sg;
-        cnw[i] = st[o.cnew + i] / vsum;
+        const double cn = st[o.cnew + i] / vsum;
+        dc[i] = cn - c[i];                  /* for the mu shift */
+        c[i] = cn;
         double kk = 0.0, ll = 0.0;
         for (int j = 0; j < m; ++j) {
             const long q = (long)j * n + i;
@@ -262,41 +284,36 @@ __global__ __launch_bounds__(kBlk) void mstep_a_kernel(MstepArgs a) {
     }
 }
 
-/* phi_h = Phi_h / vsum_h and the direction B_h, one thread per (i, k) over
- * grid (., M): Newton's B (updateBDiagonal / getB) where model h takes a
- * Newton step, I - phi (geteyemphi) otherwise. */
-__global__ __launch_bounds__(256) void mstep_bmat_kernel(MstepArgs a) {
-    const int h = blockIdx.y, n = a.n;
-    const long nn = (long)n * n;
-    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nn) return;
-    const int i = (int)((unsigned)q % (unsigned)n), k = (int)((unsigned)q / (unsigned)n);
-    const COff o(n, a.m);
-    const double* st = a.stats + (size_t)h * a.stride;
-    const double vsum = st[0];
-    const double ph = st[o.phi + q] / vsum;
-    a.phis[(size_t)h * nn + q] = ph;
-    double bv;
-    if (a.newton[h]) {
-        const double* sig = a.sigma2 + (size_t)h * n;
-        const double* kap = a.kappa + (size_t)h * n;
-        if (i == k) {
-            bv = (1.0 - ph) / a.lambda[(size_t)h * n + i];          /* updateBDiagonal */
-        } else {
-            const double D = (kap[i] * sig[i]) * (kap[k] * sig[k]);
-            const double nom = -sig[i] * kap[k];
-            const double pt = st[o.phi + k + (long)i * n] / vsum;
-            bv = (nom * -ph + -pt) / (D - 1.0);                    /* getB */
-        }
-    } else {
-        bv = (i == k ? 1.0 : 0.0) - ph;                             /* geteyemphi */
+/* Entry (i, k) of the direction B_h: Newton's B (updateBDiagonal / getB)
+ * where model h takes a Newton step, I - phi (geteyemphi) otherwise, with
+ * phi_h = Phi_h / vsum_h. */
+struct Direction {
+    const double *phi, *sig, *kap, *lam;
+    double vsum;
+    int n, newton;
+    __device__ Direction(const MstepArgs& a, int h) {
+        n = a.n;
+        const double* st = a.stats + (size_t)h * a.stride;
+        vsum = st[0];
+        phi = st + COff(n, a.m).phi;
+        sig = a.sigma2 + (size_t)h * n;
+        kap = a.kappa + (size_t)h * n;
+        lam = a.lambda + (size_t)h * n;
+        newton = a.newton[h];
     }
-    a.B[(size_t)h * nn + q] = bv;
-}
+    __device__ double operator()(int i, int k) const {
+        const double ph = phi[i + (long)k * n] / vsum;
+        if (!newton) return (i == k ? 1.0 : 0.0) - ph;              /* geteyemphi */
+        if (i == k) return (1.0 - ph) / lam[i];                     /* updateBDiagonal */
+        const double D = (kap[i] * sig[i]) * (kap[k] * sig[k]);
+        const double nom = -sig[i] * kap[k];
+        const double pt = phi[k + (long)i * n] / vsum;
+        return (nom * -ph + -pt) / (D - 1.0);                       /* getB */
+    }
+};
 
 /* The scalar part: LL, the decrease rule and the lrate schedule. */
-__global__ void mstep_b_kernel(MstepArgs a) {
-    if (threadIdx.x != 0) return;
+__device__ void mstep_b(const MstepArgs& a) {
     DevState* ds = a.ds;
     const int k_it = ds->iter + 1;
     const double LL = a.stats[(size_t)a.M * a.stride] / ((double)a.n * (double)a.T);
@@ -331,25 +348,32 @@ __global__ void mstep_b_kernel(MstepArgs a) {
 
 /* AB_h = A_h B_h for every model (column-major n x n, FP64): 16 x 16
  * output tiles per workgroup over grid (n/16, n/16, M), the l sum through
- * 16-wide LDS tiles of A and B, one FMA per l in increasing l. */
+ * 16-wide LDS tiles of A and B, one FMA per l in increasing l.  B's entries
+ * are formed as they are staged (n / 16 times each: a division or three, less
+ * than a launch and a pass over memory of their own); the scalar part runs
+ * beside the tiles in workgroup (0, 0, M). */
 constexpr int kAbTile = 16;
 
 __global__ __launch_bounds__(kAbTile * kAbTile) void ab_kernel(MstepArgs a) {
     __shared__ double As[kAbTile][kAbTile + 1];   /* [l][i] */
     __shared__ double Bs[kAbTile][kAbTile + 1];   /* [k][l] */
     const int h = blockIdx.z, n = a.n;
+    if (h == a.M || !a.update_A) {
+        if (h == a.M && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) mstep_b(a);
+        return;
+    }
+    const Direction B(a, h);
     const long nn = (long)n * n;
     const int ti = threadIdx.x % kAbTile, tk = threadIdx.x / kAbTile;
     const int i = blockIdx.x * kAbTile + ti, k = blockIdx.y * kAbTile + tk;
     const double* A = a.A + (size_t)h * nn;
-    const double* B = a.B + (size_t)h * nn;
     double s = 0.0;
     for (int l0 = 0; l0 < n; l0 += kAbTile) {
         /* A tile: lanes along i (consecutive in memory); B tile: along l */
         const int ai = blockIdx.x * kAbTile + ti, al = l0 + tk;
         As[tk][ti] = (ai < n && al < n) ? A[ai + (long)al * n] : 0.0;
         const int bl = l0 + ti, bk = blockIdx.y * kAbTile + tk;
-        Bs[tk][ti] = (bl < n && bk < n) ? B[bl + (long)bk * n] : 0.0;
+        Bs[tk][ti] = (bl < n && bk < n) ? B(bl, bk) : 0.0;
         __syncthreads();
         const int lend = min(kAbTile, n - l0);
         for (int l = 0; l < lend; ++l) s += As[l][ti] * Bs[tk][l];
@@ -361,8 +385,8 @@ __global__ __launch_bounds__(kAbTile * kAbTile) void ab_kernel(MstepArgs a) {
 /* A += +-lrate A B and the reparameterisation, one wave per column k of
  * model blockIdx.y (source k): normalizeAsave divides column k by its norm
  * nu, normalizemubeta scales mu_jk by nu and beta_jk by 1/nu^2, and the mu
- * shift subtracts (W_old (cnew - c))_k.  c itself is replaced by cnew in
- * copy_c_kernel afterwards, once every column has read the old c. */
+ * shift subtracts (W_old (cnew - c))_k, whose step of c the M-step left in dc
+ * when it replaced c. */
 constexpr int kColWaves = 4;
 constexpr int kColRegs = kInvMax / 64;
 
@@ -403,10 +427,9 @@ __global__ __launch_bounds__(64 * kColWaves) void mstep_col_kernel(MstepArgs a) 
     }
     /* (W_old (cnew - c))_k: row k of W, lanes over l */
     const double* W = a.W + (size_t)h * nn;
-    const double* c = a.c + (size_t)h * n;
-    const double* cnw = a.cnew + (size_t)h * n;
+    const double* dc = a.dc + (size_t)h * n;
     double d = 0.0;
-    for (int l = lane; l < n; l += 64) d += W[k + (long)l * n] * (cnw[l] - c[l]);
+    for (int l = lane; l < n; l += 64) d += W[k + (long)l * n] * dc[l];
     d = wave_sum_f64(d);
     double* mu = a.mu + (size_t)h * nm;
     double* beta = a.beta + (size_t)h * nm;
@@ -416,13 +439,6 @@ __global__ __launch_bounds__(64 * kColWaves) void mstep_col_kernel(MstepArgs a) 
         mu[(long)j * n + k] = ms - d;
         beta[(long)j * n + k] = beta[(long)j * n + k] / (nu * nu);
     }
-}
-
-/* c <- cnew for every model (grid (., M)) */
-__global__ __launch_bounds__(256) void copy_c_kernel(MstepArgs a) {
-    const int h = blockIdx.y;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < a.n) a.c[(size_t)h * a.n + i] = a.cnew[(size_t)h * a.n + i];
 }
 
 /* ------------------------------------------------------------------------ */
@@ -440,15 +456,22 @@ __device__ __forceinline__ double joined_w(uint16_t hi, uint16_t lo) {
     return (double)bf16_bits_to_f32(hi) + (double)bf16_bits_to_f32(lo);
 }
 
-/* After W = A^-1, for all models at once (grid (., M)): the GEMM copies of
- * W (rows h NP + i, columns k) and the per-(h, j, i) E-step constants.
- * Flat index per model: [0, n n) W entries, then the n m constants. */
-__global__ __launch_bounds__(256) void prepare_tail_kernel(MstepArgs a) {
+__device__ void wc_rows(const MstepArgs& a, int h, int i);
+
+/* After W = A^-1, for all models at once (grid (tb + n / 4, M)): workgroups
+ * below tb write the GEMM copies of W (rows h NP + i, columns k) and the
+ * per-(h, j, i) E-step constants, the others four rows of W~ c each.  Flat
+ * index per model: [0, n n) W entries, then the n m constants. */
+__global__ __launch_bounds__(256) void prepare_tail_kernel(MstepArgs a, int tb) {
     const int h = blockIdx.y, n = a.n, m = a.m, NP = a.NP;
+    if ((int)blockIdx.x >= tb) {
+        wc_rows(a, h, ((int)blockIdx.x - tb) * 4 + ((int)threadIdx.x >> 6));
+        return;
+    }
     const long nn = (long)n * n, nm = (long)n * m;
     const double* W = a.W + (size_t)h * nn;
     const long total = nn + nm;
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (long)gridDim.x * blockDim.x) {
+    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (long)tb * blockDim.x) {
         if (q < nn) {
             const int i = (int)((unsigned)q % (unsigned)n), k = (int)((unsigned)q / (unsigned)n);
             const double wv2 = W[q];
@@ -487,12 +510,10 @@ __global__ __launch_bounds__(256) void prepare_tail_kernel(MstepArgs a) {
     }
 }
 
-/* W~ c_h, one wave per row i over grid (n/4, M), lanes over k: the W~ the
- * unmixing GEMM applies (W~ = split(W diag(s)) diag(1/s) on the BF16 and FP8
+/* Row i of W~ c_h by one wave, lanes over k: the W~ the unmixing GEMM applies (W~ = split(W diag(s)) diag(1/s) on the BF16 and FP8
  * paths, fp32(W) on the plain FP32 path, W itself on the FP32 path). */
-__global__ __launch_bounds__(256) void wc_kernel(MstepArgs a) {
-    const int h = blockIdx.y, n = a.n, lane = threadIdx.x & 63;
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+__device__ void wc_rows(const MstepArgs& a, int h, int i) {
+    const int n = a.n, lane = threadIdx.x & 63;
     if (i >= n) return;
     const double* W = a.W + (size_t)h * n * n;
     const double* c = a.c + (size_t)h * n;
@@ -1110,51 +1131,47 @@ static int sum_groups(int nparts, size_t len) {
     return (int)std::max(1L, std::min<long>(g, kSumGroups));
 }
 
-/* out = sum over nparts partials: one pass, or a pass over groups into tmp
- * and a second pass over the groups */
-static void sum_parts(const double* part, int nparts, size_t pstride, size_t len, double* tmp,
-                      double* out, hipStream_t st) {
-    const dim3 blk(64 * kSumWaves);
-    const unsigned xb = (unsigned)((len + 63) / 64);
-    const int G = sum_groups(nparts, len);
-    if (G == 1) {
-        hipLaunchKernelGGL(sum_parts_kernel, dim3(xb, 1), blk, 0, st, part, nparts, pstride, len, nparts, out);
-        return;
-    }
-    const int PG = (nparts + G - 1) / G;
-    hipLaunchKernelGGL(sum_parts_kernel, dim3(xb, G), blk, 0, st, part, nparts, pstride, len, PG, tmp);
-    hipLaunchKernelGGL(sum_parts_kernel, dim3(xb, 1), blk, 0, st, (const double*)tmp, G, len, len, G, out);
+/* The first pass over one set of partials: all of them into out, or (G > 1)
+ * groups into tmp, whose sum the second pass takes into out. */
+static SumSeg first_pass(const double* part, int nparts, size_t stride, size_t len, double* tmp, double* out) {
+    const int G = sum_groups(nparts, len), PG = (nparts + G - 1) / G;
+    return SumSeg{part, G == 1 ? out : tmp, stride, len, nparts, PG, (int)((len + 63) / 64), G};
+}
+
+static SumSeg second_pass(const SumSeg& f, double* out) {
+    if (f.G == 1) return SumSeg{nullptr, nullptr, 0, 0, 0, 0, 0, 0};
+    return SumSeg{f.out, out, f.len, f.len, f.G, f.G, f.xb, 1};
 }
 
 int launch_reduce(const double* part, int nparts, size_t pstride, const double* gxpart,
-                  int nchunks, double* raw, double* gxtot, double* tmp, const MstepArgs& ma,
+                  int nchunks, double* raw, double* gxtot, double* tmp, const MstepArgs& ma, bool mstep,
                   hipStream_t st) {
     const int NS = kStatsPerJ * ma.m + kStatsPerI;
     const size_t plen = (size_t)ma.M * NS * ma.NP + ma.M + 1;
-    sum_parts(part, nparts, pstride, plen, tmp, raw, st);
     const size_t glen = (size_t)ma.ldb * ma.NP;
-    sum_parts(gxpart, nchunks, glen, glen, tmp, gxtot, st);
-    /* one 16 x 16 tile of phi per workgroup (the statistics by the first) */
+    const SumSeg p = first_pass(part, nparts, pstride, plen, tmp, raw);
+    const SumSeg g = first_pass(gxpart, nchunks, glen, glen, tmp + kSumGroups * pstride, gxtot);
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(p.xb * p.G + g.xb * g.G)), dim3(64 * kSumWaves), 0, st, p, g);
+    const SumSeg p2 = second_pass(p, raw), g2 = second_pass(g, gxtot);
+    if (p2.xb + g2.xb > 0)
+        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(p2.xb + g2.xb)), dim3(64 * kSumWaves), 0, st, p2, g2);
+    /* one 16 x 16 tile of phi per workgroup, after the statistics' */
     const unsigned ntk = (unsigned)((ma.n + 15) / 16);
-    hipLaunchKernelGGL(finalize_kernel, dim3(ma.M, ntk * ntk), dim3(kBlk), 0, st, raw, gxtot, ma);
+    const dim3 grid(ma.M, 1 + ntk * ntk);
+    if (mstep) hipLaunchKernelGGL(finalize_kernel<true>, grid, dim3(kBlk), 0, st, raw, gxtot, ma);
+    else hipLaunchKernelGGL(finalize_kernel<false>, grid, dim3(kBlk), 0, st, raw, gxtot, ma);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int launch_mstep(const MstepArgs& ma, hipStream_t st) {
     const int n = ma.n;
     if (n < 1 || n > kInvMax) return -1;
-    const long nn = (long)n * n;
-    hipLaunchKernelGGL(mstep_a_kernel, dim3(ma.M), dim3(kBlk), 0, st, ma);
-    hipLaunchKernelGGL(mstep_b_kernel, dim3(1), dim3(64), 0, st, ma);
-    if (ma.update_A) {
-        hipLaunchKernelGGL(mstep_bmat_kernel, dim3((unsigned)((nn + 255) / 256), ma.M), dim3(256), 0,
-                           st, ma);
-        const unsigned nt = (unsigned)((n + kAbTile - 1) / kAbTile);
-        hipLaunchKernelGGL(ab_kernel, dim3(nt, nt, ma.M), dim3(kAbTile * kAbTile), 0, st, ma);
+    /* without an A update only the scalar part is left */
+    const unsigned nt = ma.update_A ? (unsigned)((n + kAbTile - 1) / kAbTile) : 1u;
+    hipLaunchKernelGGL(ab_kernel, dim3(nt, nt, ma.M + 1), dim3(kAbTile * kAbTile), 0, st, ma);
+    if (ma.update_A)
         hipLaunchKernelGGL(mstep_col_kernel, dim3((unsigned)((n + kColWaves - 1) / kColWaves), ma.M),
                            dim3(64 * kColWaves), 0, st, ma);
-    }
-    hipLaunchKernelGGL(copy_c_kernel, dim3((unsigned)((n + 255) / 256), ma.M), dim3(256), 0, st, ma);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1186,8 +1203,7 @@ int launch_prepare(const MstepArgs& ma, hipStream_t st) {
     launch_inverse(ma, st);
     const long total = (long)ma.n * ma.n + (long)ma.n * ma.m;
     const unsigned gx = (unsigned)std::min<long>((total + 255) / 256, 256);
-    hipLaunchKernelGGL(prepare_tail_kernel, dim3(gx, ma.M), dim3(256), 0, st, ma);
-    hipLaunchKernelGGL(wc_kernel, dim3((unsigned)((n + 3) / 4), ma.M), dim3(256), 0, st, ma);
+    hipLaunchKernelGGL(prepare_tail_kernel, dim3(gx + (unsigned)((n + 3) / 4), ma.M), dim3(256), 0, st, ma, (int)gx);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
