@@ -16,16 +16,16 @@
  *   dc_h   = W_h^T sum_t g_t
  * with f = rho sign(y)|y|^(rho-1).
  *
- * Kernels: prep (per model: W^-1 by LU, log|det W|, W c, the constant part
- * of Q), the unmixing GEMM b = W x - W c on MFMA (the engine's FP64 or plain
- * FP32 kernels, into a [T][M NP] buffer), ll (one wave per (model, 64-channel
+ * Kernels: the inverse and log|det W| (the M-step's Gauss-Jordan), prep (W c,
+ * the constant part of Q, GEMM operands), then per chunk of samples the
+ * unmixing GEMM b = W x - W c on MFMA (the engine's FP64 or plain FP32
+ * kernels, into a [T][M NP] buffer), ll (one wave per (model, 64-channel
  * block) over a range of samples, all M ceil(n/64) waves in one workgroup
- * where they fit in 8, else three passes through per-sample buffers; b read
- * from the GEMM's buffer -- the allocation-free forward instead forms it per
- * lane from x tiles in LDS), gx (sum_t g_t x_t^T: FP32 MFMA on the FP32
- * variant, 64 x 64 FP64 tiles on the FP64 one, over sample chunks), and
- * finish (fixed-order sums over workgroups and the assembly of the
- * gradients).
+ * where they fit in 8, else three passes through per-sample buffers; the
+ * allocation-free forward instead forms b there, 16 samples at a time on
+ * MFMA), gx (sum_t g_t x_t^T on FP32 or FP64 MFMA over sample chunks) and the
+ * sums of their partials; finish assembles the gradients from the chunks'
+ * totals.
  * Every reduction is in a fixed order, so results repeat bit for bit.
  */
 #include <hip/hip_runtime.h>
@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "../../../include/amica_adjoint.h"
 #include "../../../include/amica_engine.h"
@@ -54,14 +55,12 @@ struct AdjArgs {
     double* ll;          /* [T] or null */
     /* workspace */
     double* Winv;        /* [M][n][n] column-major */
-    double* ldet;        /* [M] log|det W_h| */
+    double* ldet;        /* [M] -log|det W_h| */
     double* cq;          /* [M][m][n] log alpha + .5 log beta - log2 - lgamma(1+1/rho) */
     double* wc;          /* [M][NP] W_h c_h */
-    double* lu;          /* [M][n][n] LU scratch */
-    double* X;           /* [M][n][n] inverse scratch */
     void* g;             /* [T][M NP] (adjoint) */
     double* part;        /* [nblocks][pstride] */
-    long chunk;          /* samples per workgroup */
+    long chunk;          /* samples per workgroup, a multiple of 16 */
     size_t pstride;
     /* split passes (M ceil(n/64) > 8 waves): workgroups of pg (model,
      * channel-block) pairs, blockIdx.y = pair group; qbuf [T][M CW] the
@@ -69,284 +68,367 @@ struct AdjArgs {
     double* qbuf;
     double* vbuf;
     int pg;
-    /* b = W x - W c from the unmixing GEMM, [T][M NP] Real, or null: each
-     * lane then forms its b from an LDS tile of x (the allocation-free
-     * forward) */
+    /* b = W x - W c from the unmixing GEMM, [T][M NP] Real (BSRC 0) */
     const void* bbuf;
 };
 
-enum { kLlFused = 0, kLlQ = 1, kLlGrad = 2 };
+/* kLlFused: a workgroup holds all M ceil(n/64) (model, channel-block) pairs of
+ * a sample range and exchanges the channel sums in LDS.  kLlM1: one model,
+ * whose posterior is 1 (the exchange serves ll alone).  Where the pairs do not
+ * fit one workgroup the same body runs in three passes: kLlQ writes each
+ * pair's channel sum of q per sample (qbuf), ll_post_kernel forms L_h, ll_t and
+ * dll_t v_ht (vbuf), and kLlGrad re-evaluates the densities and accumulates
+ * the gradients. */
+enum { kLlFused = 0, kLlQ = 1, kLlGrad = 2, kLlM1 = 3 };
 
-/* per pair (h, i): dalpha_j, dmu_j, dbeta_j, drho_j (j < m), gsum; then Omega_h */
+/* raw sums per pair (h, i): su_j, su|y|^(rho-1)sgn_j, su|y|^rho_j,
+ * su|y|^rho log|y|_j (j < m), gsum; then Omega_h */
 __host__ __device__ inline int pair_stride(int m) { return 4 * m + 1; }
 
-/* Per model: W^-1 and log|det W| -- here by LU in this workgroup (the
- * allocation-free forward, a.lu set), else already computed by the
- * Gauss-Jordan launches, which leave -log|det W| in ldet -- then W c and
- * the constant part of Q. */
-__global__ __launch_bounds__(256) void adj_prep_kernel(AdjArgs a) {
-    __shared__ int perm[1024];
-    const int h = blockIdx.x, n = a.n, m = a.m;
-    const long nn = (long)n * n;
-    const double* W = a.W + (size_t)h * nn;
-    if (a.lu) {
-        const double lad = block_lu_inverse(W, n, a.lu + (size_t)h * nn, a.X + (size_t)h * nn,
-                                            a.Winv + (size_t)h * nn, perm);
-        if (threadIdx.x == 0) a.ldet[h] = lad;
-    } else if (threadIdx.x == 0) {
-        a.ldet[h] = -a.ldet[h];
-    }
-    const double* c = a.c + (size_t)h * n;
-    for (int i = threadIdx.x; i < a.NP; i += blockDim.x) {
+/* What every sample needs of the model: W c, the constant part of Q, and
+ * (Wg not null) the unmixing GEMM's operands Wg[h NP + i][k] = W_h[i][k] (zero
+ * past n) and W c in its precision.  Grid (eb + NP / 4, M): workgroups below
+ * eb take the elementwise parts, the others four rows of W c, one per wave. */
+template <typename Real>
+__global__ __launch_bounds__(256) void adj_prep_kernel(AdjArgs a, int eb, Real* __restrict__ Wg,
+                                                       Real* __restrict__ wcr) {
+    const int h = blockIdx.y, n = a.n, m = a.m, NP = a.NP;
+    const double* W = a.W + (size_t)h * n * n;
+    if ((int)blockIdx.x >= eb) {
+        const int lane = threadIdx.x & 63, i = ((int)blockIdx.x - eb) * 4 + ((int)threadIdx.x >> 6);
+        if (i >= NP) return;
+        const double* c = a.c + (size_t)h * n;
         double s = 0.0;
         if (i < n)
-            for (int k = 0; k < n; ++k) s += W[i + (long)k * n] * c[k];
-        a.wc[(size_t)h * a.NP + i] = s;
+            for (int k = lane; k < n; k += 64) s += W[i + (size_t)k * n] * c[k];
+        s = wave_sum_f64(s);
+        if (lane == 0) {
+            a.wc[(size_t)h * NP + i] = s;
+            if (Wg) wcr[(size_t)h * NP + i] = (Real)s;
+        }
+        return;
     }
-    const long nm = (long)n * m;
-    for (long q = threadIdx.x; q < nm; q += blockDim.x) {
-        const size_t e = (size_t)h * nm + q;
-        a.cq[e] = log(a.alpha[e]) + 0.5 * log(a.beta[e]) - AMICA_LOG2_REF - lgamma(1.0 + 1.0 / a.rho[e]);
+    const int nm = n * m, total = Wg ? NP * NP : 0;
+    for (int q = (int)blockIdx.x * 256 + threadIdx.x; q < max(nm, total); q += eb * 256) {
+        if (q < nm) {
+            const size_t e = (size_t)h * nm + q;
+            a.cq[e] = log(a.alpha[e]) + 0.5 * log(a.beta[e]) - AMICA_LOG2_REF - lgamma(1.0 + 1.0 / a.rho[e]);
+        }
+        if (q < total) {
+            /* rows along the threads: the column-major W is read in order */
+            const int i = q % NP, k = q / NP;
+            Wg[((size_t)h * NP + i) * NP + k] = (i < n && k < n) ? (Real)W[(size_t)k * n + i] : (Real)0;
+        }
     }
 }
 
-/* FP32: the hardware base-2 logarithm and exponential (v_log_f32,
- * v_exp_f32; arguments here are normal or underflow to 0) and reciprocal. */
-template <typename Real> __device__ __forceinline__ Real r_log(Real v);
-template <> __device__ __forceinline__ float r_log<float>(float v) {
-    return __builtin_amdgcn_logf(v) * 0.6931471805599453f;
+/* Base-2 logarithm and exponential on the FP32 variant (v_log_f32, v_exp_f32;
+ * arguments here are normal or underflow to 0), natural ones in FP64: kLn is
+ * the logarithm of the variant's base, kUnit its reciprocal. */
+template <typename Real> struct Base;
+template <> struct Base<float> {
+    static constexpr double kLn = 0.6931471805599453, kUnit = 1.4426950408889634;
+    static constexpr float kTiny = 1.17549435e-38f;
+    static __device__ __forceinline__ float log(float v) { return __builtin_amdgcn_logf(v); }
+    static __device__ __forceinline__ float exp(float v) { return __builtin_amdgcn_exp2f(v); }
+    static __device__ __forceinline__ float rcp(float v) { return __builtin_amdgcn_rcpf(v); }
+};
+template <> struct Base<double> {
+    static constexpr double kLn = 1.0, kUnit = 1.0;
+    static constexpr double kTiny = 2.2250738585072014e-308;
+    static __device__ __forceinline__ double log(double v) { return ::log(v); }
+    static __device__ __forceinline__ double exp(double v) { return ::exp(v); }
+    static __device__ __forceinline__ double rcp(double v) { return 1.0 / v; }
+};
+
+/* Samples per tile, held in registers between the densities and the gradient
+ * sums (4 values per component and sample on the adjoint): as many as keep the
+ * kernel within 256 VGPRs. */
+template <typename Real, int MJ, bool ADJ> constexpr int tile_samples() {
+    return sizeof(Real) == 4 ? (MJ <= 5 || !ADJ ? 4 : 2) : (!ADJ || MJ <= 3 ? 4 : MJ <= 5 ? 2 : 1);
 }
-template <> __device__ __forceinline__ double r_log<double>(double v) { return log(v); }
-template <typename Real> __device__ __forceinline__ Real r_exp(Real v);
-template <> __device__ __forceinline__ float r_exp<float>(float v) {
-    return __builtin_amdgcn_exp2f(v * 1.4426950408889634f);
+
+/* 64-bit value of the lane a row rotation by R brings in (rows of 16) */
+template <int R> __device__ __forceinline__ double row_ror(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)u, 0x120 + R, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), 0x120 + R, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
-template <> __device__ __forceinline__ double r_exp<double>(double v) { return exp(v); }
-template <typename Real> __device__ __forceinline__ Real r_rcp(Real v);
-template <> __device__ __forceinline__ float r_rcp<float>(float v) { return __builtin_amdgcn_rcpf(v); }
-template <> __device__ __forceinline__ double r_rcp<double>(double v) { return 1.0 / v; }
 
-template <typename Real> struct RealTiny;
-template <> struct RealTiny<float> { static constexpr float v = 1.17549435e-38f; };
-template <> struct RealTiny<double> { static constexpr double v = 2.2250738585072014e-308; };
+__device__ __forceinline__ double row_sum(double v) {
+    v += row_ror<8>(v);
+    v += row_ror<4>(v);
+    v += row_ror<2>(v);
+    return v + row_ror<1>(v);
+}
 
-/* Samples per tile held in LDS and registers. */
-template <typename Real> struct Tile { static constexpr int S = sizeof(Real) == 8 ? 4 : 8; };
+__device__ __forceinline__ double row_max(double v) {
+    v = fmax(v, row_ror<8>(v));
+    v = fmax(v, row_ror<4>(v));
+    v = fmax(v, row_ror<2>(v));
+    return fmax(v, row_ror<1>(v));
+}
 
-/* Component j of channel i of model h at sample value b: y, Q, and (for the
- * adjoint) f y, f and |y|^rho ln|y|. */
+/* Two values folded onto each other across the halves (H 32) or the row pairs
+ * (H 16) of the wave: swapping a's odd halves (rows) with b's even ones and
+ * adding leaves a's pair sums in the even ones, b's in the odd ones. */
+template <int H> __device__ __forceinline__ double fold(double a, double b) {
+    const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+    auto swap = [](uint32_t p, uint32_t q) {
+        if constexpr (H == 32) return __builtin_amdgcn_permlane32_swap(p, q, false, false);
+        else return __builtin_amdgcn_permlane16_swap(p, q, false, false);
+    };
+    const auto lo = swap((uint32_t)ua, (uint32_t)ub), hi = swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+           __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+
+/* Wave sums of S samples' values at once: every lane of row r ends with the
+ * total of sample sample_of_row(r). */
+template <int S> __device__ __forceinline__ double wave_totals(const double (&q)[S]) {
+    double v;
+    if constexpr (S == 4) v = fold<16>(fold<32>(q[0], q[1]), fold<32>(q[2], q[3]));
+    else if constexpr (S == 2) { v = fold<32>(q[0], q[1]); v = fold<16>(v, v); }
+    else { v = fold<32>(q[0], q[0]); v = fold<16>(v, v); }
+    return row_sum(v);
+}
+
+template <int S> __device__ __forceinline__ int sample_of_row(int r) {
+    return S == 4 ? ((r & 1) << 1) | (r >> 1) : S == 2 ? r >> 1 : 0;
+}
+
+__device__ __forceinline__ double readlane_f64(double v, int l) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+/* 16 samples x this wave's 64 channels of W_h x by MFMA into the wave's LDS
+ * tile [16][64]: x rows and W straight from global memory as fragments
+ * (element (l % 16, l / 16) per lane), rows past T and inputs past n as
+ * zeros. */
 template <typename Real>
-__device__ __forceinline__ void density(Real b, Real sb, Real mu, Real rho, Real cq, Real& y,
-                                        Real& Q, Real& yr, Real& lny) {
-    y = sb * (b - mu);
-    const Real ay = fmax(fabs(y), RealTiny<Real>::v);
-    lny = r_log<Real>(ay);
-    yr = r_exp<Real>(rho * lny);     /* |y|^rho */
-    Q = cq - yr;
+__device__ __forceinline__ void unmix_tile(const AdjArgs& a, const double* __restrict__ Wh, int ch0, long t0,
+                                           Real* __restrict__ tile) {
+    const int lane = threadIdx.x & 63, l15 = lane & 15, kq = lane >> 4, n = a.n;
+    const Real* xr = (const Real*)a.x + (size_t)min(t0 + l15, a.T - 1) * n;
+    const bool row = t0 + l15 < a.T;
+    typedef Real R4 __attribute__((ext_vector_type(4)));
+    R4 acc[4];
+    const double* wp[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        acc[q] = (R4){(Real)0, (Real)0, (Real)0, (Real)0};
+        wp[q] = Wh + min(ch0 + 16 * q + l15, n - 1);       /* columns past n are not used */
+    }
+#pragma unroll 4
+    for (int k0 = 0; k0 < n; k0 += 4) {
+        const int k = min(k0 + kq, n - 1);
+        const Real xv = xr[k];
+        const Real av = row && k0 + kq < n ? xv : (Real)0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            /* a repeated W entry meets a zero; one that is not finite is met
+             * at its own k as well */
+            const Real wv = (Real)wp[q][(size_t)k * n];
+            if constexpr (sizeof(Real) == 4) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, wv, acc[q], 0, 0, 0);
+            else acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, wv, acc[q], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            tile[(sizeof(Real) == 4 ? 4 * kq + r : kq + 4 * r) * 64 + 16 * q + l15] = acc[q][r];
 }
 
-/* MODE kLlFused: a workgroup holds all M ceil(n/64) (model, channel-block)
- * pairs of a sample range and exchanges the channel and model sums in LDS.
- * Where they do not fit one workgroup the same body runs in three passes:
- * kLlQ writes each pair's channel sum of q per sample (qbuf),
- * ll_post_kernel forms L_h, ll_t and dll_t v_ht (vbuf), and kLlGrad
- * re-evaluates the densities and accumulates the gradients. */
-template <typename Real, int MJ, bool ADJ, int MODE>
+/* One wave per (model, 64-channel block), lane = channel, over a range of
+ * samples in tiles of S.  Per component and sample, with la = log|y| in the
+ * variant's base: p = |y|^(rho-1), |y|^rho = p |y|, Q = cq - |y|^rho; the
+ * score is rho p sgn(y).  A tile's S channel sums of q reduce together
+ * (wave_totals) and cross the waves through one double-buffered LDS slot and
+ * one barrier, after which every wave evaluates the model posteriors of the
+ * tile for itself (row = sample, lane in row = model): no second barrier, and
+ * the tile's densities stay in registers for the gradient sums.  Those are
+ * FP64 throughout; the factors rho, sqrt(beta), psi are applied to the totals.
+ * The next tile's b (and dll) are loaded before a tile's arithmetic.  Bound by
+ * VALU issue (three transcendentals and, on the adjoint, 12 FP64 operations
+ * and conversions per component). */
+template <typename Real, int MJ, bool ADJ, int MODE, int BSRC>
 __global__ __launch_bounds__(512) void ll_kernel(AdjArgs a) {
-    constexpr int S = Tile<Real>::S;
+    constexpr int S = tile_samples<Real, MJ, ADJ>();
+    using B = Base<Real>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int n = a.n, NP = a.NP, M = a.M;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, nw = blockDim.x >> 6;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int CW = NP / 64;
-    int h, pair = 0;
-    bool wreal = true;   /* wave-uniform: the wave owns a real pair */
-    if constexpr (MODE == kLlFused) {
-        h = wv / CW;
-        pair = wv;
-    } else {
-        pair = blockIdx.y * a.pg + wv;
-        wreal = pair < M * CW;
-        if (!wreal) pair = M * CW - 1;
-        h = pair / CW;
+    int pair = wv;
+    if constexpr (MODE == kLlQ || MODE == kLlGrad) {
+        pair = (int)blockIdx.y * a.pg + wv;
+        if (pair >= M * CW) return;                  /* no barriers in these modes */
     }
+    const int h = pair / CW;
     const int i = (pair - h * CW) * 64 + lane;
-    const bool act = wreal && i < n;
-    /* LDS: xs[S][NP] (Real), qp[S][nw], Lh[S][M], vh[S][M] (double) */
-    Real* xs = (Real*)smem_raw;
-    double* qp = (double*)(smem_raw + (size_t)S * NP * sizeof(Real));
-    double* Lh = qp + S * nw;
-    double* vh = Lh + S * M;
+    const bool act = i < n;
+    /* LDS: qp[2][S][nw] (double), and with BSRC 1 a [16][64] tile per wave */
+    double* qp = (double*)smem_raw;
+    Real* tile = (Real*)(qp + 2 * S * nw) + wv * 1024;
 
-    Real sb[MJ], mu[MJ], rho[MJ], cq[MJ];
-    double psi1[ADJ ? MJ : 1], al[ADJ ? MJ : 1], be[ADJ ? MJ : 1], sbd[ADJ ? MJ : 1], rhod[ADJ ? MJ : 1];
+    Real sb[MJ], mu[MJ], rm1[MJ], cq[MJ];
+    double sbr[ADJ ? MJ : 1];
 #pragma unroll
     for (int j = 0; j < MJ; ++j) {
         const size_t e = ((size_t)h * MJ + j) * n + (act ? i : 0);
-        sb[j] = (Real)sqrt(a.beta[e]);
+        const double be = a.beta[e], rh = a.rho[e];
+        sb[j] = (Real)sqrt(be);
         mu[j] = (Real)a.mu[e];
-        rho[j] = (Real)a.rho[e];
-        cq[j] = (Real)a.cq[e];
-        if constexpr (ADJ) {
-            psi1[j] = psi_dev(1.0 + 1.0 / a.rho[e]);
-            al[j] = a.alpha[e];
-            be[j] = a.beta[e];
-            sbd[j] = sqrt(a.beta[e]);
-            rhod[j] = a.rho[e];
-        }
+        rm1[j] = (Real)(rh - 1.0);
+        cq[j] = (Real)(a.cq[e] * B::kUnit);
+        if constexpr (ADJ) sbr[j] = sqrt(be) * rh;
     }
-    const Real wci = (Real)a.wc[(size_t)h * NP + i];
-    const double* Wh = a.W + (size_t)h * n * n;
-    /* per component: sum u, sum u f, sum u f y, sum u |y|^rho ln|y|; the
-     * gradients are these times per-(h, j, i) constants, applied at the end */
-    double su[ADJ ? MJ : 1], suf[ADJ ? MJ : 1], sufy[ADJ ? MJ : 1], surl[ADJ ? MJ : 1];
+    const Real wci = BSRC ? (Real)a.wc[(size_t)h * NP + i] : (Real)0;
+    /* lane (row, hh): the constant of model hh */
+    const int hh = lane & 15, row = lane >> 4;
+    double lc = -HUGE_VAL;
+    if constexpr (MODE == kLlFused || MODE == kLlM1)
+        if (hh < M) lc = log(a.gm[hh]) - a.ldet[hh] + a.ldetS;
+    double su[ADJ ? MJ : 1], sup[ADJ ? MJ : 1], suy[ADJ ? MJ : 1], sul[ADJ ? MJ : 1];
     double gsum = 0.0, om = 0.0;
 #pragma unroll
-    for (int j = 0; j < (ADJ ? MJ : 1); ++j) su[j] = suf[j] = sufy[j] = surl[j] = 0.0;
+    for (int j = 0; j < (ADJ ? MJ : 1); ++j) su[j] = sup[j] = suy[j] = sul[j] = 0.0;
 
     const long t0 = (long)blockIdx.x * a.chunk;
     const long t1 = min(a.T, t0 + a.chunk);
-    const Real* x = (const Real*)a.x;
-    const Real* const bb = (const Real*)a.bbuf;
-    const size_t bcol = (size_t)h * NP + i, ldb = (size_t)M * NP;
-    for (long tb = t0; tb < t1; tb += S) {
-        Real bv[S];
-        if (bb) {                                    /* block-uniform */
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const long t = tb + s;
-                bv[s] = (act && t < t1) ? bb[(size_t)t * ldb + bcol] : (Real)0;
-            }
-        } else {
-            for (int q = tid; q < S * NP; q += blockDim.x) {
-                const int s = q / NP, k = q - (q / NP) * NP;
-                const long t = tb + s;
-                xs[q] = (t < t1 && k < n) ? x[(size_t)t * n + k] : (Real)0;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int s = 0; s < S; ++s) bv[s] = (Real)0;
-            if (act)
-                for (int k = 0; k < n; ++k) {
-                    const Real wik = (Real)Wh[i + (long)k * n];
-#pragma unroll
-                    for (int s = 0; s < S; ++s) bv[s] = fma(wik, xs[s * NP + k], bv[s]);
-                }
-#pragma unroll
-            for (int s = 0; s < S; ++s) bv[s] -= wci;
-        }
-        if constexpr (MODE != kLlGrad) {
+    const size_t ldb = (size_t)M * NP;
+    const Real* const bb = (const Real*)a.bbuf + (size_t)h * NP + i;
+    Real bn[S];
+    double dn[ADJ ? S : 1];
+    auto load = [&](long tb) {
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            double q = 0.0;
-            if (act) {
-                Real Qj[MJ], mx = (Real)0;
-#pragma unroll
-                for (int j = 0; j < MJ; ++j) {
-                    Real y, yr, lny;
-                    density<Real>(bv[s], sb[j], mu[j], rho[j], cq[j], y, Qj[j], yr, lny);
-                    mx = (j == 0) ? Qj[j] : fmax(mx, Qj[j]);
-                }
-                Real se = (Real)0;
-#pragma unroll
-                for (int j = 0; j < MJ; ++j) se += r_exp<Real>(Qj[j] - mx);
-                q = (double)mx + (double)r_log<Real>(se);
+            const long t = min(tb + s, t1 - 1);      /* past the range: the last sample again, weight 0 */
+            if constexpr (BSRC == 0) bn[s] = bb[(size_t)t * ldb];
+            if constexpr (ADJ && MODE == kLlGrad) dn[s] = a.vbuf[(size_t)t * M + h];
+            if constexpr (ADJ && MODE == kLlM1) dn[s] = a.dll[t];
+        }
+        if constexpr (ADJ && MODE == kLlFused) dn[0] = a.dll[min(tb + min(row, S - 1), t1 - 1)];
+    };
+    load(t0);
+    int buf = 0;
+    for (long tb = t0; tb < t1; tb += S) {
+        Real bv[S];
+        double dv[ADJ ? S : 1];
+        if constexpr (BSRC == 1) {
+            if (((tb - t0) & 15) == 0) {
+                unmix_tile<Real>(a, a.W + (size_t)h * n * n, (pair - h * CW) * 64, tb, tile);
+                __builtin_amdgcn_wave_barrier();
             }
-            q = wave_sum_f64(q);
-            if constexpr (MODE == kLlQ) {
-                const long t = tb + s;
-                if (lane == 0 && wreal && t < t1) a.qbuf[(size_t)t * M * CW + pair] = q;
-            } else if constexpr (MODE == kLlFused) {
-                if (lane == 0) qp[s * nw + wv] = q;
-            }
-        }
-        }
-        if constexpr (MODE == kLlQ) {
-            __syncthreads();            /* xs is rewritten by the next tile */
-            continue;
-        }
-        if constexpr (MODE == kLlFused) {
-        __syncthreads();
-        if (tid < S * M) {
-            const int s = tid / M, hh = tid - (tid / M) * M;
-            double L = log(a.gm[hh]) + a.ldet[hh] + a.ldetS;
-            for (int c = 0; c < CW; ++c) L += qp[s * nw + hh * CW + c];
-            Lh[s * M + hh] = L;
-        }
-        __syncthreads();
-        if (tid < S) {
-            const int s = tid;
-            const long t = tb + s;
-            double mx = Lh[s * M];
-            for (int hh = 1; hh < M; ++hh) mx = fmax(mx, Lh[s * M + hh]);
-            double se = 0.0;
-            for (int hh = 0; hh < M; ++hh) se += exp(Lh[s * M + hh] - mx);
-            const double P = mx + log(se);
-            const bool valid = t < t1;
-            if (valid && a.ll) a.ll[t] = P;
-            const double w = (ADJ && valid) ? a.dll[t] : 0.0;
-            for (int hh = 0; hh < M; ++hh) vh[s * M + hh] = w * exp(Lh[s * M + hh] - P);
-        }
-        __syncthreads();
+#pragma unroll
+            for (int s = 0; s < S; ++s) bv[s] = tile[(((tb - t0) & 15) + s) * 64 + lane] - wci;
+            __builtin_amdgcn_wave_barrier();
+        } else {
+#pragma unroll
+            for (int s = 0; s < S; ++s) bv[s] = bn[s];
         }
         if constexpr (ADJ) {
-            Real* g = (Real*)a.g;
-            const size_t ldg = (size_t)M * NP;
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const long t = tb + s;
-                if (t >= t1) break;
-                double omh;
-                if constexpr (MODE == kLlGrad) omh = a.vbuf[(size_t)t * M + h];
-                else omh = vh[s * M + h];
-                double gv = 0.0;
-                if (act) {
-                    Real Qj[MJ], Yj[MJ], YRj[MJ], LNj[MJ], mx = (Real)0;
+            for (int s = 0; s < S; ++s) dv[s] = dn[s];
+        }
+        load(tb + S);
+        /* densities */
+        Real ez[S][MJ], ps[S][MJ], yr[S][MJ], la[S][MJ], rse[S];
+        double q[S];
 #pragma unroll
-                    for (int j = 0; j < MJ; ++j) {
-                        density<Real>(bv[s], sb[j], mu[j], rho[j], cq[j], Yj[j], Qj[j], YRj[j], LNj[j]);
-                        mx = (j == 0) ? Qj[j] : fmax(mx, Qj[j]);
-                    }
-                    Real ez[MJ], se = (Real)0;
+        for (int s = 0; s < S; ++s) {
+            Real Qj[MJ], mx = (Real)0, se = (Real)0;
 #pragma unroll
-                    for (int j = 0; j < MJ; ++j) {
-                        ez[j] = r_exp<Real>(Qj[j] - mx);
-                        se += ez[j];
-                    }
-                    const Real rse = r_rcp<Real>(se);
+            for (int j = 0; j < MJ; ++j) {
+                const Real y = sb[j] * (bv[s] - mu[j]);
+                const Real ay = fmax(fabs(y), B::kTiny);
+                la[s][j] = B::log(ay);
+                const Real p = B::exp(rm1[j] * la[s][j]);         /* |y|^(rho-1) */
+                yr[s][j] = p * ay;
+                if constexpr (ADJ) ps[s][j] = y > (Real)0 ? p : y < (Real)0 ? -p : y;   /* 0 at 0, NaN stays */
+                Qj[j] = fma(yr[s][j], (Real)-B::kUnit, cq[j]);
+                mx = (j == 0) ? Qj[j] : fmax(mx, Qj[j]);
+            }
 #pragma unroll
-                    for (int j = 0; j < MJ; ++j) {
-                        const double u = omh * (double)(ez[j] * rse);
-                        /* f y = rho |y|^rho and f = f y / y (0 at y = 0) */
-                        const Real fy = rho[j] * YRj[j];
-                        const Real f = (Yj[j] == (Real)0) ? (Real)0 : fy * r_rcp<Real>(Yj[j]);
-                        const double uf = u * (double)f;
-                        su[j] += u;
-                        suf[j] += uf;
-                        sufy[j] += u * (double)fy;
-                        surl[j] += u * ((double)YRj[j] * (double)LNj[j]);
-                        gv += sbd[j] * uf;
+            for (int j = 0; j < MJ; ++j) {
+                ez[s][j] = B::exp(Qj[j] - mx);
+                se += ez[s][j];
+            }
+            if constexpr (ADJ) rse[s] = B::rcp(se);
+            if constexpr (MODE != kLlGrad) q[s] = act ? (double)mx + (double)B::log(se) : 0.0;
+        }
+        /* channel sums, and per sample the models' log-sum-exp */
+        double w = 0.0;                              /* lane (row, hh): dll v of sample row, model hh */
+        if constexpr (MODE != kLlGrad) {
+            const double tot = wave_totals<S>(q) * B::kLn;
+            const int ts = sample_of_row<S>(row);
+            if constexpr (MODE == kLlQ) {
+                if (hh == 0 && tb + ts < t1) a.qbuf[(size_t)(tb + ts) * M * CW + pair] = tot;
+            } else {
+                if (hh == 0) qp[(buf * S + ts) * nw + wv] = tot;
+                __syncthreads();
+                if (MODE == kLlFused || wv == 0) {
+                    const int sr = min(row, S - 1);
+                    double L = lc;
+                    if (hh < M)
+                        for (int c = 0; c < CW; ++c) L += qp[(buf * S + sr) * nw + hh * CW + c];
+                    const bool out = a.ll && wv == 0 && hh == 0 && row < S && tb + row < t1;
+                    if constexpr (MODE == kLlM1) {
+                        if (out) a.ll[tb + row] = L;
+                    } else {
+                        const double mx = row_max(L);
+                        const double e = exp(L - mx), se = row_sum(e);
+                        if (ADJ) w = tb + row < t1 ? dv[0] * (e / se) : 0.0;
+                        if (wv == 0) {
+                            const double P = mx + log(se);
+                            if (out) a.ll[tb + row] = P;
+                        }
                     }
                 }
-                if (wreal) g[(size_t)t * ldg + (size_t)h * NP + i] = (Real)gv;
-                gsum += gv;
-                if (i == 0) om += omh;
+                buf ^= 1;
             }
         }
-        __syncthreads();
+        if constexpr (ADJ) {
+            Real* g = (Real*)a.g + (size_t)h * NP + i;
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const bool in = tb + s < t1;         /* uniform */
+                double omh;
+                if constexpr (MODE == kLlFused) omh = readlane_f64(w, 16 * s + h);
+                else omh = in ? dv[s] : 0.0;
+                double gv = 0.0;
+#pragma unroll
+                for (int j = 0; j < MJ; ++j) {
+                    const double u = omh * (double)(ez[s][j] * rse[s]);
+                    const double up = u * (double)ps[s][j], uy = u * (double)yr[s][j];
+                    su[j] += u;
+                    sup[j] += up;
+                    suy[j] += uy;
+                    sul[j] = fma(uy, (double)la[s][j], sul[j]);
+                    gv = fma(sbr[j], up, gv);
+                }
+                if (!act) gv = 0.0;
+                if (in) g[(size_t)(tb + s) * ldb] = (Real)gv;
+                gsum += gv;
+                om += omh;
+            }
+        }
     }
     if constexpr (ADJ && MODE != kLlQ) {
-        if (!wreal) return;
         double* base = a.part + (size_t)blockIdx.x * a.pstride;
         double* pp = base + ((size_t)h * NP + i) * pair_stride(MJ);
-        /* dalpha = sum u / alpha, dmu = sqrt(beta) sum u f,
-         * dbeta = sum u (1 - f y) / (2 beta),
-         * drho = sum u (psi(1 + 1/rho) / rho^2 - |y|^rho ln|y|) */
 #pragma unroll
         for (int j = 0; j < MJ; ++j) {
-            pp[j] = su[j] / al[j];
-            pp[MJ + j] = sbd[j] * suf[j];
-            pp[2 * MJ + j] = (su[j] - sufy[j]) / (2.0 * be[j]);
-            pp[3 * MJ + j] = su[j] * psi1[j] / (rhod[j] * rhod[j]) - surl[j];
+            pp[j] = su[j];
+            pp[MJ + j] = sup[j];
+            pp[2 * MJ + j] = suy[j];
+            pp[3 * MJ + j] = sul[j] * B::kLn;
         }
         pp[4 * MJ] = gsum;
         if (i == 0) base[(size_t)M * NP * pair_stride(MJ) + h] = om;
@@ -361,94 +443,104 @@ __global__ __launch_bounds__(256) void ll_post_kernel(AdjArgs a) {
     if (t >= a.T) return;
     const int M = a.M, CW = a.NP / 64;
     const double* q = a.qbuf + (size_t)t * M * CW;
+    auto model = [&](int hh) {
+        double L = log(a.gm[hh]) - a.ldet[hh] + a.ldetS;
+        for (int c = 0; c < CW; ++c) L += q[hh * CW + c];
+        return L;
+    };
     double mx = -HUGE_VAL;
-    for (int hh = 0; hh < M; ++hh) {
-        double L = log(a.gm[hh]) + a.ldet[hh] + a.ldetS;
-        for (int c = 0; c < CW; ++c) L += q[hh * CW + c];
-        mx = fmax(mx, L);
-    }
+    for (int hh = 0; hh < M; ++hh) mx = fmax(mx, model(hh));
     double se = 0.0;
-    for (int hh = 0; hh < M; ++hh) {
-        double L = log(a.gm[hh]) + a.ldet[hh] + a.ldetS;
-        for (int c = 0; c < CW; ++c) L += q[hh * CW + c];
-        se += exp(L - mx);
-    }
+    for (int hh = 0; hh < M; ++hh) se += exp(model(hh) - mx);
     const double P = mx + log(se);
     if (a.ll) a.ll[t] = P;
     if (a.dll) {
         const double w = a.dll[t];
-        for (int hh = 0; hh < M; ++hh) {
-            double L = log(a.gm[hh]) + a.ldet[hh] + a.ldetS;
-            for (int c = 0; c < CW; ++c) L += q[hh * CW + c];
-            a.vbuf[(size_t)t * M + hh] = w * exp(L - P);
-        }
+        for (int hh = 0; hh < M; ++hh) a.vbuf[(size_t)t * M + hh] = w * exp(model(hh) - P);
     }
 }
 
-/* part[chunk][r][k] = sum_{t in chunk} g[t][r] x[t][k]   (r < M NP, k < n) */
-template <typename Real>
-__global__ __launch_bounds__(256) void adj_gx_kernel(const Real* __restrict__ g,
-                                                     const Real* __restrict__ x, long T, int n,
-                                                     int ldg, long chunk, double* __restrict__ part) {
-    __shared__ double ga[32][64];
-    __shared__ double xb[32][64];
-    const int tid = threadIdx.x;
+/* FP64 statistic GEMM part[chunk][r][k] = sum_{t in chunk} g[t][r] x[t][k]
+ * (r < ldg, k < n) on the FP64 MFMA units: 64 x 64 per workgroup, whose four
+ * waves take every fourth group of two 4-sample steps and add their tiles
+ * through LDS in wave order; fragments come straight from memory, a group
+ * ahead. */
+__global__ __launch_bounds__(256, 2) void adj_gx_kernel(const double* __restrict__ g,
+                                                        const double* __restrict__ x, long T, int n, int ldg,
+                                                        long chunk, double* __restrict__ part) {
+    constexpr int kU = 2;
+    __shared__ double sum[16][256];
+    const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, kq = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rb = blockIdx.y * 64, kb = blockIdx.z * 64;
     const long ts = (long)blockIdx.x * chunk, te = min(T, ts + chunk);
-    const int ti = (tid & 15) * 4, tk = (tid >> 4) * 4;
-    double acc[4][4];
+    int ck[4];
+    bool vk[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int k = kb + 16 * q + l15;
+        vk[q] = k < n;
+        ck[q] = vk[q] ? k : n - 1;
+    }
+    f64x4 acc[4][4];
 #pragma unroll
     for (int p = 0; p < 4; ++p)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[p][q] = 0.0;
-    for (long t0 = ts; t0 < te; t0 += 32) {
-        for (int q = tid; q < 32 * 64; q += 256) {
-            const int s = q >> 6, col = q & 63;
-            const long t = t0 + s;
-            double va = 0.0, vb = 0.0;
-            if (t < te) {
-                if (rb + col < ldg) va = (double)g[(size_t)t * ldg + rb + col];
-                if (kb + col < n) vb = (double)x[(size_t)t * n + kb + col];
+        for (int q = 0; q < 4; ++q) acc[p][q] = (f64x4){0.0, 0.0, 0.0, 0.0};
+    double fa[kU][4], fb[kU][4];
+    auto load = [&](long t0) {
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const long t = t0 + 4 * u + kq, tc = t < te ? t : te - 1;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                fa[u][p] = g[(size_t)tc * ldg + rb + 16 * p + l15];
+                fb[u][p] = x[(size_t)tc * n + ck[p]];
             }
-            ga[s][col] = va;
-            xb[s][col] = vb;
         }
-        __syncthreads();
-        for (int s = 0; s < 32; ++s) {
-            double av[4], bv[4];
+    };
+    const long step = 4 * 4 * kU;
+    long t0 = ts + (long)w * 4 * kU;
+    if (t0 < te) load(t0);
+    for (; t0 < te; t0 += step) {
+        double av[kU][4], bv[kU][4];
 #pragma unroll
-            for (int p = 0; p < 4; ++p) av[p] = ga[s][ti + p];
+        for (int u = 0; u < kU; ++u) {
+            const bool ok = t0 + 4 * u + kq < te;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) bv[q] = xb[s][tk + q];
+            for (int p = 0; p < 4; ++p) {
+                av[u][p] = ok ? fa[u][p] : 0.0;
+                bv[u][p] = ok && vk[p] ? fb[u][p] : 0.0;
+            }
+        }
+        if (t0 + step < te) load(t0 + step);
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
 #pragma unroll
             for (int p = 0; p < 4; ++p)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc[p][q] = fma(av[p], bv[q], acc[p][q]);
+                for (int q = 0; q < 4; ++q)
+                    acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u][p], bv[u][q], acc[p][q], 0, 0, 0);
+    }
+    for (int v = 0; v < 4; ++v) {
+        if (v == w) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        double* s = &sum[p * 4 + q][(kq + 4 * r) * 16 + l15];
+                        *s = v == 0 ? acc[p][q][r] : *s + acc[p][q][r];
+                    }
         }
         __syncthreads();
     }
     double* out = part + (size_t)blockIdx.x * ldg * n;
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int r = rb + ti + p, k = kb + tk + q;
-            if (r < ldg && k < n) out[(size_t)r * n + k] = acc[p][q];
-        }
-}
-
-/* The unmixing GEMM's operands: Wg[h NP + i][k] = W_h[i][k] (zero past n)
- * and W c in the GEMM's precision. */
-template <typename Real>
-__global__ __launch_bounds__(256) void adj_wg_kernel(AdjArgs a, Real* __restrict__ Wg,
-                                                     Real* __restrict__ wcr) {
-    const int NP = a.NP, n = a.n;
-    const long total = (long)a.M * NP * NP;
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (long)gridDim.x * blockDim.x) {
-        const long r = q / NP;
-        const int k = (int)(q - r * NP), h = (int)(r / NP), i = (int)(r - (long)h * NP);
-        Wg[q] = (i < n && k < n) ? (Real)a.W[(size_t)h * n * n + (size_t)k * n + i] : (Real)0;
-        if (k == 0) wcr[r] = (Real)a.wc[r];
+    for (int t = 0; t < 16; ++t) {
+        const int r = rb + (t >> 2) * 16 + (tid >> 4), k = kb + (t & 3) * 16 + (tid & 15);
+        if (k < n) out[(size_t)r * n + k] = sum[t][tid];
     }
 }
 
@@ -464,92 +556,69 @@ __global__ __launch_bounds__(256) void adj_pad_kernel(const Real* __restrict__ x
     }
 }
 
-/* Fixed-order sums over slots: out[e] = sum_{b < nslots} in[b stride + e]
- * for e < count, one thread per entry (consecutive entries coalesce). */
-__global__ __launch_bounds__(256) void adj_slot_sum_kernel(const double* __restrict__ in, size_t stride,
-                                                           int nslots, size_t count,
-                                                           double* __restrict__ out) {
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < count;
-         e += (size_t)gridDim.x * blockDim.x) {
-        double acc = 0.0;
-        for (int b = 0; b < nslots; ++b) acc += in[(size_t)b * stride + e];
-        out[e] = acc;
-    }
-}
-
 struct AdjOut {
     double *dW, *dc, *dalpha, *dmu, *dbeta, *drho, *dgm;
 };
 
-/* One workgroup per model: fixed-order sums over the ll workgroups and the
- * gx chunks, then the gradients. */
-__global__ __launch_bounds__(256) void adj_finish_kernel(AdjArgs a, int nblocks,
-                                                         const double* __restrict__ gxpart,
-                                                         int nchunks, int gxs, AdjOut o) {
-    extern __shared__ double gs[];   /* gsum_h[n] */
-    __shared__ double om_sh;
-    const int h = blockIdx.x, n = a.n, m = a.m, NP = a.NP, M = a.M;
-    const int ps = pair_stride(m);
-    const long nm = (long)n * m;
-    for (long q = threadIdx.x; q < nm + n; q += blockDim.x) {
-        /* q < nm: (j, i) of the four per-component gradients; then gsum_i */
-        const int j = q < nm ? (int)(q / n) : 0;
-        const int i = q < nm ? (int)(q % n) : (int)(q - nm);
-        const size_t off = ((size_t)h * NP + i) * ps;
-        if (q < nm) {
-            double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-            for (int b = 0; b < nblocks; ++b) {
-                const double* pp = a.part + (size_t)b * a.pstride + off;
-                s0 += pp[j];
-                s1 += pp[m + j];
-                s2 += pp[2 * m + j];
-                s3 += pp[3 * m + j];
-            }
-            const size_t e = (size_t)h * nm + q;
-            o.dalpha[e] = s0;
-            o.dmu[e] = s1;
-            o.dbeta[e] = s2;
-            o.drho[e] = s3;
+/* The gradients from the totals of the raw sums (raw, nc sets of pcount, one
+ * per chunk of samples) and of sum_t g_t x_t^T (G, nc sets of ldg gxs).  Grid
+ * (eb + n / 4, M): workgroups below eb take dW and the densities' gradients,
+ * the others four entries of dc, one per wave. */
+__global__ __launch_bounds__(256) void adj_finish_kernel(AdjArgs a, int eb, const double* __restrict__ raw,
+                                                         size_t pcount, const double* __restrict__ G, int gxs,
+                                                         int nc, AdjOut o) {
+    const int h = blockIdx.y, n = a.n, m = a.m, NP = a.NP, ps = pair_stride(m);
+    const int nm = n * m, nn = n * n;
+    const size_t ldg = (size_t)a.M * NP;
+    auto total = [&](size_t e) {
+        double s = 0.0;
+        for (int c = 0; c < nc; ++c) s += raw[(size_t)c * pcount + e];
+        return s;
+    };
+    auto gsum = [&](int i) { return total(((size_t)h * NP + i) * ps + 4 * m); };
+    const double* W = a.W + (size_t)h * nn;
+    if ((int)blockIdx.x >= eb) {
+        const int lane = threadIdx.x & 63, k = ((int)blockIdx.x - eb) * 4 + ((int)threadIdx.x >> 6);
+        if (k >= n) return;
+        double s = 0.0;
+        for (int i = lane; i < n; i += 64) s += W[i + (size_t)k * n] * gsum(i);
+        s = wave_sum_f64(s);
+        if (lane == 0) o.dc[(size_t)h * n + k] = s;
+        return;
+    }
+    const double om = total((size_t)ldg * ps + h);
+    for (int q = (int)blockIdx.x * 256 + threadIdx.x; q < nn + nm; q += eb * 256) {
+        if (q >= nn) {
+            const int e0 = q - nn, j = e0 / n, i = e0 - j * n;
+            const size_t e = (size_t)h * nm + e0, off = ((size_t)h * NP + i) * ps + j;
+            const double be = a.beta[e], rh = a.rho[e];
+            const double su = total(off), sup = total(off + m), suy = total(off + 2 * m), sul = total(off + 3 * m);
+            o.dalpha[e] = su / a.alpha[e];
+            o.dmu[e] = sqrt(be) * rh * sup;
+            o.dbeta[e] = (su - rh * suy) / (2.0 * be);
+            o.drho[e] = su * psi_dev(1.0 + 1.0 / rh) / (rh * rh) - sul;
         } else {
+            const int i = q % n, k = q / n;
             double s = 0.0;
-            for (int b = 0; b < nblocks; ++b) s += a.part[(size_t)b * a.pstride + off + 4 * m];
-            gs[i] = s;
+            for (int c = 0; c < nc; ++c) s += G[((size_t)c * ldg + (size_t)h * NP + i) * gxs + k];
+            o.dW[(size_t)h * nn + q] = om * a.Winv[(size_t)h * nn + k + (size_t)i * n] -
+                                       (s - gsum(i) * a.c[(size_t)h * n + k]);
         }
     }
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int b = 0; b < nblocks; ++b) s += a.part[(size_t)b * a.pstride + (size_t)M * NP * ps + h];
-        om_sh = s;
-        o.dgm[h] = s / a.gm[h];
-    }
-    __syncthreads();
-    const double om = om_sh;
-    const long nn = (long)n * n;
-    const double* W = a.W + (size_t)h * nn;
-    const double* Wi = a.Winv + (size_t)h * nn;
-    const double* c = a.c + (size_t)h * n;
-    const size_t ldg = (size_t)M * NP;
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
-        double s = 0.0;
-        for (int i = 0; i < n; ++i) s += W[i + (long)k * n] * gs[i];
-        o.dc[(size_t)h * n + k] = s;
-    }
-    for (long q = threadIdx.x; q < nn; q += blockDim.x) {
-        const int i = (int)(q % n), k = (int)(q / n);
-        double G = 0.0;
-        for (int ch = 0; ch < nchunks; ++ch) G += gxpart[((size_t)ch * ldg + (size_t)h * NP + i) * gxs + k];
-        o.dW[(size_t)h * nn + q] = om * Wi[k + (long)i * n] - (G - gs[i] * c[k]);
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) o.dgm[h] = om / a.gm[h];
 }
 
-template <typename Real, bool ADJ, int MODE>
-int launch_ll_mode(int MJ, const AdjArgs& a, dim3 grid, dim3 block, size_t shm, hipStream_t st) {
+template <typename Real, bool ADJ, int MODE, int BSRC>
+int launch_ll_mode(int MJ, const AdjArgs& a, dim3 grid, dim3 block, hipStream_t st) {
+    const size_t nw = block.x / 64;
+    const size_t shm = 2 * 4 * nw * 8 + (BSRC ? nw * 1024 * sizeof(Real) : 0);
 #define AMICA_LL_CASE(J)                                                                           \
     case J:                                                                                        \
-        if (hipFuncSetAttribute((const void*)ll_kernel<Real, J, ADJ, MODE>,                        \
+        if (shm > 65536 &&                                                                         \
+            hipFuncSetAttribute((const void*)ll_kernel<Real, J, ADJ, MODE, BSRC>,                  \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm) != hipSuccess) \
             return -1;                                                                             \
-        hipLaunchKernelGGL((ll_kernel<Real, J, ADJ, MODE>), grid, block, shm, st, a);             \
+        hipLaunchKernelGGL((ll_kernel<Real, J, ADJ, MODE, BSRC>), grid, block, shm, st, a);        \
         break;
     switch (MJ) {
         AMICA_LL_CASE(1)
@@ -567,46 +636,138 @@ int launch_ll_mode(int MJ, const AdjArgs& a, dim3 grid, dim3 block, size_t shm, 
 }
 
 template <typename Real, bool ADJ>
-int launch_ll(int MJ, const AdjArgs& a, int nblocks, size_t shm, hipStream_t st) {
+int launch_ll(int MJ, const AdjArgs& a, int nblocks, hipStream_t st) {
     const int pairs = a.M * (a.NP / 64);
-    if (!a.qbuf)
-        return launch_ll_mode<Real, ADJ, kLlFused>(MJ, a, dim3(nblocks), dim3(64 * pairs), shm, st);
+    if (!a.qbuf) {
+        const dim3 grid(nblocks), block(64 * pairs);
+        if constexpr (!ADJ)
+            if (!a.bbuf)
+                return a.M == 1 ? launch_ll_mode<Real, ADJ, kLlM1, 1>(MJ, a, grid, block, st)
+                                : launch_ll_mode<Real, ADJ, kLlFused, 1>(MJ, a, grid, block, st);
+        return a.M == 1 ? launch_ll_mode<Real, ADJ, kLlM1, 0>(MJ, a, grid, block, st)
+                        : launch_ll_mode<Real, ADJ, kLlFused, 0>(MJ, a, grid, block, st);
+    }
     const dim3 grid(nblocks, (pairs + a.pg - 1) / a.pg), block(64 * a.pg);
-    const size_t shx = (size_t)Tile<Real>::S * a.NP * sizeof(Real);
-    if (launch_ll_mode<Real, false, kLlQ>(MJ, a, grid, block, shx, st)) return -1;
+    if (launch_ll_mode<Real, false, kLlQ, 0>(MJ, a, grid, block, st)) return -1;
     hipLaunchKernelGGL(ll_post_kernel, dim3((unsigned)((a.T + 255) / 256)), dim3(256), 0, st, a);
     if (hipGetLastError() != hipSuccess) return -1;
-    return ADJ ? launch_ll_mode<Real, true, kLlGrad>(MJ, a, grid, block, shx, st) : 0;
+    return ADJ ? launch_ll_mode<Real, true, kLlGrad, 0>(MJ, a, grid, block, st) : 0;
 }
 
-/* Workspace of one call, freed on every exit path. */
-struct Workspace {
-    static constexpr int kMax = 20;
-    void* ptrs[kMax] = {nullptr};
-    int n = 0;
+/* One block of device memory per call, from a pool that outlives it: hipMalloc
+ * and hipFree of a call's buffers took longer than its kernels (up to 30 ms for
+ * a gigabyte).  A call owns its block until its stream has drained (the
+ * destructor waits where the call did not), so blocks in the pool are idle and
+ * any thread and stream may take one.  At most kPoolBlocks stay per device, of
+ * kPoolBytes in all; the rest, and every idle block when an allocation fails,
+ * goes back to the device. */
+constexpr size_t kPoolBytes = (size_t)1 << 30;
+constexpr int kPoolBlocks = 2;
+
+struct PoolBlock {
+    int dev;
+    void* p;
+    size_t bytes;
+};
+std::mutex g_pool_mu;
+std::vector<PoolBlock> g_pool;
+
+class Workspace {
+public:
+    Workspace(int dev, hipStream_t st) : dev_(dev), st_(st) {}
+    Workspace(const Workspace&) = delete;
+    Workspace& operator=(const Workspace&) = delete;
     ~Workspace() {
-        for (int k = 0; k < n; ++k) (void)hipFree(ptrs[k]);
+        if (!b_.p) return;
+        if (!drained_) (void)hipStreamSynchronize(st_);
+        std::vector<void*> drop;
+        {
+            std::lock_guard<std::mutex> lock(g_pool_mu);
+            g_pool.push_back(b_);
+            /* the smallest blocks leave first */
+            for (;;) {
+                size_t sum = 0, least = 0;
+                int cnt = 0;
+                for (size_t k = 0; k < g_pool.size(); ++k) {
+                    if (g_pool[k].dev != dev_) continue;
+                    if (!cnt || g_pool[k].bytes < g_pool[least].bytes) least = k;
+                    sum += g_pool[k].bytes;
+                    ++cnt;
+                }
+                if (cnt <= kPoolBlocks && sum <= kPoolBytes) break;
+                drop.push_back(g_pool[least].p);
+                g_pool.erase(g_pool.begin() + least);
+            }
+        }
+        for (void* p : drop) (void)hipFree(p);
     }
-    bool alloc(void** p, size_t bytes) {
-        if (n == kMax) return false;
-        if (hipMalloc(p, std::max<size_t>(bytes, 8)) != hipSuccess) return false;
-        ptrs[n++] = *p;
-        return true;
+    /* the smallest idle block of at least `bytes`, or a new one */
+    void* take(size_t bytes) {
+        bytes = (bytes + ((size_t)1 << 20) - 1) >> 20 << 20;
+        std::vector<void*> drop;
+        {
+            std::lock_guard<std::mutex> lock(g_pool_mu);
+            size_t best = g_pool.size();
+            for (size_t k = 0; k < g_pool.size(); ++k)
+                if (g_pool[k].dev == dev_ && g_pool[k].bytes >= bytes &&
+                    (best == g_pool.size() || g_pool[k].bytes < g_pool[best].bytes))
+                    best = k;
+            if (best < g_pool.size()) {
+                b_ = g_pool[best];
+                g_pool.erase(g_pool.begin() + best);
+                return b_.p;
+            }
+        }
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            {
+                std::lock_guard<std::mutex> lock(g_pool_mu);
+                for (size_t k = g_pool.size(); k-- > 0;)
+                    if (g_pool[k].dev == dev_) {
+                        drop.push_back(g_pool[k].p);
+                        g_pool.erase(g_pool.begin() + k);
+                    }
+            }
+            for (void* q : drop) (void)hipFree(q);
+            if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
+        }
+        b_ = PoolBlock{dev_, p, bytes};
+        return p;
+    }
+    void drained() { drained_ = true; }
+
+private:
+    PoolBlock b_ = {0, nullptr, 0};
+    int dev_;
+    hipStream_t st_;
+    bool drained_ = false;
+};
+
+/* The buffers of a call as offsets into its block (base null: only the size) */
+struct Carve {
+    char* base;
+    size_t off = 0;
+    template <typename T> T* take(size_t count) {
+        T* p = base ? (T*)(base + off) : nullptr;
+        off += (count * sizeof(T) + 255) / 256 * 256;
+        return p;
     }
 };
 
 /* The fixed device workspace of amica_ll_forward_noalloc (callers that
  * cannot allocate: code under hipGraph capture, tight serving loops).  It
- * holds, in doubles: W^-1, the LU and inverse scratch (M n n each), the
- * per-(h, j, i) constants (M m n), W c (M NP) and log|det W| (M).  Limits:
- * M n n <= kNoAllocNN (e.g. 256 channels x 1 model, 128 x 4), plus the
- * forward's own M ceil(n/64) 64 <= 512, m <= 8.  1.6 MB per device, held
- * until the process ends; every call on a device shares it. */
+ * holds, in doubles: W^-1 (M n n), the inverse's scratch (M n n + 8 and
+ * inverse_work_doubles), the per-(h, j, i) constants (M m n), W c (M NP) and
+ * log|det W| (M).  Limits: M n n <= kNoAllocNN (e.g. 256 channels x 1 model,
+ * 128 x 4), plus the forward's own M ceil(n/64) 64 <= 512, m <= 8.  1.6 MB per
+ * device, held until the process ends; every call on a device shares it. */
 constexpr size_t kNoAllocNN = 65536;
 constexpr size_t kNoAllocNM = 4096;        /* 8 components x 512 padded channels */
 constexpr size_t kNoAllocNP = 512;
 constexpr size_t kNoAllocM = 8;
-constexpr size_t kNoAllocDoubles = 3 * kNoAllocNN + kNoAllocNM + kNoAllocNP + kNoAllocM;
+constexpr size_t kNoAllocWork = 2 * kNoAllocNN + 8 + 2 * kNoAllocNP;   /* M n <= M NP */
+constexpr size_t kNoAllocDoubles = kNoAllocNN + kNoAllocWork + kNoAllocNM + kNoAllocNP + kNoAllocM;
 
 __device__ __align__(256) double scratch[kNoAllocDoubles];
 
@@ -631,6 +792,153 @@ int noalloc_scratch(double** out) {
         g_scratch_ptr[dev] = ptr;
     }
     *out = g_scratch_ptr[dev];
+    return 0;
+}
+
+/* W^-1, log|det W|, W c, the constants of Q and (Wg) the GEMM operands */
+template <typename Real>
+int prepare_model(const AdjArgs& a, double* work, Real* Wg, Real* wcr, hipStream_t st) {
+    if (launch_gj_inverse(a.W, a.Winv, a.ldet, a.n, a.M, work, st))
+        return report_error(AMICA_E_DEVICE, "inverse launch failed");
+    const long items = std::max((long)a.n * a.m, Wg ? (long)a.NP * a.NP : 0L);
+    const int eb = (int)std::min<long>(1024, (items + 255) / 256);
+    hipLaunchKernelGGL(adj_prep_kernel<Real>, dim3(eb + a.NP / 4, a.M), dim3(256), 0, st, a, eb, Wg, wcr);
+    return hipGetLastError() == hipSuccess ? 0 : report_error(AMICA_E_DEVICE, "prep launch failed");
+}
+
+/* Workgroups of the likelihood kernel over T samples and the samples of each
+ * (whole 16-sample groups): 16 waves per CU, which its registers allow on
+ * the forward passes; where the adjoint's allow half, the rest queue. */
+int ll_grid(long T, int pairs, int cus, long* chunk) {
+    const long waves = pairs <= 8 ? pairs : 8L * ((pairs + 7) / 8);
+    const long nb = std::max(1L, std::min(16L * cus / waves, (T + 15) / 16));
+    *chunk = ((T + nb - 1) / nb + 15) / 16 * 16;
+    return (int)((T + *chunk - 1) / *chunk);
+}
+
+/* b is formed in the likelihood kernel, 16 samples at a time on MFMA: nothing
+ * of the size of the data is stored, and the call only enqueues. */
+template <typename Real>
+int forward_noalloc(AdjArgs a, const void* x, long T, double* ll, double* work, int cus, hipStream_t st) {
+    const int rc = prepare_model<Real>(a, work, nullptr, nullptr, st);
+    if (rc) return rc;
+    a.x = x;
+    a.T = T;
+    a.ll = ll;
+    const int nb = ll_grid(T, a.M * (a.NP / 64), cus, &a.chunk);
+    return launch_ll<Real, false>(a.m, a, nb, st) ? report_error(AMICA_E_DEVICE, "likelihood kernel launch failed")
+                                                  : 0;
+}
+
+/* Per-sample buffers (b, g, padded x) of one chunk of samples: small enough
+ * that what one kernel writes the next reads from the 256 MB last-level
+ * cache, large enough that a chunk's launches fill the GPU. */
+constexpr size_t kChunkBytes = (size_t)256 << 20;
+
+template <typename Real>
+int run_chunks(AdjArgs a, const void* x, long T, const double* dll, double* ll, const AdjOut* out, bool split,
+               int dev, int cus, hipStream_t st) {
+    const bool adj = out != nullptr;
+    const int n = a.n, NP = a.NP, M = a.M, m = a.m, ldb = M * NP, pairs = ldb / 64;
+    const size_t nn = (size_t)n * n;
+    constexpr size_t rb = sizeof(Real);
+    const size_t per = rb * ((size_t)ldb * (adj ? 2 : 1) + (n != NP ? NP : 0)) + (split ? 8 * (size_t)(pairs + M) : 0);
+    const long most = std::max(4096L, (long)(kChunkBytes / per));
+    const long nc = (T + most - 1) / most;
+    const long Tc = nc == 1 ? T : ((T + nc - 1) / nc + 63) / 64 * 64;
+    const int C = (int)((T + Tc - 1) / Tc);
+    const int nb = ll_grid(Tc, pairs, cus, &a.chunk);
+    /* the statistic GEMM sum_t g_t x_t^T: FP32 MFMA over padded rows of x
+     * (gx_f32_slab_kernel, row stride NP) on the FP32 variant, FP64 MFMA over
+     * the unpadded rows (row stride n) on the FP64 one */
+    const bool gx32 = rb == 4;
+    const int slabs = (ldb / 64) * ((n + 63) / 64);
+    const int gchunks = gx32 ? gx_f32_chunks(Tc, NP, ldb, cus)
+                             : (int)std::max(1L, std::min(std::max(1L, 2L * cus / slabs), (Tc + 255) / 256));
+    const int gxs = gx32 ? NP : n;
+    const size_t pcount = (size_t)ldb * pair_stride(m) + M, gcount = (size_t)ldb * gxs;
+    Workspace ws(dev, st);
+    Real *Wg, *wcr, *bb, *xpad;
+    double *work, *gxpart, *ptot, *gtot, *tmp;
+    auto carve = [&](char* base) {
+        Carve k{base};
+        a.Winv = k.take<double>(M * nn);
+        a.ldet = k.take<double>(M);
+        a.cq = k.take<double>((size_t)M * m * n);
+        a.wc = k.take<double>(ldb);
+        work = k.take<double>(8 + M * nn + inverse_work_doubles(n, M));
+        Wg = k.take<Real>((size_t)ldb * NP);
+        wcr = k.take<Real>(ldb);
+        bb = k.take<Real>((size_t)Tc * ldb);
+        xpad = n != NP ? k.take<Real>((size_t)Tc * NP) : nullptr;
+        if (split) {
+            a.qbuf = k.take<double>((size_t)Tc * pairs);
+            a.vbuf = k.take<double>((size_t)Tc * M);
+        }
+        if (adj) {
+            a.g = k.take<Real>((size_t)Tc * ldb);
+            a.part = k.take<double>((size_t)nb * a.pstride);
+            gxpart = k.take<double>((size_t)gchunks * gcount);
+            ptot = k.take<double>((size_t)C * pcount);
+            gtot = k.take<double>((size_t)C * gcount);
+            tmp = k.take<double>(sum_tmp_doubles(nb, pcount) + sum_tmp_doubles(gchunks, gcount));
+        }
+        return k.off;
+    };
+    char* base = (char*)ws.take(carve(nullptr));
+    if (!base) return report_error(AMICA_E_NOMEM, "workspace allocation failed");
+    carve(base);
+    const int prc = prepare_model<Real>(a, work, Wg, wcr, st);
+    if (prc) return prc;
+    for (int c = 0; c < C; ++c) {
+        const long t0 = (long)c * Tc, Tn = std::min(Tc, T - t0);
+        AdjArgs k = a;
+        const Real* xc = (const Real*)x + (size_t)t0 * n;
+        const Real* xp = xc;
+        k.x = xc;
+        k.T = Tn;
+        k.dll = adj ? dll + t0 : nullptr;
+        k.ll = ll ? ll + t0 : nullptr;
+        k.bbuf = bb;
+        if (n != NP) {
+            const unsigned pg = (unsigned)std::min<long>(65536, (Tn * NP + 255) / 256);
+            hipLaunchKernelGGL(adj_pad_kernel<Real>, dim3(pg), dim3(256), 0, st, xc, xpad, Tn, n, NP);
+            xp = xpad;
+        }
+        /* b = W x - W c by the unmixing GEMM on MFMA */
+        int urc;
+        if constexpr (rb == 8) urc = launch_unmix_f64(xp, Wg, wcr, bb, Tn, NP, ldb, cus, st);
+        else urc = launch_unmix_f32(xp, Wg, wcr, bb, Tn, NP, ldb, cus, st);
+        if (urc || hipGetLastError() != hipSuccess)
+            return report_error(AMICA_E_DEVICE, "unmixing GEMM launch failed");
+        const int nbn = (int)((Tn + a.chunk - 1) / a.chunk);
+        if (adj ? launch_ll<Real, true>(m, k, nbn, st) : launch_ll<Real, false>(m, k, nbn, st))
+            return report_error(AMICA_E_DEVICE, "likelihood kernel launch failed");
+        if (!adj) continue;
+        int gc = gchunks;
+        if constexpr (rb == 4) {
+            if (launch_gx_f32((const float*)a.g, xp, gxpart, Tn, NP, ldb, gchunks, st))
+                return report_error(AMICA_E_DEVICE, "statistic GEMM launch failed");
+        } else {
+            const long gch = ((Tn + gchunks - 1) / gchunks + 31) / 32 * 32;
+            gc = (int)((Tn + gch - 1) / gch);
+            hipLaunchKernelGGL(adj_gx_kernel, dim3(gc, ldb / 64, (n + 63) / 64), dim3(256), 0, st,
+                               (const double*)a.g, xc, Tn, n, ldb, gch, gxpart);
+        }
+        if (hipGetLastError() != hipSuccess ||
+            launch_sum_parts(a.part, nbn, a.pstride, pcount, ptot + (size_t)c * pcount, gxpart, gc, gcount,
+                             gtot + (size_t)c * gcount, tmp, st))
+            return report_error(AMICA_E_DEVICE, "adjoint launch failed");
+    }
+    if (adj) {
+        const int eb = (int)std::min<size_t>(1024, (nn + (size_t)n * m + 255) / 256);
+        hipLaunchKernelGGL(adj_finish_kernel, dim3(eb + (n + 3) / 4, M), dim3(256), 0, st, a, eb, ptot, pcount, gtot,
+                           gxs, C, *out);
+        if (hipGetLastError() != hipSuccess) return report_error(AMICA_E_DEVICE, "adjoint launch failed");
+    }
+    const hipError_t e = hipStreamSynchronize(st);
+    ws.drained();
+    if (e != hipSuccess) return report_error(AMICA_E_DEVICE, hipGetErrorString(e));
     return 0;
 }
 
@@ -659,146 +967,29 @@ int ll_call(int real_bits, const void* x, long T, int n, int M, int m, const dou
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return report_error(AMICA_E_DEVICE, "no HIP device");
 
-    const size_t rb = real_bits == 64 ? 8 : 4;
-    const int S = real_bits == 64 ? 4 : 8;
-    const int nw = M * NP / 64;
-    const long nblocks = std::max(1L, std::min((long)cus * 2, (T + S - 1) / S));
-    long chunk = (T + nblocks - 1) / nblocks;
-    chunk = (chunk + S - 1) / S * S;
-    const int nb = (int)((T + chunk - 1) / chunk);
-
     AdjArgs a = {};
-    a.x = x; a.T = T; a.n = n; a.NP = NP; a.M = M; a.m = m;
+    a.n = n; a.NP = NP; a.M = M; a.m = m;
     a.W = W; a.c = c; a.alpha = alpha; a.mu = mu; a.beta = beta; a.rho = rho; a.gm = gm;
-    a.ldetS = ldetS; a.dll = adj ? dll : nullptr; a.ll = ll; a.chunk = chunk;
+    a.ldetS = ldetS;
     a.pstride = ((size_t)M * NP * pair_stride(m) + M + 31) & ~(size_t)31;
-    Workspace ws;
-    const size_t nn = (size_t)n * n;
+    a.pg = 8;
     if (noalloc) {
         /* forward only, workspace carved from the static device array */
-        if ((size_t)M * nn > kNoAllocNN)
+        if ((size_t)M * n * n > kNoAllocNN)
             return report_error(AMICA_E_INVALID, "M * n * n exceeds the allocation-free workspace (65536)");
         double* sp = nullptr;
         const int rc = noalloc_scratch(&sp);
         if (rc) return rc;
         a.Winv = sp;
-        a.lu = sp + kNoAllocNN;
-        a.X = sp + 2 * kNoAllocNN;
-        a.cq = sp + 3 * kNoAllocNN;
+        double* work = sp + kNoAllocNN;
+        a.cq = work + kNoAllocWork;
         a.wc = a.cq + kNoAllocNM;
         a.ldet = a.wc + kNoAllocNP;
-    } else if (!ws.alloc((void**)&a.Winv, M * nn * 8) || !ws.alloc((void**)&a.ldet, M * 8) ||
-               !ws.alloc((void**)&a.cq, (size_t)M * m * n * 8) || !ws.alloc((void**)&a.wc, (size_t)M * NP * 8)) {
-        return report_error(AMICA_E_NOMEM, "workspace allocation failed");
+        return real_bits == 64 ? forward_noalloc<double>(a, x, T, ll, work, cus, st)
+                               : forward_noalloc<float>(a, x, T, ll, work, cus, st);
     }
-    if (!noalloc) {
-        /* W^-1 and log|det W| by the M-step's blocked Gauss-Jordan */
-        double* gjw = nullptr;
-        if (!ws.alloc((void**)&gjw, (8 + M * nn + inverse_work_doubles(n, M)) * 8))
-            return report_error(AMICA_E_NOMEM, "workspace allocation failed");
-        if (launch_gj_inverse(W, a.Winv, a.ldet, n, M, gjw, st))
-            return report_error(AMICA_E_DEVICE, "inverse launch failed");
-    }
-    if (split) {
-        a.pg = 8;
-        if (!ws.alloc((void**)&a.qbuf, (size_t)T * (M * NP / 64) * 8) ||
-            (adj && !ws.alloc((void**)&a.vbuf, (size_t)T * M * 8)))
-            return report_error(AMICA_E_NOMEM, "workspace allocation failed");
-    }
-    const int ldb = M * NP;
-    /* the statistic GEMM sum_t g_t x_t^T: FP32 MFMA over padded rows of x
-     * (gx_f32_slab_kernel, row stride NP) on the FP32 variant, FP64 tiles
-     * over the unpadded rows (row stride n) on the FP64 one */
-    const bool gx_mfma = adj && real_bits == 32;
-    const int gchunks = gx_mfma ? gx_f32_chunks(T, NP, ldb, cus)
-                                : (int)std::max(1L, std::min((long)cus, (T + 255) / 256));
-    const int gxs = gx_mfma ? NP : n;
-    double* gxpart = nullptr;
-    if (adj) {
-        if (!ws.alloc(&a.g, (size_t)T * ldb * rb) ||
-            !ws.alloc((void**)&a.part, (size_t)nb * a.pstride * 8) ||
-            !ws.alloc((void**)&gxpart, (size_t)gchunks * ldb * gxs * 8))
-            return report_error(AMICA_E_NOMEM, "workspace allocation failed");
-    }
-    hipLaunchKernelGGL(adj_prep_kernel, dim3(M), dim3(256), 0, st, a);
-    if (hipGetLastError() != hipSuccess) return report_error(AMICA_E_DEVICE, "prep launch failed");
-    /* b = W x - W c by the unmixing GEMM on MFMA (FP64 or FP32 operands)
-     * into a [T][M NP] buffer; the allocation-free forward forms b per lane */
-    const void* xp = x;
-    if (!noalloc) {
-        void *Wg = nullptr, *wcr = nullptr, *bb = nullptr;
-        if (!ws.alloc(&Wg, (size_t)ldb * NP * rb) || !ws.alloc(&wcr, (size_t)ldb * rb) ||
-            !ws.alloc(&bb, (size_t)T * ldb * rb))
-            return report_error(AMICA_E_NOMEM, "workspace allocation failed");
-        const unsigned eg = (unsigned)std::min<long>(4096, ((long)ldb * NP + 255) / 256);
-        if (n != NP) {
-            void* xpad = nullptr;
-            if (!ws.alloc(&xpad, (size_t)T * NP * rb))
-                return report_error(AMICA_E_NOMEM, "workspace allocation failed");
-            const unsigned pg = (unsigned)std::min<long>(65536, (T * NP + 255) / 256);
-            if (real_bits == 64)
-                hipLaunchKernelGGL(adj_pad_kernel<double>, dim3(pg), dim3(256), 0, st, (const double*)x,
-                                   (double*)xpad, T, n, NP);
-            else
-                hipLaunchKernelGGL(adj_pad_kernel<float>, dim3(pg), dim3(256), 0, st, (const float*)x,
-                                   (float*)xpad, T, n, NP);
-            xp = xpad;
-        }
-        int urc;
-        if (real_bits == 64) {
-            hipLaunchKernelGGL(adj_wg_kernel<double>, dim3(eg), dim3(256), 0, st, a, (double*)Wg, (double*)wcr);
-            urc = launch_unmix_f64((const double*)xp, (const double*)Wg, (const double*)wcr, (double*)bb, T,
-                                   NP, ldb, cus, st);
-        } else {
-            hipLaunchKernelGGL(adj_wg_kernel<float>, dim3(eg), dim3(256), 0, st, a, (float*)Wg, (float*)wcr);
-            urc = launch_unmix_f32((const float*)xp, (const float*)Wg, (const float*)wcr, (float*)bb, T, NP,
-                                   ldb, cus, st);
-        }
-        if (urc || hipGetLastError() != hipSuccess)
-            return report_error(AMICA_E_DEVICE, "unmixing GEMM launch failed");
-        a.bbuf = bb;
-    }
-    const size_t shm = (size_t)S * NP * rb + (size_t)S * nw * 8 + 2 * (size_t)S * M * 8;
-    int rc;
-    if (real_bits == 64)
-        rc = adj ? launch_ll<double, true>(m, a, nb, shm, st) : launch_ll<double, false>(m, a, nb, shm, st);
-    else
-        rc = adj ? launch_ll<float, true>(m, a, nb, shm, st) : launch_ll<float, false>(m, a, nb, shm, st);
-    if (rc) return report_error(AMICA_E_DEVICE, "likelihood kernel launch failed");
-    if (adj) {
-        int gc = gchunks;
-        if (gx_mfma) {
-            if (launch_gx_f32((const float*)a.g, (const float*)xp, gxpart, T, NP, ldb, gchunks, st))
-                return report_error(AMICA_E_DEVICE, "statistic GEMM launch failed");
-        } else {
-            long gch = (T + gchunks - 1) / gchunks;
-            gch = (gch + 31) / 32 * 32;
-            gc = (int)((T + gch - 1) / gch);
-            const dim3 grid(gc, (ldb + 63) / 64, (n + 63) / 64);
-            hipLaunchKernelGGL(adj_gx_kernel<double>, grid, dim3(256), 0, st, (const double*)a.g,
-                               (const double*)x, T, n, ldb, gch, gxpart);
-        }
-        /* the partial slots summed across the GPU, then one workgroup per
-         * model assembles the gradients from the totals */
-        double *ptot = nullptr, *gtot = nullptr;
-        const size_t pcount = (size_t)ldb * pair_stride(m) + M, gcount = (size_t)ldb * gxs;
-        if (!ws.alloc((void**)&ptot, pcount * 8) || !ws.alloc((void**)&gtot, gcount * 8))
-            return report_error(AMICA_E_NOMEM, "workspace allocation failed");
-        hipLaunchKernelGGL(adj_slot_sum_kernel, dim3((unsigned)std::min<size_t>(4096, (pcount + 255) / 256)),
-                           dim3(256), 0, st, a.part, a.pstride, nb, pcount, ptot);
-        hipLaunchKernelGGL(adj_slot_sum_kernel, dim3((unsigned)std::min<size_t>(4096, (gcount + 255) / 256)),
-                           dim3(256), 0, st, gxpart, gcount, gc, gcount, gtot);
-        AdjArgs at = a;
-        at.part = ptot;
-        at.pstride = pcount;
-        hipLaunchKernelGGL(adj_finish_kernel, dim3(M), dim3(256), (size_t)n * 8, st, at, 1, gtot, 1, gxs,
-                           *out);
-        if (hipGetLastError() != hipSuccess) return report_error(AMICA_E_DEVICE, "adjoint launch failed");
-    }
-    if (noalloc) return 0;     /* asynchronous: the caller synchronises `stream` */
-    const hipError_t e = hipStreamSynchronize(st);
-    if (e != hipSuccess) return report_error(AMICA_E_DEVICE, hipGetErrorString(e));
-    return 0;
+    return real_bits == 64 ? run_chunks<double>(a, x, T, dll, ll, out, split, dev, cus, st)
+                           : run_chunks<float>(a, x, T, dll, ll, out, split, dev, cus, st);
 }
 
 }  // namespace

@@ -1143,18 +1143,29 @@ static SumSeg second_pass(const SumSeg& f, double* out) {
     return SumSeg{f.out, out, f.len, f.len, f.G, f.G, f.xb, 1};
 }
 
+size_t sum_tmp_doubles(int nparts, size_t len) {
+    const int G = sum_groups(nparts, len);
+    return G > 1 ? (size_t)G * len : 0;
+}
+
+int launch_sum_parts(const double* pa, int na, size_t stride_a, size_t len_a, double* out_a, const double* pb,
+                     int nb, size_t len_b, double* out_b, double* tmp, hipStream_t st) {
+    const SumSeg p = first_pass(pa, na, stride_a, len_a, tmp, out_a);
+    const SumSeg g = first_pass(pb, nb, len_b, len_b, tmp + sum_tmp_doubles(na, len_a), out_b);
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(p.xb * p.G + g.xb * g.G)), dim3(64 * kSumWaves), 0, st, p, g);
+    const SumSeg p2 = second_pass(p, out_a), g2 = second_pass(g, out_b);
+    if (p2.xb + g2.xb > 0)
+        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(p2.xb + g2.xb)), dim3(64 * kSumWaves), 0, st, p2, g2);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 int launch_reduce(const double* part, int nparts, size_t pstride, const double* gxpart,
                   int nchunks, double* raw, double* gxtot, double* tmp, const MstepArgs& ma, bool mstep,
                   hipStream_t st) {
     const int NS = kStatsPerJ * ma.m + kStatsPerI;
     const size_t plen = (size_t)ma.M * NS * ma.NP + ma.M + 1;
     const size_t glen = (size_t)ma.ldb * ma.NP;
-    const SumSeg p = first_pass(part, nparts, pstride, plen, tmp, raw);
-    const SumSeg g = first_pass(gxpart, nchunks, glen, glen, tmp + kSumGroups * pstride, gxtot);
-    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(p.xb * p.G + g.xb * g.G)), dim3(64 * kSumWaves), 0, st, p, g);
-    const SumSeg p2 = second_pass(p, raw), g2 = second_pass(g, gxtot);
-    if (p2.xb + g2.xb > 0)
-        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(p2.xb + g2.xb)), dim3(64 * kSumWaves), 0, st, p2, g2);
+    if (launch_sum_parts(part, nparts, pstride, plen, raw, gxpart, nchunks, glen, gxtot, tmp, st)) return -1;
     /* one 16 x 16 tile of phi per workgroup, after the statistics' */
     const unsigned ntk = (unsigned)((ma.n + 15) / 16);
     const dim3 grid(ma.M, 1 + ntk * ntk);
