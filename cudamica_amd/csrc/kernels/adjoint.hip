@@ -60,7 +60,7 @@ struct AdjArgs {
     double* wc;          /* [M][NP] W_h c_h */
     void* g;             /* [T][M NP] (adjoint) */
     double* part;        /* [nblocks][pstride] */
-    long chunk;          /* samples per workgroup, a multiple of 16 */
+    long chunk;          /* samples per workgroup, a multiple of 4 */
     size_t pstride;
     /* split passes (M ceil(n/64) > 8 waves): workgroups of pg (model,
      * channel-block) pairs, blockIdx.y = pair group; qbuf [T][M CW] the
@@ -807,12 +807,13 @@ int prepare_model(const AdjArgs& a, double* work, Real* Wg, Real* wcr, hipStream
 }
 
 /* Workgroups of the likelihood kernel over T samples and the samples of each
- * (whole 16-sample groups): 16 waves per CU, which its registers allow on
- * the forward passes; where the adjoint's allow half, the rest queue. */
+ * (whole tiles of 4): 16 waves per CU, which its registers allow on the
+ * forward passes; where the adjoint's allow half, the rest queue.  A short
+ * call runs one tile per wave (a tile is a chain of ~5 us in FP64). */
 int ll_grid(long T, int pairs, int cus, long* chunk) {
     const long waves = pairs <= 8 ? pairs : 8L * ((pairs + 7) / 8);
-    const long nb = std::max(1L, std::min(16L * cus / waves, (T + 15) / 16));
-    *chunk = ((T + nb - 1) / nb + 15) / 16 * 16;
+    const long nb = std::max(1L, std::min(16L * cus / waves, (T + 3) / 4));
+    *chunk = ((T + nb - 1) / nb + 3) / 4 * 4;
     return (int)((T + *chunk - 1) / *chunk);
 }
 
@@ -853,7 +854,8 @@ int run_chunks(AdjArgs a, const void* x, long T, const double* dll, double* ll, 
      * the unpadded rows (row stride n) on the FP64 one */
     const bool gx32 = rb == 4;
     const int slabs = (ldb / 64) * ((n + 63) / 64);
-    const int gchunks = gx32 ? gx_f32_chunks(Tc, NP, ldb, cus)
+    const GxChunks gc32 = gx32 ? gx_f32_chunks(Tc, NP, ldb, cus) : GxChunks{0, 0, 1};
+    const int gchunks = gx32 ? gc32.n
                              : (int)std::max(1L, std::min(std::max(1L, 2L * cus / slabs), (Tc + 255) / 256));
     const int gxs = gx32 ? NP : n;
     const size_t pcount = (size_t)ldb * pair_stride(m) + M, gcount = (size_t)ldb * gxs;
@@ -917,7 +919,8 @@ int run_chunks(AdjArgs a, const void* x, long T, const double* dll, double* ll, 
         if (!adj) continue;
         int gc = gchunks;
         if constexpr (rb == 4) {
-            if (launch_gx_f32((const float*)a.g, xp, gxpart, Tn, NP, ldb, gchunks, st))
+            gc = (int)((Tn + gc32.chunk - 1) / gc32.chunk) * gc32.spread;
+            if (launch_gx_f32((const float*)a.g, xp, gxpart, Tn, NP, ldb, GxChunks{gc, gc32.chunk, gc32.spread}, st))
                 return report_error(AMICA_E_DEVICE, "statistic GEMM launch failed");
         } else {
             const long gch = ((Tn + gchunks - 1) / gchunks + 31) / 32 * 32;

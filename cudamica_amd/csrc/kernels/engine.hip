@@ -111,6 +111,7 @@ struct amica_engine {
     size_t pstride = 0;
     double* part = nullptr;
     int nchunks = 0;
+    GxChunks gx = {0, 0, 1};          /* FP32 statistic GEMM */
     double* gxpart = nullptr;
     double* raw = nullptr;
     double* sumtmp = nullptr;      /* first-pass group sums of the partials */
@@ -167,7 +168,8 @@ struct amica_engine {
         chunk = (T + nblocks - 1) / nblocks;
         chunk = ((chunk + 31) / 32) * 32;     /* whole packed 8-sample groups */
         nblocks = (int)((T + chunk - 1) / chunk);
-        nchunks = bf16 ? gx_bf16_chunks(T, NP, ldb, cu_budget) : gx_f32_chunks(T, NP, ldb, cu_budget);
+        if (!bf16) gx = gx_f32_chunks(T, NP, ldb, cu_budget);
+        nchunks = bf16 ? gx_bf16_chunks(T, NP, ldb, cu_budget) : gx.n;
         if (gexec) {   /* the captured grids are stale */
             (void)hipGraphExecDestroy(gexec);
             (void)hipGraphDestroy(graph);
@@ -265,7 +267,7 @@ struct amica_engine {
             if (bf16)
                 LCHK(launch_gx_bf16((const uint16_t*)g, x8, gxpart, o.T, NP, ldb, nchunks, st));
             else
-                LCHK(launch_gx_f32((const float*)g, xw, gxpart, o.T, NP, ldb, nchunks, st));
+                LCHK(launch_gx_f32((const float*)g, xw, gxpart, o.T, NP, ldb, gx, st));
         }
         if (with_timing) HIPCHK(hipEventRecord(ev[4], st));
         StageRange r("amica: reductions");

@@ -144,16 +144,21 @@ int launch_gx_bf16_batch(const GxArgs* args, const BatchItem* items, int nitems,
 int launch_unmix_fp8(const uint8_t* xq, const uint16_t* Whi, const uint16_t* Wlo, const float* wc,
                      float* b, long T, int NP, int ldb, int cus, hipStream_t st);
 /* part[chunk][c][k] = sum_{t in chunk} g[t][c] x[t][k]   (FP64 partials) */
-int launch_gx_f32(const float* g, const float* x, double* part, long T, int NP, int ldb,
-                  int nchunks, hipStream_t st);
+struct GxChunks {
+    int n;          /* partials */
+    long chunk;     /* samples of `spread` consecutive ones */
+    int spread;
+};
+int launch_gx_f32(const float* g, const float* x, double* part, long T, int NP, int ldb, const GxChunks& c,
+                  hipStream_t st);
 /* BF16 path: g and x packed 8 samples per column ([T32/8][cols][8], T32 =
  * T rounded up to 32, zero padded); part is [nchunks][ldb][NP]. */
 int launch_gx_bf16(const uint16_t* g8, const uint16_t* x8, double* part, long T, int NP, int ldb,
                    int nchunks, hipStream_t st);
-/* Number of sample chunks (partials) launch_gx_bf16 / launch_gx_f32 should
- * be given for a budget of `cus` CUs (nondecreasing in cus). */
+/* Sample chunks (partials) launch_gx_bf16 / launch_gx_f32 should be given for
+ * a budget of `cus` CUs (their number is nondecreasing in cus). */
 int gx_bf16_chunks(long T, int NP, int ldb, int cus);
-int gx_f32_chunks(long T, int NP, int ldb, int cus);
+GxChunks gx_f32_chunks(long T, int NP, int ldb, int cus);
 /* x8[(t/8) NP + i][t%8] = xhi[t][i] (the packed B operand of the BF16
  * statistic GEMM); padding stays as allocated (zero). */
 int launch_pack8(const uint16_t* xhi, long T, int NP, uint16_t* x8, hipStream_t st);

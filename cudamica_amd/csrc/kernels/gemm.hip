@@ -682,30 +682,32 @@ __global__ __launch_bounds__(256) void unmix_f32_kernel(const float* __restrict_
  * waves), a workgroup of 8 waves runs S = 8 / rw sub-ranges of its chunk
  * side by side and adds their totals in FP64 through LDS in a fixed order, a
  * quarter of the tile at a time so that every width fits the LDS, before the
- * one partial is written (128 ch x 500k x 2 models: 438 -> 403 us and, with
- * half the partials, reductions 123 -> 91 us). */
-template <int CT>
+ * one partial is written (128 ch x 500k x 2 models: 440 -> 406 us and, with
+ * half the partials, reductions 122 -> 91 us). */
+template <int CT, int D>
 __global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restrict__ g,
                                                           const float* __restrict__ x,
                                                           double* __restrict__ part, long T,
-                                                          int NP, int ldb, long chunk) {
-    constexpr int D = 2;                            /* 4-sample steps in flight */
+                                                          int NP, int ldb, long chunk, int spread) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int rw = min(ldb - (int)blockIdx.z * 512, 512) / 64;   /* row waves */
     /* sample sub-ranges: only below 512 columns, where the launch gives 8
-     * waves for fewer row waves and the LDS tile with them */
-    const int S = ldb < 512 ? max(1, (int)(blockDim.x >> 6) / rw) : 1;
-    const int sr = w / rw, wr = w - sr * rw;
+     * waves for fewer row waves and the LDS tile with them.  spread > 1: the
+     * workgroups spread c .. spread c + spread - 1 take the sub-ranges of
+     * chunk c, each with a partial of its own */
+    const int S = spread > 1 || ldb >= 512 ? 1 : max(1, (int)(blockDim.x >> 6) / rw);
+    const int sr = spread > 1 ? (int)(blockIdx.x % spread) : w / rw, wr = spread > 1 ? w : w - sr * rw;
     const int r0 = blockIdx.z * 512 + wr * 64;     /* grid.z: groups of 512 g columns */
     /* the last group of 512 columns may have fewer rows than the workgroup has
      * waves: the others would write zeros over its partial (no barriers below
      * when S = 1) */
     if (S == 1 && w >= rw) return;
     const int k0 = blockIdx.y * 16 * CT;
-    long ts = (long)blockIdx.x * chunk;
+    long ts = (long)(blockIdx.x / spread) * chunk;
     long te = min(T, ts + chunk);
     {
-        const long sub = ((chunk + S - 1) / S + 3) / 4 * 4;      /* whole 4-sample steps */
+        const int parts = max(S, spread);
+        const long sub = ((chunk + parts - 1) / parts + 3) / 4 * 4;      /* whole 4-sample steps */
         ts = min(te, ts + sr * sub);
         te = min(te, ts + sub);
     }
@@ -723,10 +725,11 @@ __global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restric
         const long t = t4 + (lane >> 4);
         const bool ok = t < te;
         A[d] = ok ? *(const f32x4*)(g + (size_t)t * ldb + r0 + 4 * (lane & 15)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+        const float* xr = x + (size_t)t * NP + k0 + CT * (lane & 15);
+        if constexpr (CT == 1) B[d][0] = ok ? *xr : 0.f;
 #pragma unroll
-        for (int c4 = 0; c4 < CT; c4 += 4) {
-            const f32x4 v = ok ? *(const f32x4*)(x + (size_t)t * NP + k0 + CT * (lane & 15) + c4)
-                               : (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int c4 = 0; c4 + 4 <= CT; c4 += 4) {
+            const f32x4 v = ok ? *(const f32x4*)(xr + c4) : (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int e = 0; e < 4; ++e) B[d][c4 + e] = v[e];
         }
@@ -759,12 +762,14 @@ __global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restric
             for (int r = 0; r < 4; ++r) {
                 const int row = r0 + 16 * (lane >> 4) + 4 * r + rt;
                 double* o = out + (size_t)row * NP + k0 + CT * (lane & 15);
+                if constexpr (CT == 1) *o = (double)acc[rt][0][r];
 #pragma unroll
-                for (int ct = 0; ct < CT; ct += 2)
+                for (int ct = 0; ct + 2 <= CT; ct += 2)
                     *(double2*)(o + ct) = make_double2((double)acc[rt][ct][r], (double)acc[rt][ct + 1][r]);
             }
         return;
     }
+    if constexpr (CT > 1) {
     /* a quarter of the tile (one rt) at a time: sub-ranges S-1 .. 0 add their
      * totals in FP64 into the LDS of their row wave (register layout:
      * lane-consecutive doubles), in that order; sub-range 0 then writes the
@@ -802,6 +807,7 @@ __global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restric
             }
         }
         __syncthreads();                            /* read before the next quarter */
+    }
     }
 }
 
@@ -1147,7 +1153,7 @@ static long gx_chunk(long T, int nchunks, int mult) {
 
 static int gx_f32_ct(int NP) { return NP % 128 == 0 ? 8 : 4; }
 
-/* workgroups of 8 waves that split their chunk's samples (g narrower than
+/* workgroups of 8 waves that share the samples of a chunk (g narrower than
  * 512 columns): a quarter of the FP64 tile in LDS */
 static size_t gx_f32_split_lds(int NP, int ldb) {
     return (size_t)(ldb / 64) * 4 * gx_f32_ct(NP) * 64 * sizeof(double);
@@ -1155,37 +1161,52 @@ static size_t gx_f32_split_lds(int NP, int ldb) {
 
 static bool gx_f32_split(int ldb) { return ldb < 512 && 8 % (ldb / 64) == 0; }
 
-int gx_f32_chunks(long T, int NP, int ldb, int cus) {
-    /* per wave (S of them split a chunk where g has fewer than 512 columns)
-     * 512 samples, 256 below 256 columns of 64 inputs, fewer -- down to 32 --
-     * where the launch would otherwise have less than one workgroup of 8 waves
-     * per CU; at most 256 MB of partials, which are written and read back
-     * once.  A wave's samples are a serial chain of loads and MFMAs: 16 ch x
-     * 20k samples took 62 us with 10 workgroups of 256 samples per wave, 21 us
-     * with 79; two workgroups per CU measured slower (71 ch x 200k, M = 2: 188
-     * instead of 165 us, the partials written twice as often) */
+GxChunks gx_f32_chunks(long T, int NP, int ldb, int cus) {
+    /* The FP32 accumulation ranges, one per wave: for 128 columns of 64 inputs
+     * and fewer, chunks of >= 2048 (one model) or 1024 samples whose S waves
+     * take a share each, else chunks of >= 512 samples; at most 256 MB of
+     * partials, and at least one chunk per CU of the budget where T allows. */
+    const bool shared = NP == 64 && ldb <= 128;
     const int S = gx_f32_split(ldb) ? 8 / (ldb / 64) : 1;
-    const long len = (NP == 64 && ldb <= 128 ? 256L : 512L) * S;
-    const int slabs = NP / (16 * gx_f32_ct(NP)) * ((ldb + 511) / 512);
-    const long want = std::max(1L, (long)cus / slabs);
-    const long by_len = std::max((T + len - 1) / len, std::min(want, (T + 32L * S - 1) / (32L * S)));
+    const long per = shared ? 256L * S : 512L;
+    const long by_len = (T + per - 1) / per;
     const long by_mem = std::max(1L, (256L << 20) / ((long)ldb * NP * 8));
-    return (int)std::max(1L, std::min(by_len, std::max(want, by_mem)));
+    const long want = std::max(1L, (long)cus / (NP / (16 * gx_f32_ct(NP))));
+    const long n = std::max(1L, std::min(by_len, std::max(want, by_mem)));
+    GxChunks c;
+    c.chunk = gx_chunk(T, (int)n, 4);
+    /* other widths below 512 columns: S such ranges in one workgroup, whose
+     * totals meet in LDS: S times fewer partials */
+    if (!shared && S > 1) c.chunk *= S;
+    c.n = (int)((T + c.chunk - 1) / c.chunk);
+    /* Where that leaves most of the GPU idle, a chunk's ranges go to
+     * workgroups of their own, 16 columns of x to each (the sums inside a range
+     * are the same): 16 ch x 20k samples ran 10 workgroups of 8 waves, 62 us;
+     * 316 of one wave take 16 us. */
+    c.spread = S > 1 && c.n < 64 ? S : 1;
+    c.n *= c.spread;
+    return c;
 }
 
-int launch_gx_f32(const float* g, const float* x, double* part, long T, int NP, int ldb,
-                  int nchunks, hipStream_t st) {
-    if (NP % 64 || ldb % 64 || nchunks < 1) return -1;
+int launch_gx_f32(const float* g, const float* x, double* part, long T, int NP, int ldb, const GxChunks& c,
+                  hipStream_t st) {
+    if (NP % 64 || ldb % 64 || c.n < 1 || c.spread < 1 || (long)(c.n / c.spread) * c.chunk < T) return -1;
+    if (c.spread > 1) {
+        hipLaunchKernelGGL((gx_f32_slab_kernel<1, 8>), dim3(c.n, NP / 16), dim3(ldb), 0, st, g, x, part, T, NP, ldb,
+                           c.chunk, c.spread);
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
     const int CT = gx_f32_ct(NP);
-    dim3 grid(nchunks, NP / (16 * CT), (ldb + 511) / 512), block(std::min(ldb, 512));
-    const long chunk = gx_chunk(T, nchunks, 4);
+    dim3 grid(c.n, NP / (16 * CT), (ldb + 511) / 512), block(std::min(ldb, 512));
     const bool split = gx_f32_split(ldb);
     if (split) block = dim3(512);
     const size_t shm = split ? gx_f32_split_lds(NP, ldb) : 0;
     if (CT == 8)
-        hipLaunchKernelGGL(gx_f32_slab_kernel<8>, grid, block, shm, st, g, x, part, T, NP, ldb, chunk);
+        hipLaunchKernelGGL((gx_f32_slab_kernel<8, 2>), grid, block, shm, st, g, x, part, T, NP, ldb, c.chunk, 1);
+    else if (c.n < 256)   /* less than a workgroup per CU: more of a wave's loads in flight */
+        hipLaunchKernelGGL((gx_f32_slab_kernel<4, 4>), grid, block, shm, st, g, x, part, T, NP, ldb, c.chunk, 1);
     else
-        hipLaunchKernelGGL(gx_f32_slab_kernel<4>, grid, block, shm, st, g, x, part, T, NP, ldb, chunk);
+        hipLaunchKernelGGL((gx_f32_slab_kernel<4, 2>), grid, block, shm, st, g, x, part, T, NP, ldb, c.chunk, 1);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
