@@ -39,13 +39,23 @@
  * workgroup's own slot of the partial buffer, which the reduction kernel
  * sums over workgroups in a fixed order (no atomics, run-to-run identical).
  *
- * Latency: the b and x loads of tile k+1 are issued before tile k's math
- * (raw buffer loads, scalar row offsets), the per-sample channel sums use
- * DPP row shifts instead of LDS permutes, two barriers per tile of 2
- * samples (1 for m >= 4) publish the per-row channel sums and then the
- * model posteriors, which one wave evaluates for the workgroup, and the
- * per-lane LDS footprint (FP32 level-2 totals) leaves room for two
- * 512-thread workgroups per CU.
+ * Bound: the vector ALU.  The arithmetic alone takes about 310 cycles per
+ * sample and wave at m = 3 (three transcendentals at 8.3 and some fifteen
+ * FP32 operations at 2.8-3.4 cycles each, per component), the kernel about
+ * 450: the rest is loads, the row sums, the exchange between the waves (about
+ * 40) and the flushes.  So the fixed work is shared out: tiles of four samples
+ * (two for m = 4, one above) pass the two barriers that publish the channel
+ * sums and then the model posteriors, which one wave evaluates for the
+ * workgroup, a row of 16 lanes to a sample; one underflow test serves a tile;
+ * b loads are issued a tile ahead, x loads before the tile's densities.  What
+ * that costs in registers comes back by keeping only what an FMA or two cannot
+ * form again.  The per-lane LDS footprint (FP32 level-2 totals) leaves room
+ * for two 512-thread workgroups per CU.  Against tiles of two samples (one for
+ * m = 4) with every intermediate kept, in us: 128 ch x 1M x 4 models m = 3
+ * 1526 -> 1463, 256 ch x 500k x 2 models m = 4 1036 -> 961, 128 ch x 500k x 2
+ * models with FP64 b 469 -> 440, the split launch's passes (300 ch x 60k x 3
+ * models) 515 -> 350.  One barrier with the posteriors formed in every wave
+ * (1628) or a tile later (1754) is slower than either.
  *
  * B64 = true (FP32 path): b is FP64 and y = sqrt(beta)(b - mu) is formed in
  * FP64 before the FP32 density math, so |y| near 0 -- where mu_denom's
@@ -136,7 +146,12 @@ __device__ __forceinline__ void l3_accumulate(double* l3, bool started, bool kee
     }
 }
 
-/* MODE selects the launch the kernel serves:
+/* Samples per tile: as many as keep the kernel at two workgroups of 8 waves
+ * per CU (128 VGPRs); with FP64 b at m = 3, where y is kept, four samples leave
+ * one, which is faster still (128 ch x 500k x 2 models: 440 us, 522 with two). */
+constexpr int estep_tile_samples(int MJ, bool B64) { return MJ <= 3 ? 4 : MJ == 4 && !B64 ? 2 : 1; }
+
+/* MODE selects the launch the kernel serves (GB: g as packed bf16):
  *   kEstepFused  all M models x CW channel blocks in one workgroup (M CW <= 8):
  *                the cross-channel and cross-model sums stay on chip;
  *   kEstepLsum   split launch, first pass: a workgroup holds a group of models
@@ -145,11 +160,11 @@ __device__ __forceinline__ void l3_accumulate(double* l3, bool started, bool kee
  *   kEstepStats  split launch, last pass: the densities again, the model
  *                posteriors read from vq (written between the passes by
  *                estep_post_kernel), then the statistics and g. */
-template <int MJ, bool B64, int MODE>
+template <int MJ, bool B64, int MODE, bool GB>
 __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
-    /* samples per barrier tile: 2, or 1 where m >= 4 so that the per-sample
-     * values stay within 128 VGPRs (two workgroups per CU) */
-    constexpr int kS = MJ >= 4 ? 1 : 2;
+    constexpr int kS = estep_tile_samples(MJ, B64);
+    /* y is not kept between the phases but formed again, where that is one FMA */
+    constexpr bool kRecY = !B64;
     constexpr int kFlush = 32 / kS;     /* tiles summed in FP32 registers (32 samples) */
     /* FP64 flushes with batched loads, except in the split launch's
      * statistics pass, which they would push past 128 VGPRs on the FP32
@@ -182,9 +197,9 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
 
     /* per-row channel sums of one tile, double buffered:
      * [buf][wave][sample][row of 16 lanes] (a sample's 4 rows in 16 bytes),
-     * and the tile's model posteriors [buf][model h * kS + sample] */
+     * and the tile's model posteriors [buf][model][sample] */
     __shared__ __align__(16) float Lp[2][kMaxEstepWaves][kS][4];
-    __shared__ __align__(8) float Vp[2][AMICA_MAX_M * 2];
+    __shared__ __align__(16) float Vp[2][kMaxEstepWaves][kS];
     __shared__ float dc2[AMICA_MAX_M];
     /* per-lane FP32 level-2 totals, [blockDim.x][NSP] (odd stride: the
      * lanes of a wave hit distinct banks) */
@@ -261,7 +276,7 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
      * (the padding rows of W and entries of W c are zero, and x's padding
      * columns are written as zero), so every load is unconditional and the
      * wait for a prefetch can sit where its value is first used. */
-    float bn[kS], xn[kS];
+    float bn[kS];
     double bn64[B64 ? kS : 1];
     /* b and x through buffer resources based at row t0: the lane's byte
      * offset is fixed, the row's a scalar (launch_estep bounds it below
@@ -289,7 +304,6 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
             bn64[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rb, vob, r * browb, 0));
         else
             bn[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, vob, r * browb, 0));
-        xn[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, vox, r * xrowb, 0));
     };
 #pragma unroll
     for (int s = 0; s < kS; ++s) load_tile(t0 + s, s);
@@ -309,26 +323,34 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
 #pragma unroll
         for (int sub = 0; sub < kTPG; ++sub) {
             const long tb = tg + sub * kS;
-            float E[kS][MJ], SY[kS][MJ], YM2[kS][MJ], YR[kS][MJ], LA[kS][MJ];
-            float RS[kS], BV[kS], XV[kS];
+            /* kept per component and sample: |y|^(rho-2), log2|y|, 2^Q and, where
+             * it is formed in FP64, y (sy and |y|^rho are one product each away) */
+            float E[kS][MJ], Y[kS][MJ], YM2[kS][MJ], LA[kS][MJ];
+            float RS[kS], BV[kS], XV[kS], SE[kS];
             double BV64[B64 ? kS : 1];
 #pragma unroll
             for (int s = 0; s < kS; ++s) {
                 if constexpr (B64) { BV64[s] = bn64[s]; BV[s] = (float)bn64[s]; }
                 else BV[s] = bn[s];
-                XV[s] = xn[s];
             }
-            /* issue the next tile's b and x loads now; they complete under this
-             * tile's math.  Rows past t1 are read without a check (the next
-             * range's samples, or the kEstepRowPad zero rows after the last
-             * one) and get posterior 0. */
+            /* issue the next tile's b loads and this one's x loads (first
+             * used after the exchange) now; they complete under this tile's
+             * math.  Rows past t1 are read without a check (the next range's
+             * samples, or the kEstepRowPad zero rows after the last one) and
+             * get posterior 0. */
+            if constexpr (MODE != kEstepLsum) {
+#pragma unroll
+                for (int s = 0; s < kS; ++s)
+                    XV[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                          rx, vox, (int)(tb - tbase + s) * xrowb, 0));
+            }
 #pragma unroll
             for (int s = 0; s < kS; ++s) load_tile(tb + kS + s, s);
             /* ---- phase 1: densities, component posteriors, channel sums ---- */
             float QS[kS];
 #pragma unroll
             for (int s = 0; s < kS; ++s) {
-                float q2[MJ];
+                SE[s] = 0.f;
 #pragma unroll
                 for (int j = 0; j < MJ; ++j) {
                     float y;
@@ -339,35 +361,48 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                     else y = fmaf(sb[j], BV[s], nsbmu[j]);
                     const float la = fast_log2(fmaxf(fabsf(y), y_floor<B64>()));
                     const float ym2 = fast_exp2(rm2[j] * la);
-                    const float sy = ym2 * y;
-                    const float yr = sy * y;
-                    q2[j] = fmaf(yr, -AMICA_L2E, cq2[j]);
-                    SY[s][j] = sy; YM2[s][j] = ym2; YR[s][j] = yr; LA[s][j] = la;
+                    const float yr = (ym2 * y) * y;
+                    E[s][j] = fast_exp2(fmaf(yr, -AMICA_L2E, cq2[j]));
+                    SE[s] = j == 0 ? E[s][j] : SE[s] + E[s][j];
+                    Y[s][j] = y; YM2[s][j] = ym2; LA[s][j] = la;
                 }
-                /* q2 <= log2(alpha sqrt(beta) / (2 Gamma(1 + 1/rho))), a few
-                 * units, so 2^q2 needs no max shift unless every component
-                 * underflows (a sample far from all of them): then, for the
-                 * whole wave, shift by the per-lane max */
-#pragma unroll
-                for (int j = 0; j < MJ; ++j) E[s][j] = fast_exp2(q2[j]);
-                float se = E[s][0];
-#pragma unroll
-                for (int j = 1; j < MJ; ++j) se += E[s][j];
-                const bool under = __any(se < 0x1p-100f);
-                QS[s] = fast_log2(se);            /* exactly 0 on padding channels */
-                if (__builtin_expect(under, 0)) {
-                    float off = q2[0];
-#pragma unroll
-                    for (int j = 1; j < MJ; ++j) off = fmaxf(off, q2[j]);
-#pragma unroll
-                    for (int j = 0; j < MJ; ++j) E[s][j] = fast_exp2(q2[j] - off);
-                    se = E[s][0];
-#pragma unroll
-                    for (int j = 1; j < MJ; ++j) se += E[s][j];
-                    QS[s] = off + fast_log2(se);
-                }
-                RS[s] = fast_rcp(se);
+                QS[s] = fast_log2(SE[s]);         /* exactly 0 on padding channels */
             }
+            /* q2 <= log2(alpha sqrt(beta) / (2 Gamma(1 + 1/rho))), a few units,
+             * so 2^q2 needs no max shift unless every component underflows (a
+             * sample far from all of them): then, for the whole wave, that
+             * sample's are shifted by the per-lane max.  One test per tile: the
+             * samples' densities stay one block of independent chains.  (The
+             * empty asm, here and before phase 2, keeps the compiler from
+             * holding on to the y it could form again.) */
+            if constexpr (kRecY)
+#pragma unroll
+                for (int s = 0; s < kS; ++s) __asm__ volatile("" : "+v"(BV[s]));
+            float smin = SE[0];
+#pragma unroll
+            for (int s = 1; s < kS; ++s) smin = fminf(smin, SE[s]);
+            if (__builtin_expect(__any(smin < 0x1p-100f), 0)) {
+#pragma unroll
+                for (int s = 0; s < kS; ++s) {
+                    if (!__any(SE[s] < 0x1p-100f)) continue;
+                    float q2[MJ], off = 0.f;
+#pragma unroll
+                    for (int j = 0; j < MJ; ++j) {
+                        const float yv = kRecY ? fmaf(sb[j], BV[s], nsbmu[j]) : Y[s][j];
+                        const float yr = (YM2[s][j] * yv) * yv;
+                        q2[j] = fmaf(yr, -AMICA_L2E, cq2[j]);
+                        off = j == 0 ? q2[0] : fmaxf(off, q2[j]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < MJ; ++j) {
+                        E[s][j] = fast_exp2(q2[j] - off);
+                        SE[s] = j == 0 ? E[s][j] : SE[s] + E[s][j];
+                    }
+                    QS[s] = off + fast_log2(SE[s]);
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < kS; ++s) RS[s] = fast_rcp(SE[s]);
             const int nval = (int)min(t1 - tb, (long)kS);    /* samples of the tile before t1 */
             float GV[kS], VV[kS];
             if constexpr (MODE == kEstepStats) {
@@ -399,80 +434,84 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                 buf ^= 1;
                 continue;
             } else {
-            /* ---- model posteriors, by wave 0 alone: lane hh*kS + s holds model
-             * hh, sample s; the other waves read them from LDS after a second
-             * barrier ---- */
+            /* ---- model posteriors, by wave 0 alone: row s of 16 lanes holds
+             * sample s, lane hh of it model hh (M <= 8), so that row rotations
+             * by 1, 2, 4 (and 8) reach every model; the other waves read them
+             * from LDS after a second barrier.  For m <= 3 lane hh + 8 holds
+             * model hh again, else nothing: the order the models' sum has been
+             * formed in with tiles of two samples and of one. ---- */
+            constexpr bool kRow16 = MJ >= 4;
             if (w == 0) {
                 /* the other waves wait for this one at the next barrier: let it
                  * issue ahead of the other workgroup's waves on its SIMD */
                 __builtin_amdgcn_s_setprio(3);
-                float vl;
-                const int hh = lane / kS;
-                const int s = lane - hh * kS;
-                const long t = tb + s;
-                const bool valid = s < nval;
+                const int s = min(lane >> 4, kS - 1), hh = lane & (kRow16 ? 15 : 7);
                 float l = -3.0e38f;
                 if (hh < a.M) {
                     l = dc2[hh];
-                    for (int c = 0; c < a.CW; ++c)
-#pragma unroll
-                        for (int row = 0; row < 4; ++row) l += Lp[buf][hh * a.CW + c][s][row];
+                    for (int c = 0; c < a.CW; ++c) {
+                        const float4 r = *(const float4*)Lp[buf][hh * a.CW + c][s];
+                        l += r.x;
+                        l += r.y;
+                        l += r.z;
+                        l += r.w;
+                    }
                 }
-                /* logsumexp over the models: the lanes of one sample are kS
-                 * apart inside the first row of 16 lanes (M <= 8), so row
-                 * rotations by (1,) 2, 4 and 8 reach all of them */
-                float lmax = l;
-                if constexpr (kS == 1) lmax = row_ror_max<1>(lmax);
+                float lmax = row_ror_max<1>(l);
                 lmax = row_ror_max<2>(lmax);
                 lmax = row_ror_max<4>(lmax);
-                lmax = row_ror_max<8>(lmax);
-                /* lanes hh >= M hold l = -3e38: e = 0 (the first row's lmax is
-                 * a finite model value; lanes past it are never read) */
+                if constexpr (kRow16) lmax = row_ror_max<8>(lmax);
+                /* lanes hh >= M hold l = -3e38: e = 0 */
                 const float e = fast_exp2(l - lmax);
                 float esum = e;
-                if constexpr (kS == 1) esum += dpp<0x121, 0xf, 0xf, false>(esum);
+                esum += dpp<0x121, 0xf, 0xf, false>(esum);
                 esum += dpp<0x122, 0xf, 0xf, false>(esum);
                 esum += dpp<0x124, 0xf, 0xf, false>(esum);
-                esum += dpp<0x128, 0xf, 0xf, false>(esum);
-                vl = valid ? e * fast_rcp(esum) : 0.f;
-                if (lane < a.M * kS) Vp[buf][lane] = vl;
-                if (valid && hh < a.M) {
+                if constexpr (kRow16) esum += dpp<0x128, 0xf, 0xf, false>(esum);
+                const bool mine = (lane & 8) == 0 && (lane >> 4) < kS, valid = s < nval;
+                const float vl = valid ? e * fast_rcp(esum) : 0.f;
+                if (mine) Vp[buf][hh][s] = vl;
+                if (mine && valid && hh < a.M) {
                     vsum_acc += (double)vl;
                     if (hh == 0) ll_acc += (double)(lmax + fast_log2(esum)) * AMICA_LN2;
-                    if (a.ltall) a.ltall[(size_t)hh * a.T + t] = l * (float)AMICA_LN2;
+                    if (a.ltall) a.ltall[(size_t)hh * a.T + tb + s] = l * (float)AMICA_LN2;
                 }
                 __builtin_amdgcn_s_setprio(0);
             }
             __syncthreads();
-            if constexpr (kS == 2) {                      /* both samples in one 8-byte read */
-                const float2 vp = *(const float2*)&Vp[buf][h * 2];
-                VV[0] = vp.x;
-                VV[1] = vp.y;
-            } else {
-                VV[0] = Vp[buf][h];
-            }
+#pragma unroll
+            for (int q = 0; q < kS; ++q) VV[q] = Vp[buf][h][q];
             }
             }
             /* ---- phase 2: responsibilities and statistics ---- */
+            if constexpr (kRecY)
+#pragma unroll
+                for (int s = 0; s < kS; ++s) __asm__ volatile("" : "+v"(BV[s]));
 #pragma unroll
             for (int s = 0; s < kS; ++s) {
-                const long t = tb + s;
                 const float v = VV[s];
                 const float vrs = v * RS[s];
                 float g = 0.f;
 #pragma unroll
                 for (int j = 0; j < MJ; ++j) {
-                    const float u = E[s][j] * vrs;
-                    const float uf = u * SY[s][j];
+                    float u = E[s][j] * vrs;
+                    const float yv = kRecY ? fmaf(sb[j], BV[s], nsbmu[j]) : Y[s][j];
+                    const float sy = YM2[s][j] * yv, yr = sy * yv;
+                    float uf = u * sy;
+                    /* two of the sums round u and u f before they add them (the
+                     * empty asm), or take the products into an FMA: which one is
+                     * fixed here, as it has been for these m and samples, so that
+                     * no other tiling moves a fit's FP32 rounding */
+                    if (MJ >= 5 || (MJ <= 3 && s % 2 == 0)) __asm__ volatile("" : "+v"(u), "+v"(uf));
                     g = fmaf(uf, rsb[j], g);
                     float* aj = acc + j * NSJ;
                     aj[0] += u;
                     aj[1] += uf;
-                    aj[2] = fmaf(uf, SY[s][j], aj[2]);
+                    aj[2] = fmaf(uf, sy, aj[2]);
                     aj[3] = fmaf(u, YM2[s][j], aj[3]);
-                    const float uyr = u * YR[s][j];
+                    const float uyr = u * yr;
                     aj[4] += uyr;
-                    aj[5] = fmaf(uyr, YR[s][j], aj[5]);
+                    aj[5] = fmaf(uyr, yr, aj[5]);
                     aj[6] = fmaf(uyr, LA[s][j], aj[6]);
                 }
                 /* g is 0 on padding channels (rsb = 0) and past t1 (v = 0) */
@@ -481,10 +520,22 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                 acc[NSJ * MJ + 1] = fmaf(v, XV[s], acc[NSJ * MJ + 1]);
                 acc[NSJ * MJ + 2] += g;
                 GV[s] = g;
-                if (!a.g_bf16 && s < nval && wreal) ((float*)a.g)[(size_t)t * a.ldb + bcol] = g;
+                /* one sample at a time: the sums are complete here (empty asm
+                 * with them as operands, no instruction), or the compiler would
+                 * keep several samples' products live, beyond 128 VGPRs */
+#pragma unroll
+                for (int q = 0; q < NS; ++q) __asm__ volatile("" : "+v"(acc[q]));
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (kS == 2) gw[sub] = pack_bf16x2(GV[0], GV[1]);
-            else if (sub & 1) gw[sub >> 1] = pack_bf16x2(gpend, GV[0]);
+            if constexpr (!GB) {
+                if (wreal)
+#pragma unroll
+                    for (int s = 0; s < kS; ++s)
+                        if (s < nval) ((float*)a.g)[(size_t)(tb + s) * a.ldb + bcol] = GV[s];
+            } else if constexpr (kS >= 2) {
+#pragma unroll
+                for (int s = 0; s < kS; s += 2) gw[(sub * kS + s) >> 1] = pack_bf16x2(GV[s], GV[s + 1]);
+            } else if (sub & 1) gw[sub >> 1] = pack_bf16x2(gpend, GV[0]);
             else gpend = GV[0];
             buf ^= 1;
             if (++tiles == kFlush) {
@@ -514,7 +565,7 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
             }
         }
         if constexpr (MODE != kEstepLsum)
-            if (a.g_bf16 && wreal) g8[(size_t)(tg >> 3) * a.ldb + bcol] = make_uint4(gw[0], gw[1], gw[2], gw[3]);
+            if (GB && wreal) g8[(size_t)(tg >> 3) * a.ldb + bcol] = make_uint4(gw[0], gw[1], gw[2], gw[3]);
     }
     if constexpr (MODE == kEstepLsum) return;
     if constexpr (kL3Batched) {
@@ -529,11 +580,11 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
         }
     }
     if constexpr (MODE == kEstepStats) return;   /* vsum and the LL sum: estep_post_kernel */
-    /* per-model vsum (lanes hh*kS + s of wave 0) and the LL sum (lanes s) */
+    /* per-model vsum (lanes 16 s + hh of wave 0) and the LL sum (lanes 16 s) */
     if (w == 0) {
         const size_t tail = (size_t)a.M * NS * a.NP;
         for (int hh = 0; hh < a.M; ++hh) {
-            const double vs = wave_sum_f64((lane / kS == hh) ? vsum_acc : 0.0);
+            const double vs = wave_sum_f64((lane & 15) == hh ? vsum_acc : 0.0);
             if (lane == 0) base[tail + hh] = vs;
         }
         const double ls = wave_sum_f64(ll_acc);
@@ -870,17 +921,15 @@ int estep_configure(int MJ, size_t lds_bytes) {
     hipError_t r = hipSuccess;
 #define AMICA_ESTEP_ATTR(J)                                                                       \
     case J:                                                                                       \
-        r = hipFuncSetAttribute((const void*)estep_kernel<J, true, kEstepFused>,                 \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);      \
-        if (r == hipSuccess)                                                                      \
-            r = hipFuncSetAttribute((const void*)estep_kernel<J, false, kEstepFused>,            \
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);  \
-        if (r == hipSuccess)                                                                      \
-            r = hipFuncSetAttribute((const void*)estep_kernel<J, true, kEstepStats>,             \
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);  \
-        if (r == hipSuccess)                                                                      \
-            r = hipFuncSetAttribute((const void*)estep_kernel<J, false, kEstepStats>,            \
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);  \
+        for (const void* fn : {(const void*)estep_kernel<J, true, kEstepFused, false>,            \
+                               (const void*)estep_kernel<J, false, kEstepFused, false>,           \
+                               (const void*)estep_kernel<J, false, kEstepFused, true>,            \
+                               (const void*)estep_kernel<J, true, kEstepStats, false>,            \
+                               (const void*)estep_kernel<J, false, kEstepStats, false>,           \
+                               (const void*)estep_kernel<J, false, kEstepStats, true>})           \
+            if (r == hipSuccess)                                                                  \
+                r = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,           \
+                                        (int)lds_bytes);                                          \
         if (r == hipSuccess)                                                                      \
             r = hipFuncSetAttribute((const void*)estep_m1_batch_kernel<J, false>,                \
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);  \
@@ -913,27 +962,29 @@ size_t estep_lds_bytes(int MJ, int threads, bool m1b64) {
     return (m1b64 && MJ == 3) ? (tot + 7) / 8 * 8 + (size_t)2 * MJ * threads * sizeof(double) : tot;
 }
 
+/* Workgroups per CU that the sample ranges are cut for.  A range decides where
+ * its FP32 sums round, so for the kernels that exchange posteriors it follows
+ * from the shape alone -- these waves per SIMD and LDS bytes -- and not from the
+ * registers a build happens to use; where fewer workgroups fit, the rest of
+ * the ranges run in a second wave of equal length. */
 int estep_blocks_per_cu(int MJ, bool b64, int threads, bool m1, bool split) {
+    if (MJ < 1 || MJ > AMICA_MAX_MJ || threads < 64) return -1;
+    if (!m1) {
+        static const int fused[2][AMICA_MAX_MJ] = {{4, 4, 4, 4, 3, 3, 2, 2}, {4, 4, 4, 3, 3, 2, 2, 2}};
+        static const int stats[2][AMICA_MAX_MJ] = {{5, 4, 3, 4, 3, 3, 2, 2}, {6, 4, 4, 4, 3, 3, 2, 2}};
+        const int waves = 4 * (split ? stats : fused)[b64][MJ - 1];
+        const size_t lds = estep_lds_bytes(MJ, threads) + (MJ <= 3 ? 832 : 576) + (b64 && MJ == 3 ? 24576 : 0);
+        return (int)std::max<size_t>(1, std::min<size_t>(waves / (threads / 64), 163840 / lds));
+    }
     int nb = 0;
-    const size_t shm = estep_lds_bytes(MJ, threads, m1 && b64);
+    const size_t shm = estep_lds_bytes(MJ, threads, b64);
     hipError_t r = hipErrorInvalidValue;
 #define AMICA_ESTEP_OCC(J)                                                                        \
     case J:                                                                                       \
-        if (m1)                                                                                   \
-            r = b64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, estep_m1_kernel<J, true>, \
-                                                                   threads, shm)                  \
-                    : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, estep_m1_kernel<J, false>,\
-                                                                   threads, shm);                 \
-        else if (split)                                                                           \
-            r = b64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(                               \
-                          &nb, estep_kernel<J, true, kEstepStats>, threads, shm)                  \
-                    : hipOccupancyMaxActiveBlocksPerMultiprocessor(                               \
-                          &nb, estep_kernel<J, false, kEstepStats>, threads, shm);                \
-        else                                                                                      \
-            r = b64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(                               \
-                          &nb, estep_kernel<J, true, kEstepFused>, threads, shm)                  \
-                    : hipOccupancyMaxActiveBlocksPerMultiprocessor(                               \
-                          &nb, estep_kernel<J, false, kEstepFused>, threads, shm);                \
+        r = b64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, estep_m1_kernel<J, true>,     \
+                                                               threads, shm)                      \
+                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, estep_m1_kernel<J, false>,    \
+                                                               threads, shm);                     \
         break;
     switch (MJ) {
         AMICA_ESTEP_OCC(1)
@@ -960,11 +1011,12 @@ static int launch_estep_split(const EstepArgs& a, int MJ, int nblocks, hipStream
     const bool b64 = a.b64 != nullptr;
 #define AMICA_ESTEP_SPLIT(J)                                                                          \
     case J:                                                                                           \
-        if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepLsum>), grid, block, 0, st, a);      \
-        else hipLaunchKernelGGL((estep_kernel<J, false, kEstepLsum>), grid, block, 0, st, a);         \
+        if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepLsum, false>), grid, block, 0, st, a); \
+        else hipLaunchKernelGGL((estep_kernel<J, false, kEstepLsum, false>), grid, block, 0, st, a);  \
         hipLaunchKernelGGL(estep_post_kernel, dim3(nblocks), dim3(256), 0, st, a);                   \
-        if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepStats>), grid, block, shm, st, a);   \
-        else hipLaunchKernelGGL((estep_kernel<J, false, kEstepStats>), grid, block, shm, st, a);      \
+        if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepStats, false>), grid, block, shm, st, a); \
+        else if (a.g_bf16) hipLaunchKernelGGL((estep_kernel<J, false, kEstepStats, true>), grid, block, shm, st, a); \
+        else hipLaunchKernelGGL((estep_kernel<J, false, kEstepStats, false>), grid, block, shm, st, a); \
         break;
     switch (MJ) {
         AMICA_ESTEP_SPLIT(1)
@@ -1021,8 +1073,9 @@ int launch_estep(const EstepArgs& a, int MJ, int nblocks, hipStream_t st) {
             if (b64) hipLaunchKernelGGL((estep_m1_kernel<J, true>), grid, block, shm, st, a); \
             else hipLaunchKernelGGL((estep_m1_kernel<J, false>), grid, block, shm, st, a);    \
         } else {                                                                              \
-            if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepFused>), grid, block, shm, st, a); \
-            else hipLaunchKernelGGL((estep_kernel<J, false, kEstepFused>), grid, block, shm, st, a);    \
+            if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepFused, false>), grid, block, shm, st, a); \
+            else if (a.g_bf16) hipLaunchKernelGGL((estep_kernel<J, false, kEstepFused, true>), grid, block, shm, st, a); \
+            else hipLaunchKernelGGL((estep_kernel<J, false, kEstepFused, false>), grid, block, shm, st, a); \
         }                                                                                     \
         break;
     switch (MJ) {
