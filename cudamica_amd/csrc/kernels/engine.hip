@@ -207,10 +207,14 @@ struct amica_engine {
         return a;
     }
 
+    /* the E-step forms b itself */
+    bool unmixes(const float* lt) const { return b64 && !split && !lt && estep_unmixes(o.M, NP, o.m); }
+
     EstepArgs eargs(float* lt) const {
         EstepArgs a;
         std::memset(&a, 0, sizeof(a));
         a.b = b; a.b64 = b64; a.cst64 = cst64;
+        if (unmixes(lt)) { a.x64 = xw64; a.Wg64 = Wg64; a.wc64 = wc64; }
         a.x = xw; a.g = g; a.cst = cst; a.lconst = lconst; a.part = part; a.ltall = lt;
         a.T = o.T; a.chunk = chunk; a.pstride = pstride;
         a.n = o.n; a.NP = NP; a.M = o.M; a.CW = CW; a.ldb = ldb; a.g_bf16 = bf16;
@@ -253,13 +257,13 @@ struct amica_engine {
         }
         else if (plain)
             LCHK(launch_unmix_f32(xw, Wg32, wc, b, o.T, NP, ldb, cu_budget, st));
-        else
+        else if (!unmixes(ltall_on ? ltall : nullptr))
             LCHK(launch_unmix_f64(xw64, Wg64, wc64, b64, o.T, NP, ldb, cu_budget, st));
         }
         if (with_timing) HIPCHK(hipEventRecord(ev[2], st));
         {
             StageRange r("amica: E-step");
-            LCHK(launch_estep(eargs(ltall_on ? ltall : nullptr), o.m, nblocks, st));
+            LCHK(launch_estep(eargs(ltall_on ? ltall : nullptr), o.m, nblocks, cu_budget, st));
         }
         if (with_timing) HIPCHK(hipEventRecord(ev[3], st));
         {
@@ -852,6 +856,10 @@ int amica_engine_output(amica_engine* e, double* A_out, double* c_out) {
 int amica_engine_debug_buffer(amica_engine* e, const char* name, void* out, size_t bytes) {
     if (!e || !name || !out) return fail(AMICA_E_INVALID, "null argument");
     HIPCHK(hipSetDevice(e->o.device));
+    /* b of the last E-step where that formed it itself, from the same W */
+    if (std::strcmp(name, "b64") == 0 && e->unmixes(nullptr))
+        if (launch_unmix_f64(e->xw64, e->Wg64, e->wc64, e->b64, e->o.T, e->NP, e->ldb, e->cus, e->st))
+            return fail(AMICA_E_DEVICE, "unmixing launch failed");
     HIPCHK(hipStreamSynchronize(e->st));
     const long T = e->o.T;
     const size_t NP = e->NP, ldb = e->ldb;

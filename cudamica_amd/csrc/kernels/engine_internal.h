@@ -81,6 +81,9 @@ struct EstepArgs {
     const float* b;        /* [T][ldb] (FP32 unmixing) */
     const double* b64;     /* [T][ldb] (FP64 unmixing), or null */
     const double* cst64;   /* [M][kNumCst64][m][NP] when b64 is set */
+    const double* x64;     /* [T][NP], and the GEMM copies of W and W c: set where the */
+    const double* Wg64;    /* E-step forms b itself (estep_unmixes) */
+    const double* wc64;
     const float* x;        /* [T][NP] whitened data */
     void* g;               /* fp32 [T][ldb], or bf16 [T32/8][ldb][8] (8 samples packed) */
     const float* cst;      /* [M][kNumCst][m][NP] */
@@ -104,7 +107,9 @@ struct EstepArgs {
 /* Workgroup shape of the split E-step for M models of CW channel blocks:
  * models per group, channel blocks per group, channel groups, groups. */
 void estep_split_shape(int M, int CW, int* mg, int* cwg, int* ncg, int* ngroups);
-int launch_estep(const EstepArgs& a, int m, int nblocks, hipStream_t st);
+int launch_estep(const EstepArgs& a, int m, int nblocks, int cus, hipStream_t st);
+/* The FP32-path shapes whose E-step forms b itself (no per-sample L recorded). */
+bool estep_unmixes(int M, int NP, int m);
 /* Single-model E-steps of many recordings (BF16 path, same NP) in one
  * launch, one workgroup per work item (device arrays). */
 int launch_estep_m1_batch(const EstepArgs* args, const BatchItem* items, int nitems, int m, int NP,

@@ -592,6 +592,69 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
     }
 }
 
+/* 4 x 4 transpose between the registers r[0..3] and the four rows of 16 lanes */
+__device__ __forceinline__ void transpose_rows(uint32_t& r0, uint32_t& r1, uint32_t& r2, uint32_t& r3) {
+    auto p = __builtin_amdgcn_permlane32_swap(r0, r2, false, false);
+    auto q = __builtin_amdgcn_permlane32_swap(r1, r3, false, false);
+    auto s = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+    auto t = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+    r0 = s[0]; r1 = s[1]; r2 = t[0]; r3 = t[1];
+}
+
+/* elements 2 q and 2 q + 1 in row q of a and b -> element q in a's row q and
+ * 4 + q in b's */
+__device__ __forceinline__ void swap_pairs(uint32_t& a, uint32_t& b) {
+    auto p = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    auto q = __builtin_amdgcn_permlane32_swap(p[0], p[1], false, false);
+    a = q[0]; b = q[1];
+}
+
+/* d[s] = sum_k W[lane][k] x[tb + s][k] for 16 samples of a 64-channel block:
+ * v_mfma_f64_16x16x4f64 in the order of unmix_f64_lds_kernel (the same b), whose
+ * results -- register r of lane l holds sample l/16 + 4 r of channel l%16 of
+ * each 16 -- turn into a channel per lane by row transposes.  wfrag: the W
+ * fragments, [k / 4][16-channel block][lane]. */
+__device__ __forceinline__ void unmix_tile64(const double* __restrict__ x64, const double* wfrag, long tb,
+                                             long T, int lane, double (&d)[16]) {
+    typedef double f64x4 __attribute__((ext_vector_type(4)));
+    const double* const xr = x64 + (size_t)min(tb + (lane & 15), T - 1) * 64 + 2 * (lane >> 4);
+    uint4 xv[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) xv[k] = *(const uint4*)(xr + 8 * k);
+    double xa[16];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        uint32_t lo0 = xv[k].x, hi0 = xv[k].y, lo1 = xv[k].z, hi1 = xv[k].w;
+        swap_pairs(lo0, lo1);
+        swap_pairs(hi0, hi1);
+        xa[2 * k] = __builtin_bit_cast(double, (uint64_t)lo0 | (uint64_t)hi0 << 32);
+        xa[2 * k + 1] = __builtin_bit_cast(double, (uint64_t)lo1 | (uint64_t)hi1 << 32);
+    }
+    f64x4 acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = (f64x4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[k], wfrag[(k * 4 + c) * 64 + lane], acc[c], 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint64_t v = __builtin_bit_cast(uint64_t, (double)acc[c][r]);
+            lo[c] = (uint32_t)v;
+            hi[c] = (uint32_t)(v >> 32);
+        }
+        transpose_rows(lo[0], lo[1], lo[2], lo[3]);
+        transpose_rows(hi[0], hi[1], hi[2], hi[3]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            d[4 * r + q] = __builtin_bit_cast(double, (uint64_t)lo[q] | (uint64_t)hi[q] << 32);
+    }
+}
+
 /* M = 1: the model posterior v is 1, so the waves of a workgroup (the
  * 64-channel blocks of one range of samples) never exchange anything: no
  * barrier, no LDS, and phase 2 of a sample follows its phase 1 in
@@ -601,24 +664,23 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
  * workgroup's slot of the partial buffer.  The log-likelihood sum is sum_t sum_i q_ti (the
  * model constant is added by the reduction); vsum is the sample count.
  * Not used when per-sample L is recorded (ltall). */
-template <int MJ, bool B64>
+template <int MJ, bool B64, bool FUSE>
 __device__ __forceinline__ void estep_m1_body(const EstepArgs& a, const long t0, const long t1,
-                                              const int slot) {
+                                              const int slot, const double* wfrag, float* const tot2_all,
+                                              const double* c64s) {
     constexpr int NSJ = kStatsPerJ;
     constexpr int NS = NSJ * MJ + kStatsPerI;
     constexpr int G = 8;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const bool gpacked = !FUSE && a.g_bf16;
+    const int lane = threadIdx.x & 63, w = FUSE ? 0 : threadIdx.x >> 6;
     const int i = w * 64 + lane;
     const bool act = i < a.n;
-    __shared__ double llw[kMaxEstepWaves];
-
     constexpr int NSP = NS | 1;
-    extern __shared__ float tot2_all[];
     float* const tot2 = tot2_all + threadIdx.x * NSP;
     /* FP32 path, m = 3: the FP64 constants live in LDS ([2 j + k][thread]
      * after the totals, each thread its own slots), read once per sample:
      * 12 VGPRs fewer, so that 4 waves per SIMD fit */
-    constexpr bool kC64Lds = B64 && MJ == 3;
+    constexpr bool kC64Lds = B64 && !FUSE && MJ == 3;
     double* const c64 = (double*)((char*)tot2_all + ((size_t)blockDim.x * NSP * sizeof(float) + 7) / 8 * 8);
 
     float sb[MJ], nsbmu[MJ], rm2[MJ], cq2[MJ], rsb[MJ];
@@ -634,7 +696,7 @@ __device__ __forceinline__ void estep_m1_body(const EstepArgs& a, const long t0,
         rm2[j] = act ? cj[kCstRm2 * ks] : 0.f;
         cq2[j] = act ? cj[kCstCq2 * ks] : (j == 0 ? AMICA_L2E : -1e30f);
         rsb[j] = act ? cj[kCstRsb * ks] : 0.f;
-        if constexpr (B64) {
+        if constexpr (B64 && !FUSE) {
             const double* dj = a.cst64 + (size_t)j * a.NP + i;
             sb64[j] = act ? dj[kCst64Sb * ks] : 0.0;
             nsbmu64[j] = act ? dj[kCst64Nsbmu * ks] : 1.0;
@@ -681,7 +743,8 @@ __device__ __forceinline__ void estep_m1_body(const EstepArgs& a, const long t0,
     const int vob = (int)bcol * kEb, vox = i * 4;
     auto ld = [&](long t, float& bqv, double& dqv, float& xqv) {
         const int r = (int)(min(t, a.T) - t0);
-        if constexpr (B64)
+        if constexpr (FUSE) {
+        } else if constexpr (B64)
             dqv = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rb, vob, r * a.ldb * kEb, 0));
         else
             bqv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, vob, r * a.ldb * kEb, 0));
@@ -695,28 +758,40 @@ __device__ __forceinline__ void estep_m1_body(const EstepArgs& a, const long t0,
     }
     const long tend = t0 + (t1 - t0 + G - 1) / G * G;   /* whole 8-sample groups */
     int grp = 0;
+    double d16[FUSE ? 16 : 1];
+    double bias = 0.0;
+    if constexpr (FUSE) bias = a.wc64[lane];
 #pragma unroll 1
     for (long tg = t0; tg < tend; tg += G, ++grp) {
         uint32_t gw[G / 2];                           /* packed bf16 g, 2 samples a word */
         float gprev = 0.f;
+        if constexpr (FUSE) {
+            if ((grp & 1) == 0) unmix_tile64(a.x64, wfrag, tg, a.T, lane, d16);
+            else
+#pragma unroll
+                for (int u = 0; u < 8; ++u) d16[u] = d16[8 + u];
+        }
 #pragma unroll
         for (int u = 0; u < G; ++u) {
             const long t = tg + u;
             const bool valid = t < t1;                /* wave-uniform */
             const int sl = u % PF;
             const float bcur = B64 ? 0.f : bq[sl];
-            const double dcur = dq[sl];
+            double dcur;
+            if constexpr (FUSE) dcur = valid ? d16[u] - bias : 0.0;
+            else dcur = dq[sl];
             const float xcur = xq[sl];
             ld(t + PF, bq[sl], dq[sl], xq[sl]);
             const float bv = B64 ? (float)dcur : bcur;
             /* the constants' LDS reads stay in the loop (not hoisted back into
              * registers): a compiler-only fence, no instruction */
-            if constexpr (kC64Lds) __asm__ volatile("" ::: "memory");
+            if constexpr (kC64Lds || FUSE) __asm__ volatile("" ::: "memory");
             float q2[MJ], E[MJ], SY[MJ], YM2[MJ], YR[MJ], LA[MJ];
 #pragma unroll
             for (int j = 0; j < MJ; ++j) {
                 float y;
-                if constexpr (kC64Lds)
+                if constexpr (FUSE) y = (float)fma(c64s[2 * j * 64 + lane], dcur, c64s[(2 * j + 1) * 64 + lane]);
+                else if constexpr (kC64Lds)
                     y = (float)fma(c64[(size_t)(2 * j) * blockDim.x + threadIdx.x], dcur,
                                    c64[(size_t)(2 * j + 1) * blockDim.x + threadIdx.x]);
                 else if constexpr (B64) y = (float)fma(sb64[j], dcur, nsbmu64[j]);
@@ -766,7 +841,7 @@ __device__ __forceinline__ void estep_m1_body(const EstepArgs& a, const long t0,
             acc[NSJ * MJ + 0] = fmaf(bv, bv, acc[NSJ * MJ + 0]);
             acc[NSJ * MJ + 1] += xcur;
             acc[NSJ * MJ + 2] += g;
-            if (a.g_bf16) {
+            if (gpacked) {
                 if (u & 1) gw[u >> 1] = pack_bf16x2(gprev, g);
                 gprev = g;
             } else if (valid) {
@@ -782,7 +857,7 @@ __device__ __forceinline__ void estep_m1_body(const EstepArgs& a, const long t0,
             __builtin_amdgcn_sched_barrier(0);
         }
         /* t0 is a multiple of 8: the group's packed word */
-        if (a.g_bf16) g8[(size_t)((tg) >> 3) * a.ldb + bcol] = make_uint4(gw[0], gw[1], gw[2], gw[3]);
+        if (gpacked) g8[(size_t)((tg) >> 3) * a.ldb + bcol] = make_uint4(gw[0], gw[1], gw[2], gw[3]);
         if ((grp & 3) == 3) {                         /* 32 samples */
 #pragma unroll
             for (int s = 0; s < NS; ++s) { tot2[s] += acc[s]; acc[s] = 0.f; }
@@ -799,21 +874,69 @@ __device__ __forceinline__ void estep_m1_body(const EstepArgs& a, const long t0,
     l3_accumulate<NS, 8>(l3, l3_started, act, [&](int s) { return (double)tot2[s] + (double)acc[s]; });
     qtot += (double)qacc;
     const double ls = wave_sum_f64(qtot);
-    if (lane == 0) llw[w] = ls;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double l = 0.0;
-        for (int c = 0; c < (int)(blockDim.x >> 6); ++c) l += llw[c];
-        const size_t tail = (size_t)NS * a.NP;
-        base[tail] = (double)(t1 - t0);
-        base[tail + 1] = l * AMICA_LN2;
+    const size_t tail = (size_t)NS * a.NP;
+    if constexpr (FUSE) {
+        if (lane == 0) {
+            base[tail] = (double)(t1 - t0);
+            base[tail + 1] = ls * AMICA_LN2;
+        }
+    } else {
+        __shared__ double llw[kMaxEstepWaves];
+        if (lane == 0) llw[w] = ls;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double l = 0.0;
+            for (int c = 0; c < (int)(blockDim.x >> 6); ++c) l += llw[c];
+            base[tail] = (double)(t1 - t0);
+            base[tail + 1] = l * AMICA_LN2;
+        }
     }
 }
 
 template <int MJ, bool B64>
 __global__ __launch_bounds__(512) void estep_m1_kernel(EstepArgs a) {
+    extern __shared__ float tot2_all[];
     const long t0 = (long)blockIdx.x * a.chunk;
-    estep_m1_body<MJ, B64>(a, t0, min(a.T, t0 + a.chunk), (int)blockIdx.x);
+    estep_m1_body<MJ, B64, false>(a, t0, min(a.T, t0 + a.chunk), (int)blockIdx.x, nullptr, tot2_all, nullptr);
+}
+
+/* n <= 64 channels, one model, FP32 path: each wave forms b of its own samples,
+ * 16 at a time, and b never goes to memory -- two of the five passes of the
+ * separate unmixing and E-step (x read and b written; b and x read, g
+ * written), which are bound by HBM at 4.3-5 TB/s.  W's fragments and the FP64
+ * constants are in LDS, once for the workgroup's waves, which share nothing else
+ * (a range of samples each).  What bounds it is issue on the SIMDs: 59 % of
+ * the cycles the vector ALU (101 instructions a sample at m = 3), 32 % the FP64
+ * MFMAs, which do not run beside it; the next tile's x loaded ahead and wave
+ * priorities by phase changed nothing.  64 ch x 1M, us, unmixing and E-step
+ * together: m = 1 436 -> 355, m = 2 440 -> 332, m = 3 482 -> 400; 16 ch x 20k 35
+ * -> 32; 40 ch x 5k 28 and 28.  For m > 3 the kernel needs more than 128 VGPRs,
+ * and for NP > 64 W does not fit LDS: those keep the two launches. */
+template <int MJ>
+__global__ __launch_bounds__(1024, MJ == 1 ? 5 : 4) void estep_m1_unmix_kernel(EstepArgs a, int nranges, int nw) {
+    __shared__ double wfrag[64 * 64];
+    __shared__ double c64s[2 * MJ * 64];
+    extern __shared__ float tot2_all[];
+    /* two of W's entries a load, four loads in flight */
+#pragma unroll 4
+    for (int e = threadIdx.x; e < 32 * 64; e += blockDim.x) {
+        const int col = e >> 5, k = 2 * (e & 31);
+        const double2 v = *(const double2*)(a.Wg64 + (size_t)col * 64 + k);
+        double* const f = wfrag + ((k >> 2) * 4 + (col >> 4)) * 64 + (k & 3) * 16 + (col & 15);
+        f[0] = v.x;
+        f[16] = v.y;
+    }
+    for (int e = threadIdx.x; e < 2 * MJ * 64; e += blockDim.x) {
+        const int i = e & 63, k = (e >> 6) & 1, j = e >> 7;
+        c64s[e] = i < a.n ? a.cst64[((size_t)(k == 0 ? kCst64Sb : kCst64Nsbmu) * MJ + j) * 64 + i]
+                          : (k == 0 ? 0.0 : 1.0);
+    }
+    __syncthreads();
+    /* waves past nw only help with the copies above */
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = blockIdx.x * nw + w;
+    if (w >= nw || r >= nranges) return;
+    const long t0 = (long)r * a.chunk;
+    estep_m1_body<MJ, true, true>(a, t0, min(a.T, t0 + a.chunk), r, wfrag, tot2_all, c64s);
 }
 
 /* Many recordings in one launch: workgroup b runs work item b, a range of
@@ -824,7 +947,8 @@ __global__ __launch_bounds__(512) void estep_m1_batch_kernel(const EstepArgs* __
                                                              const BatchItem* __restrict__ items) {
     const BatchItem it = items[blockIdx.x];
     const EstepArgs a = args[it.rec];
-    estep_m1_body<MJ, B64>(a, it.t0, it.t1, it.slot);
+    extern __shared__ float tot2_all[];
+    estep_m1_body<MJ, B64, false>(a, it.t0, it.t1, it.slot, nullptr, tot2_all, nullptr);
 }
 
 /* The split launch's middle pass: per sample, the model log-likelihoods
@@ -952,6 +1076,11 @@ int estep_configure(int MJ, size_t lds_bytes) {
         default: return -1;
     }
 #undef AMICA_ESTEP_ATTR
+    if (MJ <= 3 && r == hipSuccess)
+        r = hipFuncSetAttribute(MJ == 1   ? (const void*)estep_m1_unmix_kernel<1>
+                                : MJ == 2 ? (const void*)estep_m1_unmix_kernel<2>
+                                          : (const void*)estep_m1_unmix_kernel<3>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)estep_lds_bytes(MJ, 1024));
     return r == hipSuccess ? 0 : -1;
 }
 
@@ -1033,6 +1162,17 @@ static int launch_estep_split(const EstepArgs& a, int MJ, int nblocks, hipStream
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+/* where it is faster than unmixing and E-step apart (estep_m1_unmix_kernel) */
+bool estep_unmixes(int M, int NP, int MJ) { return M == 1 && NP == 64 && MJ <= 3; }
+
+/* Waves per workgroup of estep_m1_unmix_kernel: a CU's share of the ranges up to
+ * 16, and where it is more (m = 1: five waves per SIMD) half of it, an even
+ * number, for two workgroups */
+static int estep_unmix_waves(int nranges, int cus) {
+    const int per = std::max(1, (nranges + cus - 1) / cus);
+    return per <= 16 ? per : std::min(16, (per + 3) / 4 * 2);
+}
+
 int launch_estep_m1_batch(const EstepArgs* args, const BatchItem* items, int nitems, int MJ, int NP,
                           hipStream_t st) {
     if (nitems < 1 || NP % 64 || NP > 64 * kMaxEstepWaves) return -1;
@@ -1057,7 +1197,7 @@ int launch_estep_m1_batch(const EstepArgs* args, const BatchItem* items, int nit
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int launch_estep(const EstepArgs& a, int MJ, int nblocks, hipStream_t st) {
+int launch_estep(const EstepArgs& a, int MJ, int nblocks, int cus, hipStream_t st) {
     if (a.split) return launch_estep_split(a, MJ, nblocks, st);
     if (a.M * a.CW > kMaxEstepWaves || a.M > 8 || (a.chunk % 8) != 0) return -1;
     /* byte offsets of the rows a workgroup reads (its chunk and the next
@@ -1067,6 +1207,15 @@ int launch_estep(const EstepArgs& a, int MJ, int nblocks, hipStream_t st) {
     const bool b64 = a.b64 != nullptr;
     const bool m1 = a.M == 1 && a.ltall == nullptr;
     const size_t shm = estep_lds_bytes(MJ, (int)block.x, m1 && b64);
+    if (a.Wg64 && m1 && estep_unmixes(a.M, a.NP, MJ)) {
+        const int nw = estep_unmix_waves(nblocks, cus);
+        const dim3 ug((nblocks + nw - 1) / nw), ub(64 * std::max(nw, 4));
+        const size_t us = estep_lds_bytes(MJ, (int)ub.x);
+        if (MJ == 1) hipLaunchKernelGGL((estep_m1_unmix_kernel<1>), ug, ub, us, st, a, nblocks, nw);
+        else if (MJ == 2) hipLaunchKernelGGL((estep_m1_unmix_kernel<2>), ug, ub, us, st, a, nblocks, nw);
+        else hipLaunchKernelGGL((estep_m1_unmix_kernel<3>), ug, ub, us, st, a, nblocks, nw);
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
 #define AMICA_ESTEP_CASE(J)                                                                   \
     case J:                                                                                   \
         if (m1) {                                                                             \
