@@ -1108,14 +1108,22 @@ static void launch_gj(const MstepArgs& ma, hipStream_t st) {
 }
 
 /* W_h = A_h^-1 and log|det W_h| of every model: one workgroup per model,
- * the matrix in registers, up to 192 channels; the blocked kernels beyond
- * (registers per lane of a panel: R rows x NB columns <= 64 doubles) */
+ * the matrix in registers, up to 192 channels; the blocked kernels beyond,
+ * with R = ceil(n / 64) rows a lane up to 512 channels.  A panel's columns are a
+ * serial chain in one wave (about 1.9 us each), so rows that are only padding
+ * cost the whole inverse: with R = 8 from 257 channels on, and 16-column
+ * panels at R = 4, the prepare stage took (us, before -> now) 505 -> 471 at 256
+ * channels x 2 models, 638 -> 534 at 260, 801 -> 668 at 300 x 3, 933 -> 839 at
+ * 350.  Panels of 4, 10 or 12 columns are within 5 % either way. */
 static void launch_inverse(const MstepArgs& ma, hipStream_t st) {
     const int n = ma.n;
     if (n <= 64) launch_gj_small<1, 4>(ma, st);
     else if (n <= 128) launch_gj_small<2, 8>(ma, st);
     else if (n <= 192) launch_gj_small<3, 12>(ma, st);
-    else if (n <= 256) launch_gj<4, 16>(ma, st);
+    else if (n <= 256) launch_gj<4, 8>(ma, st);
+    else if (n <= 320) launch_gj<5, 8>(ma, st);
+    else if (n <= 384) launch_gj<6, 8>(ma, st);
+    else if (n <= 448) launch_gj<7, 8>(ma, st);
     else if (n <= 512) launch_gj<8, 8>(ma, st);
     else launch_gj<16, 4>(ma, st);
 }
