@@ -680,10 +680,16 @@ public:
     ~Workspace() {
         if (!b_.p) return;
         if (!drained_) (void)hipStreamSynchronize(st_);
-        std::vector<void*> drop;
+        /* at most one block more than the pool keeps per device leaves at a time */
+        void* drop[kPoolBlocks + 2];
+        int nd = 0;
         {
             std::lock_guard<std::mutex> lock(g_pool_mu);
-            g_pool.push_back(b_);
+            try {
+                g_pool.push_back(b_);
+            } catch (...) {                 /* no host memory to remember it in */
+                drop[nd++] = b_.p;
+            }
             /* the smallest blocks leave first */
             for (;;) {
                 size_t sum = 0, least = 0;
@@ -694,17 +700,18 @@ public:
                     sum += g_pool[k].bytes;
                     ++cnt;
                 }
-                if (cnt <= kPoolBlocks && sum <= kPoolBytes) break;
-                drop.push_back(g_pool[least].p);
+                if ((cnt <= kPoolBlocks && sum <= kPoolBytes) || nd == kPoolBlocks + 2) break;
+                drop[nd++] = g_pool[least].p;
                 g_pool.erase(g_pool.begin() + least);
             }
         }
-        for (void* p : drop) (void)hipFree(p);
+        for (int k = 0; k < nd; ++k) (void)hipFree(drop[k]);
     }
     /* the smallest idle block of at least `bytes`, or a new one */
     void* take(size_t bytes) {
         bytes = (bytes + ((size_t)1 << 20) - 1) >> 20 << 20;
-        std::vector<void*> drop;
+        void* drop[kPoolBlocks + 2];
+        int nd = 0;
         {
             std::lock_guard<std::mutex> lock(g_pool_mu);
             size_t best = g_pool.size();
@@ -724,12 +731,12 @@ public:
             {
                 std::lock_guard<std::mutex> lock(g_pool_mu);
                 for (size_t k = g_pool.size(); k-- > 0;)
-                    if (g_pool[k].dev == dev_) {
-                        drop.push_back(g_pool[k].p);
+                    if (g_pool[k].dev == dev_ && nd < kPoolBlocks + 2) {
+                        drop[nd++] = g_pool[k].p;
                         g_pool.erase(g_pool.begin() + k);
                     }
             }
-            for (void* q : drop) (void)hipFree(q);
+            for (int k = 0; k < nd; ++k) (void)hipFree(drop[k]);
             if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
         }
         b_ = PoolBlock{dev_, p, bytes};

@@ -10,7 +10,8 @@
  *   part     FP64 [nblocks][pstride] E-step partial statistics
  *   gxpart   FP64 [nchunks][ldb][NP] partials of G = sum_t g x^T
  *   params   FP64 A, c, alpha, mu, beta, rho, gm, W, ldet (+ GEMM copy of W)
- * One EM iteration is eight launches on one stream, with every decision of
+ * One EM iteration is ten launches on one stream (nine where the E-step forms b
+ * itself; more beyond 192 channels and for split E-steps), with every decision of
  * the reference's host loop (LL decrease, Newton test, lrate schedule) made
  * on the device, so an iteration can be replayed as one hipGraph.
  */

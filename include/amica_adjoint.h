@@ -39,9 +39,12 @@
  *   stream     hipStream_t the work is enqueued on (NULL: the default stream)
  * Limits: 1 <= m <= 8, n <= 1024, M <= 16 (the reference's range).  Where
  * M * ceil(n/64) * 64 > 512 the likelihood runs in three passes through
- * per-sample buffers of (M ceil(n/64) + M) doubles.  The call allocates its
- * workspace, synchronises `stream` before it returns and returns 0, or a
- * negative AMICA_E_* code of amica_engine.h with amica_last_error() set.
+ * per-sample buffers of (M ceil(n/64) + M) doubles.  The samples run in chunks
+ * whose buffers stay below 256 MB; the workspace comes from a kept pool (at most
+ * two blocks, 1 GiB, per GPU; a call that needs more, or finds none free,
+ * allocates its own and frees it).  The call synchronises `stream` before it
+ * returns and returns 0, or a negative AMICA_E_* code of amica_engine.h with
+ * amica_last_error() set.
  */
 #ifndef AMICA_ADJOINT_H_
 #define AMICA_ADJOINT_H_

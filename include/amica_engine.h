@@ -132,7 +132,8 @@ int  amica_engine_output(amica_engine* eng, double* A_out, double* c_out);
 
 /* Average duration (ms) of each kernel class over the last timed
  * iterations, measured with HIP events on the engine stream (ms[5]):
- * [0] W = A^-1 and the E-step constants, [1] unmixing GEMM, [2] fused
+ * [0] W = A^-1 and the E-step constants, [1] unmixing GEMM (nothing where the
+ * E-step forms b itself: one model of up to 64 channels on the FP32 path, m <= 3), [2] fused
  * E-step, [3] statistic GEMM, [4] reductions + M-step.  Enabled by
  * amica_engine_set_timing(eng, 1). */
 int  amica_engine_set_timing(amica_engine* eng, int on);
