@@ -46,7 +46,8 @@
  * 40) and the flushes.  So the fixed work is shared out: tiles of four samples
  * (two for m = 4, one above) pass the two barriers that publish the channel
  * sums and then the model posteriors, which one wave evaluates for the
- * workgroup, a row of 16 lanes to a sample; one underflow test serves a tile;
+ * workgroup, a row of 16 lanes to a sample; one underflow test serves a tile,
+ * and decides before the densities are evaluated;
  * b loads are issued a tile ahead, x loads before the tile's densities.  What
  * that costs in registers comes back by keeping only what an FMA or two cannot
  * form again.  The per-lane LDS footprint (FP32 level-2 totals) leaves room
@@ -165,6 +166,8 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
     constexpr int kS = estep_tile_samples(MJ, B64);
     /* y is not kept between the phases but formed again, where that is one FMA */
     constexpr bool kRecY = !B64;
+    /* the underflow test before the densities (below) */
+    constexpr bool kShiftFirst = kS == 4 && MODE == kEstepFused;
     constexpr int kFlush = 32 / kS;     /* tiles summed in FP32 registers (32 samples) */
     /* FP64 flushes with batched loads, except in the split launch's
      * statistics pass, which they would push past 128 VGPRs on the FP32
@@ -348,6 +351,72 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
             for (int s = 0; s < kS; ++s) load_tile(tb + kS + s, s);
             /* ---- phase 1: densities, component posteriors, channel sums ---- */
             float QS[kS];
+            /* q2 <= log2(alpha sqrt(beta) / (2 Gamma(1 + 1/rho))), a few units,
+             * so 2^q2 needs no max shift unless every component underflows (a
+             * sample far from all of them: sum 2^q2 < 2^-100): then, for the
+             * whole wave, that sample's are shifted by the per-lane max.  The
+             * max alone says so (2^off <= sum <= 8 * 2^off) but for a narrow
+             * band, in which the sum is formed to see.  Heavy-tailed data shift
+             * some lane of nearly every wave's samples, so the densities are
+             * evaluated once, after that is known, and not again with the shift: 3.42
+             * -> 3.04 ms a launch at 128 ch x 2M x 4 models of super-Gaussian
+             * sources, no change where none is that far out.  Smaller tiles and
+             * the split launch, with fewer samples to overlap, evaluate first
+             * and shift afterwards: 961 instead of 1000 us at 256 ch x 500k x 2
+             * models m = 4, 350 instead of 369 at 300 ch x 60k x 3 models.  Both
+             * give the same bits. */
+            if constexpr (kShiftFirst) {
+            float off[kS];
+#pragma unroll
+            for (int s = 0; s < kS; ++s) {
+#pragma unroll
+                for (int j = 0; j < MJ; ++j) {
+                    float y;
+                    if constexpr (kC64Lds)
+                        y = (float)fma(c64s[(2 * j) * 512 + threadIdx.x], BV64[s],
+                                       c64s[(2 * j + 1) * 512 + threadIdx.x]);
+                    else if constexpr (B64) y = (float)fma(sb64[j], BV64[s], nsbmu64[j]);
+                    else y = fmaf(sb[j], BV[s], nsbmu[j]);
+                    const float la = fast_log2(fmaxf(fabsf(y), y_floor<B64>()));
+                    const float ym2 = fast_exp2(rm2[j] * la);
+                    const float yr = (ym2 * y) * y;
+                    E[s][j] = fmaf(yr, -AMICA_L2E, cq2[j]);               /* q2 */
+                    off[s] = j == 0 ? E[s][0] : fmaxf(off[s], E[s][j]);
+                    Y[s][j] = y; YM2[s][j] = ym2; LA[s][j] = la;
+                }
+            }
+            float omin = off[0];
+#pragma unroll
+            for (int s = 1; s < kS; ++s) omin = fminf(omin, off[s]);
+            const bool far = __builtin_expect(__any(omin < -99.5f), 0);
+            if (far) {
+#pragma unroll
+                for (int s = 0; s < kS; ++s) {
+                    bool shift = __any(off[s] < -103.5f);
+                    if (!shift && __any(off[s] < -99.5f)) {
+                        float se = 0.f;
+#pragma unroll
+                        for (int j = 0; j < MJ; ++j) se = j == 0 ? fast_exp2(E[s][0]) : se + fast_exp2(E[s][j]);
+                        shift = __any(se < 0x1p-100f);
+                    }
+                    off[s] = shift ? off[s] : 0.f;
+#pragma unroll
+                    for (int j = 0; j < MJ; ++j) E[s][j] -= off[s];
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < kS; ++s) {
+#pragma unroll
+                for (int j = 0; j < MJ; ++j) {
+                    E[s][j] = fast_exp2(E[s][j]);
+                    SE[s] = j == 0 ? E[s][j] : SE[s] + E[s][j];
+                }
+                QS[s] = fast_log2(SE[s]);         /* exactly 0 on padding channels */
+            }
+            if (far)
+#pragma unroll
+                for (int s = 0; s < kS; ++s) QS[s] += off[s];
+            } else {
 #pragma unroll
             for (int s = 0; s < kS; ++s) {
                 SE[s] = 0.f;
@@ -368,13 +437,8 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                 }
                 QS[s] = fast_log2(SE[s]);         /* exactly 0 on padding channels */
             }
-            /* q2 <= log2(alpha sqrt(beta) / (2 Gamma(1 + 1/rho))), a few units,
-             * so 2^q2 needs no max shift unless every component underflows (a
-             * sample far from all of them): then, for the whole wave, that
-             * sample's are shifted by the per-lane max.  One test per tile: the
-             * samples' densities stay one block of independent chains.  (The
-             * empty asm, here and before phase 2, keeps the compiler from
-             * holding on to the y it could form again.) */
+            /* (the empty asm, here and before phase 2, keeps the compiler from
+             * holding on to the y it could form again) */
             if constexpr (kRecY)
 #pragma unroll
                 for (int s = 0; s < kS; ++s) __asm__ volatile("" : "+v"(BV[s]));
@@ -400,6 +464,7 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                     }
                     QS[s] = off + fast_log2(SE[s]);
                 }
+            }
             }
 #pragma unroll
             for (int s = 0; s < kS; ++s) RS[s] = fast_rcp(SE[s]);
