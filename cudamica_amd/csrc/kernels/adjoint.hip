@@ -350,7 +350,7 @@ __global__ __launch_bounds__(512) void ll_kernel(AdjArgs a) {
                 const Real ay = fmax(fabs(y), B::kTiny);
                 la[s][j] = B::log(ay);
                 const Real p = B::exp(rm1[j] * la[s][j]);         /* |y|^(rho-1) */
-                yr[s][j] = p * ay;
+                yr[s][j] = p * fabs(y);       /* not ay, which is kTiny for a NaN */
                 if constexpr (ADJ) ps[s][j] = y > (Real)0 ? p : y < (Real)0 ? -p : y;   /* 0 at 0, NaN stays */
                 Qj[j] = fma(yr[s][j], (Real)-B::kUnit, cq[j]);
                 mx = (j == 0) ? Qj[j] : fmax(mx, Qj[j]);
