@@ -659,8 +659,9 @@ int launch_ll(int MJ, const AdjArgs& a, int nblocks, hipStream_t st) {
  * a gigabyte).  A call owns its block until its stream has drained (the
  * destructor waits where the call did not), so blocks in the pool are idle and
  * any thread and stream may take one.  At most kPoolBlocks stay per device, of
- * kPoolBytes in all; the rest, and every idle block when an allocation fails,
- * goes back to the device. */
+ * kPoolBytes in all; the rest goes back to the device, and every idle block on
+ * request (amica_ll_release_workspace) and where an allocation of this library
+ * fails (device_malloc). */
 constexpr size_t kPoolBytes = (size_t)1 << 30;
 constexpr int kPoolBlocks = 2;
 
@@ -672,6 +673,25 @@ struct PoolBlock {
 std::mutex g_pool_mu;
 std::vector<PoolBlock> g_pool;
 
+/* frees the idle blocks of device dev (-1: of all) */
+hipError_t release_pool(int dev) {
+    hipError_t first = hipSuccess;
+    for (;;) {
+        void* p = nullptr;
+        {
+            std::lock_guard<std::mutex> lock(g_pool_mu);
+            for (size_t k = 0; k < g_pool.size() && !p; ++k) {
+                if (dev >= 0 && g_pool[k].dev != dev) continue;
+                p = g_pool[k].p;
+                g_pool.erase(g_pool.begin() + k);
+            }
+        }
+        if (!p) return first;
+        const hipError_t e = hipFree(p);
+        if (first == hipSuccess) first = e;
+    }
+}
+
 class Workspace {
 public:
     Workspace(int dev, hipStream_t st) : dev_(dev), st_(st) {}
@@ -679,7 +699,12 @@ public:
     Workspace& operator=(const Workspace&) = delete;
     ~Workspace() {
         if (!b_.p) return;
-        if (!drained_) (void)hipStreamSynchronize(st_);
+        if (!drained_ && hipStreamSynchronize(st_) != hipSuccess) {
+            /* the stream's work may still run: not for another call (hipFree waits
+             * for the device) */
+            (void)hipFree(b_.p);
+            return;
+        }
         /* at most one block more than the pool keeps per device leaves at a time */
         void* drop[kPoolBlocks + 2];
         int nd = 0;
@@ -710,8 +735,6 @@ public:
     /* the smallest idle block of at least `bytes`, or a new one */
     void* take(size_t bytes) {
         bytes = (bytes + ((size_t)1 << 20) - 1) >> 20 << 20;
-        void* drop[kPoolBlocks + 2];
-        int nd = 0;
         {
             std::lock_guard<std::mutex> lock(g_pool_mu);
             size_t best = g_pool.size();
@@ -726,19 +749,7 @@ public:
             }
         }
         void* p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            {
-                std::lock_guard<std::mutex> lock(g_pool_mu);
-                for (size_t k = g_pool.size(); k-- > 0;)
-                    if (g_pool[k].dev == dev_ && nd < kPoolBlocks + 2) {
-                        drop[nd++] = g_pool[k].p;
-                        g_pool.erase(g_pool.begin() + k);
-                    }
-            }
-            for (int k = 0; k < nd; ++k) (void)hipFree(drop[k]);
-            if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
-        }
+        if (device_malloc(&p, bytes) != hipSuccess) return nullptr;
         b_ = PoolBlock{dev_, p, bytes};
         return p;
     }
@@ -947,8 +958,8 @@ int run_chunks(AdjArgs a, const void* x, long T, const double* dll, double* ll, 
         if (hipGetLastError() != hipSuccess) return report_error(AMICA_E_DEVICE, "adjoint launch failed");
     }
     const hipError_t e = hipStreamSynchronize(st);
-    ws.drained();
     if (e != hipSuccess) return report_error(AMICA_E_DEVICE, hipGetErrorString(e));
+    ws.drained();
     return 0;
 }
 
@@ -1004,7 +1015,23 @@ int ll_call(int real_bits, const void* x, long T, int n, int M, int m, const dou
 
 }  // namespace
 
+hipError_t device_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        int dev = 0;
+        if (hipGetDevice(&dev) == hipSuccess && release_pool(dev) == hipSuccess) e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) (void)hipGetLastError();     /* reported by the caller, not by a later launch */
+    return e;
+}
+
 }  // namespace amica
+
+extern "C" int amica_ll_release_workspace(void) {
+    const hipError_t e = amica::release_pool(-1);
+    return e == hipSuccess ? 0 : amica::report_error(AMICA_E_DEVICE, hipGetErrorString(e));
+}
 
 extern "C" int amica_ll_forward(int real_bits, const void* x, long T, int n, int M, int m,
                                 const double* W, const double* c, const double* alpha,

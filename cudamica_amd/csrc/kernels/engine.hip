@@ -370,7 +370,7 @@ int amica_engine_create(const amica_options* opts, amica_engine** out) {
     const int n = o.n, M = o.M, m = o.m;
     auto alloc = [&](void** p, size_t bytes) -> int {
         if (bytes == 0) bytes = 8;
-        hipError_t r = hipMalloc(p, bytes);
+        hipError_t r = device_malloc(p, bytes);
         if (r != hipSuccess) return fail(AMICA_E_NOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
         r = hipMemset(*p, 0, bytes);
         if (r != hipSuccess) return fail(AMICA_E_DEVICE, "hipMemset failed");
@@ -521,7 +521,7 @@ int amica_engine_load_raw(amica_engine* e, const float* x, int x_on_device) {
     if (!e || !x) return fail(AMICA_E_INVALID, "null argument");
     HIPCHK(hipSetDevice(e->o.device));
     const size_t bytes = (size_t)e->o.T * e->o.n * sizeof(float);
-    if (!e->xraw) HIPCHK(hipMalloc((void**)&e->xraw, bytes));
+    if (!e->xraw) HIPCHK(device_malloc((void**)&e->xraw, bytes));
     HIPCHK(hipMemcpyAsync(e->xraw, x, bytes, x_on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, e->st));
     HIPCHK(hipStreamSynchronize(e->st));
     e->have_data = 1;
@@ -535,7 +535,7 @@ int amica_engine_center(amica_engine* e) {
     const int n = e->o.n;
     const long T = e->o.T;
     double* part = nullptr;
-    HIPCHK(hipMalloc((void**)&part, sphere_part_doubles(T, n, e->cus) * sizeof(double)));
+    HIPCHK(device_malloc((void**)&part, sphere_part_doubles(T, n, e->cus) * sizeof(double)));
     const int rc = launch_colmean(e->xraw, T, n, part, e->cus, e->mean, e->st);
     const hipError_t se = hipStreamSynchronize(e->st);
     (void)hipFree(part);
@@ -566,11 +566,11 @@ int amica_engine_whiten(amica_engine* e, int do_sphere) {
     const size_t partn = std::max(std::max(sphere_part_doubles(T, n, e->cus), (size_t)nchunks * 2 * n),
                                   (size_t)nchunks * e->NP);
     double* ns = nullptr;
-    HIPCHK(hipMalloc((void**)&part, partn * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&C, (size_t)n * n * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&V, (size_t)n * n * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&d, (size_t)n * sizeof(double)));
-    if (do_sphere == 1) HIPCHK(hipMalloc((void**)&ns, inv_sqrt_doubles(n) * sizeof(double)));
+    HIPCHK(device_malloc((void**)&part, partn * sizeof(double)));
+    HIPCHK(device_malloc((void**)&C, (size_t)n * n * sizeof(double)));
+    HIPCHK(device_malloc((void**)&V, (size_t)n * n * sizeof(double)));
+    HIPCHK(device_malloc((void**)&d, (size_t)n * sizeof(double)));
+    if (do_sphere == 1) HIPCHK(device_malloc((void**)&ns, inv_sqrt_doubles(n) * sizeof(double)));
     int rc = 0;
     do {
         bool have_S = false;
@@ -618,13 +618,13 @@ int amica_engine_load_white(amica_engine* e, const double* xw, double ldetS) {
     HIPCHK(hipSetDevice(e->o.device));
     const size_t cnt = (size_t)e->o.T * e->o.n;
     double* tmp = nullptr;
-    HIPCHK(hipMalloc((void**)&tmp, cnt * sizeof(double)));
+    HIPCHK(device_malloc((void**)&tmp, cnt * sizeof(double)));
     HIPCHK(hipMemcpy(tmp, xw, cnt * sizeof(double), hipMemcpyHostToDevice));
     int rc = launch_white_from_f64(tmp, e->o.T, e->o.n, e->NP, e->xw, e->xw64, e->xbf, e->st);
     float* qpart = nullptr;
     const int qchunks = (int)std::max(1L, std::min((long)e->cus * 2, e->o.T / 64 + 1));
     if (!rc && e->fp8) {
-        if (hipMalloc((void**)&qpart, (size_t)qchunks * e->NP * sizeof(float)) != hipSuccess) rc = -1;
+        if (device_malloc((void**)&qpart, (size_t)qchunks * e->NP * sizeof(float)) != hipSuccess) rc = -1;
         else rc = launch_quantize_fp8(e->xw, e->o.T, e->NP, e->xscale, e->xq, e->x8, qpart, qchunks, e->st);
     } else if (!rc && e->x8) {
         rc = launch_pack8(e->xbf, e->o.T, e->NP, e->x8, e->st);
@@ -801,7 +801,7 @@ int amica_engine_record_ltall(amica_engine* e, int on) {
     if (!e) return fail(AMICA_E_INVALID, "null engine");
     HIPCHK(hipSetDevice(e->o.device));
     if (on && !e->ltall) {
-        HIPCHK(hipMalloc((void**)&e->ltall, (size_t)e->o.M * e->o.T * sizeof(float)));
+        HIPCHK(device_malloc((void**)&e->ltall, (size_t)e->o.M * e->o.T * sizeof(float)));
         if (e->gexec) {   /* the captured graph does not record ltall */
             (void)hipGraphExecDestroy(e->gexec);
             (void)hipGraphDestroy(e->graph);
@@ -839,10 +839,10 @@ int amica_engine_output(amica_engine* e, double* A_out, double* c_out) {
     const int n = e->o.n, M = e->o.M;
     const size_t nn = (size_t)n * n;
     double *work = nullptr, *Sinv = nullptr, *Ao = nullptr, *co = nullptr;
-    HIPCHK(hipMalloc((void**)&work, (16 + nn + inverse_work_doubles(n, 1)) * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&Sinv, nn * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&Ao, M * nn * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&co, (size_t)M * n * sizeof(double)));
+    HIPCHK(device_malloc((void**)&work, (16 + nn + inverse_work_doubles(n, 1)) * sizeof(double)));
+    HIPCHK(device_malloc((void**)&Sinv, nn * sizeof(double)));
+    HIPCHK(device_malloc((void**)&Ao, M * nn * sizeof(double)));
+    HIPCHK(device_malloc((void**)&co, (size_t)M * n * sizeof(double)));
     int rc = launch_output_transform(e->S, e->mean, e->A, e->c, n, M, work, Sinv, Ao, co, e->st);
     hipError_t se = hipStreamSynchronize(e->st);
     if (!rc && se == hipSuccess) {
@@ -1033,7 +1033,7 @@ struct amica_batch {
             const size_t b_ua = bytes(ua.size(), sizeof(UnmixArgs)), b_ea = bytes(ea.size(), sizeof(EstepArgs)),
                          b_ga = bytes(ga.size(), sizeof(GxArgs)), b_iu = bytes(iu.size(), sizeof(BatchItem)),
                          b_ie = bytes(ie.size(), sizeof(BatchItem)), b_ig = bytes(ig.size(), sizeof(BatchItem));
-            HIPCHK(hipMalloc(&g.dmem, b_ua + b_ea + b_ga + b_iu + b_ie + b_ig));
+            HIPCHK(device_malloc(&g.dmem, b_ua + b_ea + b_ga + b_iu + b_ie + b_ig));
             char* p = (char*)g.dmem;
             g.ua = (UnmixArgs*)p; p += b_ua;
             g.ea = (EstepArgs*)p; p += b_ea;

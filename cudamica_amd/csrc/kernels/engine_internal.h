@@ -13,6 +13,10 @@ namespace amica {
 /* Sets the message amica_last_error() returns; returns code. */
 int report_error(int code, const char* msg);
 
+/* hipMalloc on the current device; where that is out of memory, again after the
+ * idle workspaces of the likelihood calls went back to it. */
+hipError_t device_malloc(void** p, size_t bytes);
+
 /* Per-(h, j, i) FP32 constants of the E-step, table [M][kNumCst][m][NP]. */
 enum {
     kCstSb = 0,     /* sqrt(beta) */

@@ -10,6 +10,7 @@
 #include <algorithm>
 
 #include "amica_engine.h"
+#include "engine_internal.h"
 
 namespace {
 
@@ -80,9 +81,9 @@ extern "C" int amica_hbm_probe(int device, size_t bytes, int reps, double* copy_
     int rc = AMICA_E_DEVICE;
     double best_copy = 0.0, best_read = 0.0;
     do {
-        if (hipMalloc((void**)&a, n4 * sizeof(float4)) != hipSuccess) break;
-        if (hipMalloc((void**)&b, n4 * sizeof(float4)) != hipSuccess) break;
-        if (hipMalloc((void**)&sums, (size_t)nblk * sizeof(float)) != hipSuccess) break;
+        if (amica::device_malloc((void**)&a, n4 * sizeof(float4)) != hipSuccess) break;
+        if (amica::device_malloc((void**)&b, n4 * sizeof(float4)) != hipSuccess) break;
+        if (amica::device_malloc((void**)&sums, (size_t)nblk * sizeof(float)) != hipSuccess) break;
         if (hipStreamCreate(&st) != hipSuccess) break;
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) break;
         const unsigned fblk = (unsigned)((n4 + kProbeThreads - 1) / kProbeThreads);

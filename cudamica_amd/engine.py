@@ -98,6 +98,7 @@ _SIGNATURES = [
      + [ctypes.c_double, _V, _V]),
     ("amica_ll_adjoint", ctypes.c_int, [ctypes.c_int, _V, ctypes.c_long, ctypes.c_int, ctypes.c_int,
                                         ctypes.c_int] + [_V] * 7 + [ctypes.c_double] + [_V] * 10),
+    ("amica_ll_release_workspace", ctypes.c_int, []),
 ]
 
 _lib = None
@@ -440,3 +441,8 @@ def ll_adjoint(real_bits, x, T, n, M, m, params, ldetS, dll, grads, ll=0, stream
     _check(L.amica_ll_adjoint(real_bits, x, T, n, M, m, *[params[k] for k in PARAM_NAMES], ldetS,
                               dll, ll, *[grads[k] for k in PARAM_NAMES], stream),
            "amica_ll_adjoint")
+
+
+def ll_release_workspace():
+    """Free the device memory ll_forward and ll_adjoint keep between calls."""
+    _check(load_library().amica_ll_release_workspace(), "amica_ll_release_workspace")

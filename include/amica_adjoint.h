@@ -42,7 +42,8 @@
  * per-sample buffers of (M ceil(n/64) + M) doubles.  The samples run in chunks
  * whose buffers stay below 256 MB; the workspace comes from a kept pool (at most
  * two blocks, 1 GiB, per GPU; a call that needs more, or finds none free,
- * allocates its own and frees it).  The call synchronises `stream` before it
+ * allocates its own and frees it).  amica_ll_release_workspace gives the idle
+ * blocks back.  The call synchronises `stream` before it
  * returns and returns 0, or a negative AMICA_E_* code of amica_engine.h with
  * amica_last_error() set.
  */
@@ -62,7 +63,7 @@ int amica_ll_forward(int real_bits, const void* x, long T, int n, int M, int m,
  * for callers that cannot allocate device memory (code under hipGraph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments and result as amica_ll_forward, up to the rounding of b (it
- * forms b = W x - W c per lane, amica_ll_forward on MFMA into a buffer);
+ * forms b = W x - W c 16 samples at a time, amica_ll_forward in a GEMM);
  * its workspace is a static device array of 1.6 MB per GPU (held until the
  * process ends), so it also requires M * n * n <= 65536 and
  * M * ceil(n/64) * 64 <= 512 and rejects larger models with
@@ -79,6 +80,12 @@ int amica_ll_adjoint(int real_bits, const void* x, long T, int n, int M, int m,
                      const double* beta, const double* rho, const double* gm, double ldetS,
                      const double* dll, double* ll, double* dW, double* dc, double* dalpha,
                      double* dmu, double* dbeta, double* drho, double* dgm, void* stream);
+
+/* Frees the device memory that amica_ll_forward and amica_ll_adjoint keep for
+ * later calls (on every GPU), for programs whose other allocators need it;
+ * calls that run meanwhile keep theirs.  An engine short of memory takes it
+ * without being asked to.  Returns 0 or AMICA_E_DEVICE. */
+int amica_ll_release_workspace(void);
 
 #ifdef __cplusplus
 }
