@@ -24,8 +24,8 @@
  * where they fit in 8, else three passes through per-sample buffers; the
  * allocation-free forward instead forms b there, 16 samples at a time on
  * MFMA), gx (sum_t g_t x_t^T on FP32 or FP64 MFMA over sample chunks) and the
- * sums of their partials; finish assembles the gradients from the chunks'
- * totals.
+ * sums of their partials onto the chunks' running totals, from which finish
+ * assembles the gradients.
  * Every reduction is in a fixed order, so results repeat bit for bit.
  */
 #include <hip/hip_runtime.h>
@@ -560,22 +560,15 @@ struct AdjOut {
     double *dW, *dc, *dalpha, *dmu, *dbeta, *drho, *dgm;
 };
 
-/* The gradients from the totals of the raw sums (raw, nc sets of pcount, one
- * per chunk of samples) and of sum_t g_t x_t^T (G, nc sets of ldg gxs).  Grid
- * (eb + n / 4, M): workgroups below eb take dW and the densities' gradients,
- * the others four entries of dc, one per wave. */
+/* The gradients from the totals of the raw sums (raw) and of sum_t g_t x_t^T (G,
+ * rows of gxs).  Grid (eb + n / 4, M): workgroups below eb take dW and the
+ * densities' gradients, the others four entries of dc, one per wave. */
 __global__ __launch_bounds__(256) void adj_finish_kernel(AdjArgs a, int eb, const double* __restrict__ raw,
-                                                         size_t pcount, const double* __restrict__ G, int gxs,
-                                                         int nc, AdjOut o) {
+                                                         const double* __restrict__ G, int gxs, AdjOut o) {
     const int h = blockIdx.y, n = a.n, m = a.m, NP = a.NP, ps = pair_stride(m);
     const int nm = n * m, nn = n * n;
     const size_t ldg = (size_t)a.M * NP;
-    auto total = [&](size_t e) {
-        double s = 0.0;
-        for (int c = 0; c < nc; ++c) s += raw[(size_t)c * pcount + e];
-        return s;
-    };
-    auto gsum = [&](int i) { return total(((size_t)h * NP + i) * ps + 4 * m); };
+    auto gsum = [&](int i) { return raw[((size_t)h * NP + i) * ps + 4 * m]; };
     const double* W = a.W + (size_t)h * nn;
     if ((int)blockIdx.x >= eb) {
         const int lane = threadIdx.x & 63, k = ((int)blockIdx.x - eb) * 4 + ((int)threadIdx.x >> 6);
@@ -586,23 +579,21 @@ __global__ __launch_bounds__(256) void adj_finish_kernel(AdjArgs a, int eb, cons
         if (lane == 0) o.dc[(size_t)h * n + k] = s;
         return;
     }
-    const double om = total((size_t)ldg * ps + h);
+    const double om = raw[ldg * ps + h];
     for (int q = (int)blockIdx.x * 256 + threadIdx.x; q < nn + nm; q += eb * 256) {
         if (q >= nn) {
             const int e0 = q - nn, j = e0 / n, i = e0 - j * n;
             const size_t e = (size_t)h * nm + e0, off = ((size_t)h * NP + i) * ps + j;
             const double be = a.beta[e], rh = a.rho[e];
-            const double su = total(off), sup = total(off + m), suy = total(off + 2 * m), sul = total(off + 3 * m);
+            const double su = raw[off], sup = raw[off + m], suy = raw[off + 2 * m], sul = raw[off + 3 * m];
             o.dalpha[e] = su / a.alpha[e];
             o.dmu[e] = sqrt(be) * rh * sup;
             o.dbeta[e] = (su - rh * suy) / (2.0 * be);
             o.drho[e] = su * psi_dev(1.0 + 1.0 / rh) / (rh * rh) - sul;
         } else {
             const int i = q % n, k = q / n;
-            double s = 0.0;
-            for (int c = 0; c < nc; ++c) s += G[((size_t)c * ldg + (size_t)h * NP + i) * gxs + k];
             o.dW[(size_t)h * nn + q] = om * a.Winv[(size_t)h * nn + k + (size_t)i * n] -
-                                       (s - gsum(i) * a.c[(size_t)h * n + k]);
+                                       (G[((size_t)h * NP + i) * gxs + k] - gsum(i) * a.c[(size_t)h * n + k]);
         }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) o.dgm[h] = om / a.gm[h];
@@ -899,8 +890,8 @@ int run_chunks(AdjArgs a, const void* x, long T, const double* dll, double* ll, 
             a.g = k.take<Real>((size_t)Tc * ldb);
             a.part = k.take<double>((size_t)nb * a.pstride);
             gxpart = k.take<double>((size_t)gchunks * gcount);
-            ptot = k.take<double>((size_t)C * pcount);
-            gtot = k.take<double>((size_t)C * gcount);
+            ptot = k.take<double>(pcount);
+            gtot = k.take<double>(gcount);
             tmp = k.take<double>(sum_tmp_doubles(nb, pcount) + sum_tmp_doubles(gchunks, gcount));
         }
         return k.off;
@@ -946,15 +937,15 @@ int run_chunks(AdjArgs a, const void* x, long T, const double* dll, double* ll, 
             hipLaunchKernelGGL(adj_gx_kernel, dim3(gc, ldb / 64, (n + 63) / 64), dim3(256), 0, st,
                                (const double*)a.g, xc, Tn, n, ldb, gch, gxpart);
         }
+        /* onto the chunks' running totals, in their order */
         if (hipGetLastError() != hipSuccess ||
-            launch_sum_parts(a.part, nbn, a.pstride, pcount, ptot + (size_t)c * pcount, gxpart, gc, gcount,
-                             gtot + (size_t)c * gcount, tmp, st))
+            launch_sum_parts(a.part, nbn, a.pstride, pcount, ptot, gxpart, gc, gcount, gtot, tmp, c > 0, st))
             return report_error(AMICA_E_DEVICE, "adjoint launch failed");
     }
     if (adj) {
         const int eb = (int)std::min<size_t>(1024, (nn + (size_t)n * m + 255) / 256);
-        hipLaunchKernelGGL(adj_finish_kernel, dim3(eb + (n + 3) / 4, M), dim3(256), 0, st, a, eb, ptot, pcount, gtot,
-                           gxs, C, *out);
+        hipLaunchKernelGGL(adj_finish_kernel, dim3(eb + (n + 3) / 4, M), dim3(256), 0, st, a, eb, ptot, gtot, gxs,
+                           *out);
         if (hipGetLastError() != hipSuccess) return report_error(AMICA_E_DEVICE, "adjoint launch failed");
     }
     const hipError_t e = hipStreamSynchronize(st);

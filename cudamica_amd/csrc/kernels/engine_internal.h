@@ -221,11 +221,12 @@ struct MstepArgs {
 };
 
 /* Fixed-order sums of two sets of partials in one launch (two where a set is
- * summed in groups first): out_a[e] = sum_p pa[p stride_a + e], e < len_a, and
- * out_b likewise with stride len_b; tmp holds the sum_tmp_doubles of both. */
+ * summed in groups first): out_a[e] = sum_p pa[p stride_a + e], e < len_a (with
+ * add, += that), and out_b likewise with stride len_b; tmp holds the
+ * sum_tmp_doubles of both. */
 size_t sum_tmp_doubles(int nparts, size_t len);
 int launch_sum_parts(const double* pa, int na, size_t stride_a, size_t len_a, double* out_a, const double* pb,
-                     int nb, size_t len_b, double* out_b, double* tmp, hipStream_t st);
+                     int nb, size_t len_b, double* out_b, double* tmp, bool add, hipStream_t st);
 /* Sum E-step partials and the statistic-GEMM partials, then write the
  * canonical statistics (including phi through the unmixing identity) and, with
  * mstep, take the part of the M-step that needs no phi (launch_mstep is the

@@ -66,12 +66,12 @@ __device__ double block_sum(double v, double* sh) {
 
 /* One set of partials to sum: out[y][e] = sum of part[p][e] over the partials
  * p of group y ([y PG, (y + 1) PG)), e < len, by xb workgroups of 64 elements
- * (lanes) per group, G groups. */
+ * (lanes) per group, G groups; with add, that sum added to out. */
 struct SumSeg {
     const double* part;
     double* out;
     size_t stride, len;
-    int nparts, PG, xb, G;
+    int nparts, PG, xb, G, add;
 };
 
 /* Two sets in one launch (the E-step's partials and the statistic GEMM's):
@@ -99,7 +99,8 @@ __global__ __launch_bounds__(64 * kSumWaves) void sum_parts_kernel(SumSeg a, Sum
     if (w == 0 && e < s.len) {
         double t = 0.0;
         for (int q = 0; q < kSumWaves; ++q) t += acc[q][lane];
-        s.out[(size_t)y * s.len + e] = t;
+        double* const o = s.out + (size_t)y * s.len + e;
+        *o = s.add ? *o + t : t;
     }
 }
 
@@ -1141,14 +1142,15 @@ static int sum_groups(int nparts, size_t len) {
 
 /* The first pass over one set of partials: all of them into out, or (G > 1)
  * groups into tmp, whose sum the second pass takes into out. */
-static SumSeg first_pass(const double* part, int nparts, size_t stride, size_t len, double* tmp, double* out) {
+static SumSeg first_pass(const double* part, int nparts, size_t stride, size_t len, double* tmp, double* out,
+                         bool add) {
     const int G = sum_groups(nparts, len), PG = (nparts + G - 1) / G;
-    return SumSeg{part, G == 1 ? out : tmp, stride, len, nparts, PG, (int)((len + 63) / 64), G};
+    return SumSeg{part, G == 1 ? out : tmp, stride, len, nparts, PG, (int)((len + 63) / 64), G, G == 1 && add};
 }
 
-static SumSeg second_pass(const SumSeg& f, double* out) {
-    if (f.G == 1) return SumSeg{nullptr, nullptr, 0, 0, 0, 0, 0, 0};
-    return SumSeg{f.out, out, f.len, f.len, f.G, f.G, f.xb, 1};
+static SumSeg second_pass(const SumSeg& f, double* out, bool add) {
+    if (f.G == 1) return SumSeg{nullptr, nullptr, 0, 0, 0, 0, 0, 0, 0};
+    return SumSeg{f.out, out, f.len, f.len, f.G, f.G, f.xb, 1, add};
 }
 
 size_t sum_tmp_doubles(int nparts, size_t len) {
@@ -1157,11 +1159,11 @@ size_t sum_tmp_doubles(int nparts, size_t len) {
 }
 
 int launch_sum_parts(const double* pa, int na, size_t stride_a, size_t len_a, double* out_a, const double* pb,
-                     int nb, size_t len_b, double* out_b, double* tmp, hipStream_t st) {
-    const SumSeg p = first_pass(pa, na, stride_a, len_a, tmp, out_a);
-    const SumSeg g = first_pass(pb, nb, len_b, len_b, tmp + sum_tmp_doubles(na, len_a), out_b);
+                     int nb, size_t len_b, double* out_b, double* tmp, bool add, hipStream_t st) {
+    const SumSeg p = first_pass(pa, na, stride_a, len_a, tmp, out_a, add);
+    const SumSeg g = first_pass(pb, nb, len_b, len_b, tmp + sum_tmp_doubles(na, len_a), out_b, add);
     hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(p.xb * p.G + g.xb * g.G)), dim3(64 * kSumWaves), 0, st, p, g);
-    const SumSeg p2 = second_pass(p, out_a), g2 = second_pass(g, out_b);
+    const SumSeg p2 = second_pass(p, out_a, add), g2 = second_pass(g, out_b, add);
     if (p2.xb + g2.xb > 0)
         hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(p2.xb + g2.xb)), dim3(64 * kSumWaves), 0, st, p2, g2);
     return hipGetLastError() == hipSuccess ? 0 : -1;
@@ -1173,7 +1175,7 @@ int launch_reduce(const double* part, int nparts, size_t pstride, const double* 
     const int NS = kStatsPerJ * ma.m + kStatsPerI;
     const size_t plen = (size_t)ma.M * NS * ma.NP + ma.M + 1;
     const size_t glen = (size_t)ma.ldb * ma.NP;
-    if (launch_sum_parts(part, nparts, pstride, plen, raw, gxpart, nchunks, glen, gxtot, tmp, st)) return -1;
+    if (launch_sum_parts(part, nparts, pstride, plen, raw, gxpart, nchunks, glen, gxtot, tmp, false, st)) return -1;
     /* one 16 x 16 tile of phi per workgroup, after the statistics' */
     const unsigned ntk = (unsigned)((ma.n + 15) / 16);
     const dim3 grid(ma.M, 1 + ntk * ntk);

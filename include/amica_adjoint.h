@@ -40,9 +40,12 @@
  * Limits: 1 <= m <= 8, n <= 1024, M <= 16 (the reference's range).  Where
  * M * ceil(n/64) * 64 > 512 the likelihood runs in three passes through
  * per-sample buffers of (M ceil(n/64) + M) doubles.  The samples run in chunks
- * whose buffers stay below 256 MB; the workspace comes from a kept pool (at most
- * two blocks, 1 GiB, per GPU; a call that needs more, or finds none free,
- * allocates its own and frees it).  amica_ll_release_workspace gives the idle
+ * of about 256 MiB of per-sample buffers, or of 4096 samples where a sample
+ * takes more than 64 KiB (1.1 GB at the largest shapes: 1024 channels, 16 models,
+ * FP64); the rest of the workspace -- a few matrices of a model's size and the
+ * partial sums of one chunk -- does not grow with T either.  It comes from a
+ * kept pool (at most two blocks, 1 GiB, per GPU; a call that needs more, or finds
+ * none free, allocates its own and frees it).  amica_ll_release_workspace gives the idle
  * blocks back.  The call synchronises `stream` before it
  * returns and returns 0, or a negative AMICA_E_* code of amica_engine.h with
  * amica_last_error() set.

@@ -80,3 +80,26 @@ def test_threads_and_streams_share_the_pool(built):
         t.join()
     for a, b in zip(want, got):
         assert b is not None and all(torch.equal(u, v) for u, v in zip(a, b))
+
+
+def _adjoint_block(n, T, M):
+    """Device memory an adjoint call (FP64, one component) leaves in the pool."""
+    p = _model(n, M, 1, n)
+    x = torch.randn((T, n), device="cuda", dtype=torch.float64)
+    dll = torch.ones(T, device="cuda", dtype=torch.float64)
+    g = {k: torch.empty_like(v) for k, v in p.items()}
+    ca.ll_release_workspace()
+    before = torch.cuda.mem_get_info()[0]
+    ca.ll_adjoint(64, x.data_ptr(), T, n, M, 1, {k: v.data_ptr() for k, v in p.items()}, 0.0, dll.data_ptr(),
+                  {k: v.data_ptr() for k, v in g.items()}, 0, torch.cuda.current_stream().cuda_stream)
+    return before - torch.cuda.mem_get_info()[0]
+
+
+def test_the_workspace_does_not_grow_with_the_samples(built):
+    """One chunk of 8000 samples (250 MiB of b and g), and eight of them: the
+    sums of a chunk (16 MiB of them here) are not kept beside each other."""
+    print("[ll workspace] chunks", flush=True)
+    n, M = 1024, 2
+    one = _adjoint_block(n, 8000, M)
+    assert one >= 250 * MIB
+    assert _adjoint_block(n, 8 * 8000, M) <= one + 2 * MIB
