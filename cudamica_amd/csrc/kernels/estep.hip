@@ -164,6 +164,7 @@ constexpr int estep_tile_samples(int MJ, bool B64) { return MJ <= 3 ? 4 : MJ == 
 template <int MJ, bool B64, int MODE, bool GB>
 __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
     constexpr int kS = estep_tile_samples(MJ, B64);
+    static_assert(8 % kS == 0 && 7 + kS <= kEstepRowPad, "the unchecked loads past a range stay in the padding rows");
     /* y is not kept between the phases but formed again, where that is one FMA */
     constexpr bool kRecY = !B64;
     /* the underflow test before the densities (below) */
