@@ -3,8 +3,8 @@
  * (fraimondo/cudamica src/preprocess.cu:31-420), run by the engine of
  * gpus[0] on the GPU: FP64 means, FP64 covariance, FP64 Newton-Schulz
  * inverse square root, or a Jacobi eigen-decomposition where that does not
- * converge (in place of magma_dsyevd_gpu + magma_dgesv_gpu), S = 2 C^-1/2 (do_sphere 1), diag(1/std) (2) or I, ldetS = -log|det S|,
- * x <- S (x - mean).  whiten() writes S to spherefile like the reference.
+ * converge (in place of magma_dsyevd_gpu + magma_dgesv_gpu), S = 2 C^-1/2
+ * (do_sphere 1), diag(1/std) (2) or I, ldetS = -log|det S|, x <- S (x - mean).  whiten() writes S to spherefile like the reference.
  */
 #include "../../../include/preprocess.h"
 

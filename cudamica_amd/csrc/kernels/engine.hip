@@ -405,8 +405,8 @@ int amica_engine_create(const amica_options* opts, amica_engine** out) {
         ALLOC(e->lq, (size_t)T32 * M * e->sp_ncg * sizeof(float));
         ALLOC(e->vq, (size_t)T32 * M * sizeof(float));
     }
-    /* E-step grid: exactly as many workgroups as the CUs hold at once, each
-     * streaming one contiguous range of samples. */
+    /* E-step grid: estep_blocks_per_cu workgroups per CU, each streaming one
+     * contiguous range of samples (estep_m1_unmix_kernel: a wave per range). */
     const int waves = e->split ? e->sp_mg * e->sp_cwg : M * CW;
     {
         const int rc = estep_configure(m, estep_lds_bytes(m, 64 * waves, M == 1 && !e->split && !e->bf16 &&

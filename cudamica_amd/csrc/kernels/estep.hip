@@ -44,7 +44,7 @@
  * FP32 operations at 2.8-3.4 cycles each, per component), the kernel about
  * 450: the rest is loads, the row sums, the exchange between the waves (about
  * 40) and the flushes.  So the fixed work is shared out: tiles of four samples
- * (two for m = 4, one above) pass the two barriers that publish the channel
+ * (two for m = 4 from FP32 b, one above) pass the two barriers that publish the channel
  * sums and then the model posteriors, which one wave evaluates for the
  * workgroup, a row of 16 lanes to a sample; one underflow test serves a tile,
  * and decides before the densities are evaluated;
@@ -222,8 +222,8 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
     float sb[MJ], nsbmu[MJ], rm2[MJ], cq2[MJ], rsb[MJ];
     double sb64[B64 ? MJ : 1], nsbmu64[B64 ? MJ : 1];
     /* FP32 path, m = 3: the FP64 constants live in LDS ([j][2][thread],
-     * conflict-free) and are read once per tile (the barrier orders them),
-     * which keeps the kernel within 128 VGPRs: 4 waves per SIMD */
+     * conflict-free, each thread its own slots), read for every sample, instead
+     * of in 12 VGPRs */
     constexpr bool kC64Lds = B64 && MJ == 3;
     __shared__ double c64s[kC64Lds ? 2 * MJ * 512 : 1];
 #pragma unroll

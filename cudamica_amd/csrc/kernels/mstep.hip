@@ -511,8 +511,9 @@ __global__ __launch_bounds__(256) void prepare_tail_kernel(MstepArgs a, int tb) 
     }
 }
 
-/* Row i of W~ c_h by one wave, lanes over k: the W~ the unmixing GEMM applies (W~ = split(W diag(s)) diag(1/s) on the BF16 and FP8
- * paths, fp32(W) on the plain FP32 path, W itself on the FP32 path). */
+/* Row i of W~ c_h by one wave, lanes over k: the W~ the unmixing GEMM applies
+ * (W~ = split(W diag(s)) diag(1/s) on the BF16 and FP8 paths, fp32(W) on the
+ * plain FP32 path, W itself on the FP32 path). */
 __device__ void wc_rows(const MstepArgs& a, int h, int i) {
     const int n = a.n, lane = threadIdx.x & 63;
     if (i >= n) return;

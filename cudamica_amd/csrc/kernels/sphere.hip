@@ -88,7 +88,7 @@ __global__ __launch_bounds__(1024) void finish_mean_kernel(const double* __restr
  * meet in LDS in wave order.  Fragments are loaded straight from x (lane
  * (i, k) = channel l % 16, sample l / 16: 64-byte runs), kU steps ahead of
  * their use, and centred in registers, so that nothing but the sums goes
- * through LDS.  Bound by the FP64 MFMA rate (64 cycles per 1024 FMAs), and
+ * through LDS (the loads in flight spill 36 bytes a lane at TI = 2, 24 at 4).  Bound by the FP64 MFMA rate (64 cycles per 1024 FMAs), and
  * only one triangle is formed: 0.57 ms at 128 ch x 1M, 1.86 ms at 256 ch (44
  * TFLOP/s of 73; 1.31 ms for both triangles by FMAs from LDS at 128 ch). */
 template <int TI>
@@ -853,7 +853,8 @@ int launch_sphere_matrix(const double* V, const double* d, const double* C, int 
 int launch_whiten(const float* x, const double* mean, const double* S, long T, int n, int NP,
                   float* xw, double* xw64, uint16_t* xbf, uint16_t* x8, hipStream_t st) {
     /* one wave per 64-channel group up to eight (four where the LDS tiles of
-     * eight would not fit beside the rows), four waves at least */
+     * eight would not fit beside the rows), and rows of four waves in all where
+     * the groups are one or two */
     const int WC = NP <= 768 ? std::min(NP / 64, 8) : 4, WR = std::max(1, 4 / WC);
     const int TS = 16 * kWhitenRT * WR;
     const size_t shm = (size_t)TS * (NP + 4) * sizeof(float) + NP * sizeof(double) +
