@@ -44,13 +44,14 @@
  * FP32 operations at 2.8-3.4 cycles each, per component), the kernel about
  * 450: the rest is loads, the row sums, the exchange between the waves (about
  * 40) and the flushes.  So the fixed work is shared out: tiles of four samples
- * (two for m = 4 from FP32 b, one above) pass the two barriers that publish the channel
- * sums and then the model posteriors, which one wave evaluates for the
- * workgroup, a row of 16 lanes to a sample; one underflow test serves a tile,
- * and decides before the densities are evaluated;
- * b loads are issued a tile ahead, x loads before the tile's densities.  What
- * that costs in registers comes back by keeping only what an FMA or two cannot
- * form again.  The per-lane LDS footprint (FP32 level-2 totals) leaves room
+ * (two for m = 4 from FP32 b and for m = 3 from FP64 b in large workgroups, one
+ * above) pass the two barriers that publish the channel sums and then the model
+ * posteriors, which one wave evaluates for the workgroup, a row of 16 lanes to
+ * a sample; one underflow test serves a tile, and with four samples decides
+ * before the densities are evaluated; b loads are issued a tile ahead, x loads
+ * before the tile's densities, or with less than four samples ahead as well.
+ * What that costs in registers comes back by keeping only what an FMA or two
+ * cannot form again; one-sample tiles keep it all.  The per-lane LDS footprint (FP32 level-2 totals) leaves room
  * for two 512-thread workgroups per CU.  Against tiles of two samples (one for
  * m = 4) with every intermediate kept, in us: 128 ch x 1M x 4 models m = 3
  * 1526 -> 1463, 256 ch x 500k x 2 models m = 4 1036 -> 961, 128 ch x 500k x 2
@@ -147,10 +148,27 @@ __device__ __forceinline__ void l3_accumulate(double* l3, bool started, bool kee
     }
 }
 
-/* Samples per tile: as many as keep the kernel at two workgroups of 8 waves
- * per CU (128 VGPRs); with FP64 b at m = 3, where y is kept, four samples leave
- * one, which is faster still (128 ch x 500k x 2 models: 440 us, 522 with two). */
-constexpr int estep_tile_samples(int MJ, bool B64) { return MJ <= 3 ? 4 : MJ == 4 && !B64 ? 2 : 1; }
+/* Samples per tile: as many as keep the kernel at 4 waves per SIMD (128 VGPRs).
+ * With FP64 b at m = 3, where y is kept, four samples take 151 VGPRs and leave 3:
+ * faster for workgroups of up to four waves, which pack three waves a SIMD
+ * (estep of 128 ch x 500k x 2 models: 440 us, 469 with two), slower for larger
+ * ones, of which a CU then holds one instead of two or three (128 ch x 130k x
+ * 4 models 1.24 times, 64 ch x 208k x 5 models 1.35 times), and in the split
+ * launch (300 ch x 74k x 3 models 1.08 times). */
+constexpr int estep_tile_samples(int MJ, bool B64, bool small) {
+    return MJ <= 3 ? (B64 && MJ == 3 && !small ? 2 : 4) : MJ == 4 && !B64 ? 2 : 1;
+}
+constexpr int kSmallWaves = 4;      /* waves of a fused workgroup that counts as small */
+
+/* Whether sy and |y|^rho (and with FP32 b, y) are kept between the phases
+ * instead of formed again, by a product or two each.  One-sample tiles have the
+ * registers for it, but not the split launch's statistics pass up to m = 6, and
+ * not m = 5 on the plain path in workgroups of 5 to 7 waves: kept, it takes 148
+ * VGPRs, and one such workgroup fits a CU where two do with 124 (E-step of 64
+ * ch x 5 models, kept / formed again: 1.5 times; at 2 waves 0.83 times). */
+constexpr bool estep_keeps(int MJ, bool B64, int mode, bool GB, bool mid) {
+    return (MJ >= 5 || (MJ == 4 && B64)) && (mode == kEstepFused ? !(mid && MJ == 5 && !B64 && !GB) : MJ >= 7);
+}
 
 /* MODE selects the launch the kernel serves (GB: g as packed bf16):
  *   kEstepFused  all M models x CW channel blocks in one workgroup (M CW <= 8):
@@ -161,12 +179,16 @@ constexpr int estep_tile_samples(int MJ, bool B64) { return MJ <= 3 ? 4 : MJ == 
  *   kEstepStats  split launch, last pass: the densities again, the model
  *                posteriors read from vq (written between the passes by
  *                estep_post_kernel), then the statistics and g. */
-template <int MJ, bool B64, int MODE, bool GB>
+template <int MJ, bool B64, int MODE, bool GB, int kS, bool kKeep>
 __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
-    constexpr int kS = estep_tile_samples(MJ, B64);
     static_assert(8 % kS == 0 && 7 + kS <= kEstepRowPad, "the unchecked loads past a range stay in the padding rows");
-    /* y is not kept between the phases but formed again, where that is one FMA */
-    constexpr bool kRecY = !B64;
+    static_assert(!kKeep || kS == 1, "larger tiles have no registers to keep more");
+    constexpr bool kRecY = !B64 && !kKeep;
+    /* a tile of four samples is long enough for its own x to arrive behind its
+     * densities; with one or two, x is loaded a tile ahead, as b is (E-step of
+     * 64 ch x 2 models on the FP32 path, us at m = 4, 5, 6, 8 against loads in
+     * the tile: 0.84, 0.82, 0.80, 0.87 times) */
+    constexpr bool kXAhead = kS <= 2;
     /* the underflow test before the densities (below) */
     constexpr bool kShiftFirst = kS == 4 && MODE == kEstepFused;
     constexpr int kFlush = 32 / kS;     /* tiles summed in FP32 registers (32 samples) */
@@ -280,7 +302,7 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
      * (the padding rows of W and entries of W c are zero, and x's padding
      * columns are written as zero), so every load is unconditional and the
      * wait for a prefetch can sit where its value is first used. */
-    float bn[kS];
+    float bn[kS], xn[kXAhead ? kS : 1];
     double bn64[B64 ? kS : 1];
     /* b and x through buffer resources based at row t0: the lane's byte
      * offset is fixed, the row's a scalar (launch_estep bounds it below
@@ -308,6 +330,8 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
             bn64[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rb, vob, r * browb, 0));
         else
             bn[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, vob, r * browb, 0));
+        if constexpr (kXAhead && MODE != kEstepLsum)
+            xn[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, vox, r * xrowb, 0));
     };
 #pragma unroll
     for (int s = 0; s < kS; ++s) load_tile(t0 + s, s);
@@ -327,22 +351,23 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
 #pragma unroll
         for (int sub = 0; sub < kTPG; ++sub) {
             const long tb = tg + sub * kS;
-            /* kept per component and sample: |y|^(rho-2), log2|y|, 2^Q and, where
-             * it is formed in FP64, y (sy and |y|^rho are one product each away) */
-            float E[kS][MJ], Y[kS][MJ], YM2[kS][MJ], LA[kS][MJ];
+            /* kept per component and sample: |y|^(rho-2), log2|y|, 2^Q, where it
+             * is formed in FP64 y, and with kKeep sy and |y|^rho */
+            float E[kS][MJ], Y[kS][MJ], YM2[kS][MJ], LA[kS][MJ], SY[kKeep ? kS : 1][MJ], YR[kKeep ? kS : 1][MJ];
             float RS[kS], BV[kS], XV[kS], SE[kS];
             double BV64[B64 ? kS : 1];
 #pragma unroll
             for (int s = 0; s < kS; ++s) {
                 if constexpr (B64) { BV64[s] = bn64[s]; BV[s] = (float)bn64[s]; }
                 else BV[s] = bn[s];
+                if constexpr (kXAhead && MODE != kEstepLsum) XV[s] = xn[s];
             }
-            /* issue the next tile's b loads and this one's x loads (first
-             * used after the exchange) now; they complete under this tile's
-             * math.  Rows past t1 are read without a check (the next range's
+            /* issue the next tile's b loads and, unless they were ahead too,
+             * this one's x loads (first used after the exchange) now; they
+             * complete under this tile's math.  Rows past t1 are read without a check (the next range's
              * samples, or the kEstepRowPad zero rows after the last one) and
              * get posterior 0. */
-            if constexpr (MODE != kEstepLsum) {
+            if constexpr (!kXAhead && MODE != kEstepLsum) {
 #pragma unroll
                 for (int s = 0; s < kS; ++s)
                     XV[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
@@ -435,6 +460,7 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                     E[s][j] = fast_exp2(fmaf(yr, -AMICA_L2E, cq2[j]));
                     SE[s] = j == 0 ? E[s][j] : SE[s] + E[s][j];
                     Y[s][j] = y; YM2[s][j] = ym2; LA[s][j] = la;
+                    if constexpr (kKeep) { SY[s][j] = ym2 * y; YR[s][j] = yr; }
                 }
                 QS[s] = fast_log2(SE[s]);         /* exactly 0 on padding channels */
             }
@@ -511,7 +537,12 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                 /* the other waves wait for this one at the next barrier: let it
                  * issue ahead of the other workgroup's waves on its SIMD */
                 __builtin_amdgcn_s_setprio(3);
-                const int s = min(lane >> 4, kS - 1), hh = lane & (kRow16 ? 15 : 7);
+                /* two-sample tiles for m <= 3 use all four rows, the pairs in
+                 * turn: vsum and the LL sum then add up in the order they have
+                 * with tiles of four, to the last bit */
+                constexpr bool kPairs = kS == 2 && MJ <= 3;
+                const int row = lane >> 4, hh = lane & (kRow16 ? 15 : 7);
+                const int s = kPairs ? row & 1 : min(row, kS - 1);
                 float l = -3.0e38f;
                 if (hh < a.M) {
                     l = dc2[hh];
@@ -534,7 +565,7 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                 esum += dpp<0x122, 0xf, 0xf, false>(esum);
                 esum += dpp<0x124, 0xf, 0xf, false>(esum);
                 if constexpr (kRow16) esum += dpp<0x128, 0xf, 0xf, false>(esum);
-                const bool mine = (lane & 8) == 0 && (lane >> 4) < kS, valid = s < nval;
+                const bool mine = (lane & 8) == 0 && (kPairs ? row >> 1 == (sub & 1) : row < kS), valid = s < nval;
                 const float vl = valid ? e * fast_rcp(esum) : 0.f;
                 if (mine) Vp[buf][hh][s] = vl;
                 if (mine && valid && hh < a.M) {
@@ -561,8 +592,15 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
 #pragma unroll
                 for (int j = 0; j < MJ; ++j) {
                     float u = E[s][j] * vrs;
-                    const float yv = kRecY ? fmaf(sb[j], BV[s], nsbmu[j]) : Y[s][j];
-                    const float sy = YM2[s][j] * yv, yr = sy * yv;
+                    float sy, yr;
+                    if constexpr (kKeep) {
+                        sy = SY[s][j];
+                        yr = YR[s][j];
+                    } else {
+                        const float yv = kRecY ? fmaf(sb[j], BV[s], nsbmu[j]) : Y[s][j];
+                        sy = YM2[s][j] * yv;
+                        yr = sy * yv;
+                    }
                     float uf = u * sy;
                     /* two of the sums round u and u f before they add them (the
                      * empty asm), or take the products into an FMA: which one is
@@ -589,9 +627,11 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
                 /* one sample at a time: the sums are complete here (empty asm
                  * with them as operands, no instruction), or the compiler would
                  * keep several samples' products live, beyond 128 VGPRs */
+                if constexpr (!kKeep) {
 #pragma unroll
-                for (int q = 0; q < NS; ++q) __asm__ volatile("" : "+v"(acc[q]));
-                __builtin_amdgcn_sched_barrier(0);
+                    for (int q = 0; q < NS; ++q) __asm__ volatile("" : "+v"(acc[q]));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
             if constexpr (!GB) {
                 if (wreal)
@@ -656,6 +696,12 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
         const double ls = wave_sum_f64(ll_acc);
         if (lane == 0) base[tail + a.M] = ls;
     }
+}
+
+/* the kernel of a launch, by the workgroup's waves (fused: up to kSmallWaves; 5 to 7) */
+template <int MJ, bool B64, int MODE, bool GB, bool SMALL = false, bool MID = false>
+constexpr auto estep_variant() {
+    return &estep_kernel<MJ, B64, MODE, GB, estep_tile_samples(MJ, B64, SMALL), estep_keeps(MJ, B64, MODE, GB, MID)>;
 }
 
 /* 4 x 4 transpose between the registers r[0..3] and the four rows of 16 lanes */
@@ -1111,12 +1157,14 @@ int estep_configure(int MJ, size_t lds_bytes) {
     hipError_t r = hipSuccess;
 #define AMICA_ESTEP_ATTR(J)                                                                       \
     case J:                                                                                       \
-        for (const void* fn : {(const void*)estep_kernel<J, true, kEstepFused, false>,            \
-                               (const void*)estep_kernel<J, false, kEstepFused, false>,           \
-                               (const void*)estep_kernel<J, false, kEstepFused, true>,            \
-                               (const void*)estep_kernel<J, true, kEstepStats, false>,            \
-                               (const void*)estep_kernel<J, false, kEstepStats, false>,           \
-                               (const void*)estep_kernel<J, false, kEstepStats, true>})           \
+        for (const void* fn : {(const void*)estep_variant<J, true, kEstepFused, false, true>(),   \
+                               (const void*)estep_variant<J, true, kEstepFused, false>(),         \
+                               (const void*)estep_variant<J, false, kEstepFused, false, false, true>(), \
+                               (const void*)estep_variant<J, false, kEstepFused, false>(),        \
+                               (const void*)estep_variant<J, false, kEstepFused, true>(),         \
+                               (const void*)estep_variant<J, true, kEstepStats, false>(),         \
+                               (const void*)estep_variant<J, false, kEstepStats, false>(),        \
+                               (const void*)estep_variant<J, false, kEstepStats, true>()})        \
             if (r == hipSuccess)                                                                  \
                 r = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,           \
                                         (int)lds_bytes);                                          \
@@ -1206,12 +1254,12 @@ static int launch_estep_split(const EstepArgs& a, int MJ, int nblocks, hipStream
     const bool b64 = a.b64 != nullptr;
 #define AMICA_ESTEP_SPLIT(J)                                                                          \
     case J:                                                                                           \
-        if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepLsum, false>), grid, block, 0, st, a); \
-        else hipLaunchKernelGGL((estep_kernel<J, false, kEstepLsum, false>), grid, block, 0, st, a);  \
+        if (b64) hipLaunchKernelGGL((estep_variant<J, true, kEstepLsum, false>()), grid, block, 0, st, a); \
+        else hipLaunchKernelGGL((estep_variant<J, false, kEstepLsum, false>()), grid, block, 0, st, a); \
         hipLaunchKernelGGL(estep_post_kernel, dim3(nblocks), dim3(256), 0, st, a);                   \
-        if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepStats, false>), grid, block, shm, st, a); \
-        else if (a.g_bf16) hipLaunchKernelGGL((estep_kernel<J, false, kEstepStats, true>), grid, block, shm, st, a); \
-        else hipLaunchKernelGGL((estep_kernel<J, false, kEstepStats, false>), grid, block, shm, st, a); \
+        if (b64) hipLaunchKernelGGL((estep_variant<J, true, kEstepStats, false>()), grid, block, shm, st, a); \
+        else if (a.g_bf16) hipLaunchKernelGGL((estep_variant<J, false, kEstepStats, true>()), grid, block, shm, st, a); \
+        else hipLaunchKernelGGL((estep_variant<J, false, kEstepStats, false>()), grid, block, shm, st, a); \
         break;
     switch (MJ) {
         AMICA_ESTEP_SPLIT(1)
@@ -1282,15 +1330,20 @@ int launch_estep(const EstepArgs& a, int MJ, int nblocks, int cus, hipStream_t s
         else hipLaunchKernelGGL((estep_m1_unmix_kernel<3>), ug, ub, us, st, a, nblocks, nw);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
+    const int waves = (int)block.x / 64;
+    const bool small = waves <= kSmallWaves, mid = waves > 4 && waves < 8;
 #define AMICA_ESTEP_CASE(J)                                                                   \
     case J:                                                                                   \
         if (m1) {                                                                             \
             if (b64) hipLaunchKernelGGL((estep_m1_kernel<J, true>), grid, block, shm, st, a); \
             else hipLaunchKernelGGL((estep_m1_kernel<J, false>), grid, block, shm, st, a);    \
         } else {                                                                              \
-            if (b64) hipLaunchKernelGGL((estep_kernel<J, true, kEstepFused, false>), grid, block, shm, st, a); \
-            else if (a.g_bf16) hipLaunchKernelGGL((estep_kernel<J, false, kEstepFused, true>), grid, block, shm, st, a); \
-            else hipLaunchKernelGGL((estep_kernel<J, false, kEstepFused, false>), grid, block, shm, st, a); \
+            hipLaunchKernelGGL((b64 && small ? estep_variant<J, true, kEstepFused, false, true>()             \
+                                : b64        ? estep_variant<J, true, kEstepFused, false>()                   \
+                                : a.g_bf16   ? estep_variant<J, false, kEstepFused, true>()                   \
+                                : mid        ? estep_variant<J, false, kEstepFused, false, false, true>()     \
+                                             : estep_variant<J, false, kEstepFused, false>()),                \
+                               grid, block, shm, st, a);                                      \
         }                                                                                     \
         break;
     switch (MJ) {
