@@ -868,7 +868,7 @@ int run_chunks(AdjArgs a, const void* x, long T, const double* dll, double* ll, 
      * the unpadded rows (row stride n) on the FP64 one */
     const bool gx32 = rb == 4;
     const int slabs = (ldb / 64) * ((n + 63) / 64);
-    const GxChunks gc32 = gx32 ? gx_f32_chunks(Tc, NP, ldb, cus) : GxChunks{0, 0, 1};
+    const GxChunks gc32 = gx32 ? gx_f32_chunks(Tc, NP, ldb, cus, cus) : GxChunks{0, 0, 1, 0, 2};
     const int gchunks = gx32 ? gc32.n
                              : (int)std::max(1L, std::min(std::max(1L, 2L * cus / slabs), (Tc + 255) / 256));
     const int gxs = gx32 ? NP : n;
@@ -933,8 +933,9 @@ int run_chunks(AdjArgs a, const void* x, long T, const double* dll, double* ll, 
         if (!adj) continue;
         int gc = gchunks;
         if constexpr (rb == 4) {
-            gc = (int)((Tn + gc32.chunk - 1) / gc32.chunk) * gc32.spread;
-            if (launch_gx_f32((const float*)a.g, xp, gxpart, Tn, NP, ldb, GxChunks{gc, gc32.chunk, gc32.spread}, st))
+            GxChunks last = gc32;
+            last.n = gc = (int)((Tn + gc32.chunk - 1) / gc32.chunk) * gc32.spread;
+            if (launch_gx_f32((const float*)a.g, xp, gxpart, Tn, NP, ldb, last, st))
                 return report_error(AMICA_E_DEVICE, "statistic GEMM launch failed");
         } else {
             const long gch = ((Tn + gchunks - 1) / gchunks + 31) / 32 * 32;

@@ -112,7 +112,7 @@ struct amica_engine {
     size_t pstride = 0;
     double* part = nullptr;
     int nchunks = 0;
-    GxChunks gx = {0, 0, 1};          /* FP32 statistic GEMM */
+    GxChunks gx = {0, 0, 1, 0, 2};    /* FP32 statistic GEMM */
     double* gxpart = nullptr;
     double* raw = nullptr;
     double* sumtmp = nullptr;      /* first-pass group sums of the partials */
@@ -169,7 +169,7 @@ struct amica_engine {
         chunk = (T + nblocks - 1) / nblocks;
         chunk = ((chunk + 31) / 32) * 32;     /* whole packed 8-sample groups */
         nblocks = (int)((T + chunk - 1) / chunk);
-        if (!bf16) gx = gx_f32_chunks(T, NP, ldb, cu_budget);
+        if (!bf16) gx = gx_f32_chunks(T, NP, ldb, cu_budget, cus);
         nchunks = bf16 ? gx_bf16_chunks(T, NP, ldb, cu_budget) : gx.n;
         if (gexec) {   /* the captured grids are stale */
             (void)hipGraphExecDestroy(gexec);

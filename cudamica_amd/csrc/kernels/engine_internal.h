@@ -158,6 +158,8 @@ struct GxChunks {
     int n;          /* partials */
     long chunk;     /* samples of `spread` consecutive ones */
     int spread;
+    int grouped;    /* a workgroup's 8 waves share a chunk (narrow g) */
+    int depth;      /* steps of loads a wave has in flight */
 };
 int launch_gx_f32(const float* g, const float* x, double* part, long T, int NP, int ldb, const GxChunks& c,
                   hipStream_t st);
@@ -166,9 +168,10 @@ int launch_gx_f32(const float* g, const float* x, double* part, long T, int NP, 
 int launch_gx_bf16(const uint16_t* g8, const uint16_t* x8, double* part, long T, int NP, int ldb,
                    int nchunks, hipStream_t st);
 /* Sample chunks (partials) launch_gx_bf16 / launch_gx_f32 should be given for
- * a budget of `cus` CUs (their number is nondecreasing in cus). */
+ * a budget of `cus` CUs (their number is nondecreasing in cus) of a device of
+ * `all`. */
 int gx_bf16_chunks(long T, int NP, int ldb, int cus);
-GxChunks gx_f32_chunks(long T, int NP, int ldb, int cus);
+GxChunks gx_f32_chunks(long T, int NP, int ldb, int cus, int all);
 /* x8[(t/8) NP + i][t%8] = xhi[t][i] (the packed B operand of the BF16
  * statistic GEMM); padding stays as allocated (zero). */
 int launch_pack8(const uint16_t* xhi, long T, int NP, uint16_t* x8, hipStream_t st);

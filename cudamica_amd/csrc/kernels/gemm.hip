@@ -670,14 +670,16 @@ __global__ __launch_bounds__(256) void unmix_f32_kernel(const float* __restrict_
 }
 
 /* ---------------- statistic GEMM G = g^T x, FP32 --------------------- */
+/* waves per SIMD that the kernel's registers leave with D steps of loads in flight */
+constexpr int gx_f32_waves(int CT, int D) { return CT == 8 ? (D == 1 ? 3 : 2) : CT == 4 ? (D == 1 ? 5 : D == 2 ? 4 : 3) : 4; }
 /* FP32 statistic GEMM in slabs: workgroup = ldb/64 waves over one chunk of
  * samples (at most a few thousand, so the FP32 accumulation inside the MFMA
  * stays short); wave w owns g rows [64w, 64w+64) x the 16 CT x columns of
  * slab blockIdx.y, 4 CT accumulators of v_mfma_f32_16x16x4f32; every g
  * element is read once per slab, x once per workgroup (the other waves hit
- * the caches), each lane's operands of one sample in 16-byte loads, two
- * steps in flight (128 ch x 2M x 4 models: 2.97 -> 2.83 ms against one,
- * 3.5 ms with three; bound by the FP32 MFMA rate, 62 % of 157 TFLOP/s).  FP64
+ * the caches), each lane's operands of one sample in 16-byte loads, D
+ * steps in flight (gx_f32_chunks; 128 ch x 2M x 4 models: 2.97 ms with one,
+ * 2.83 with two, 3.5 with three; bound by the FP32 MFMA rate, 62 % of 157 TFLOP/s).  FP64
  * partial per chunk.  Where g has fewer than 512 columns (rw = ldb/64 row
  * waves), a workgroup of 8 waves runs S = 8 / rw sub-ranges of its chunk
  * side by side and adds their totals in FP64 through LDS in a fixed order, a
@@ -685,11 +687,11 @@ __global__ __launch_bounds__(256) void unmix_f32_kernel(const float* __restrict_
  * one partial is written (128 ch x 500k x 2 models: 440 -> 406 us and, with
  * half the partials, reductions 122 -> 91 us). */
 template <int CT, int D>
-__global__ __launch_bounds__(512) void gx_f32_slab_kernel(const float* __restrict__ g,
+__global__ __launch_bounds__(512, gx_f32_waves(CT, D)) void gx_f32_slab_kernel(const float* __restrict__ g,
                                                           const float* __restrict__ x,
                                                           double* __restrict__ part, long T,
                                                           int NP, int ldb, long chunk, int spread) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rw = min(ldb - (int)blockIdx.z * 512, 512) / 64;   /* row waves */
     /* sample sub-ranges: only below 512 columns, where the launch gives 8
      * waves for fewer row waves and the LDS tile with them.  spread > 1: the
@@ -1161,7 +1163,7 @@ static size_t gx_f32_split_lds(int NP, int ldb) {
 
 static bool gx_f32_split(int ldb) { return ldb < 512 && 8 % (ldb / 64) == 0; }
 
-GxChunks gx_f32_chunks(long T, int NP, int ldb, int cus) {
+GxChunks gx_f32_chunks(long T, int NP, int ldb, int cus, int all) {
     /* The FP32 accumulation ranges, one per wave: for 128 columns of 64 inputs
      * and fewer, chunks of >= 2048 (one model) or 1024 samples whose S waves
      * take a share each, else chunks of >= 512 samples; at most 256 MB of
@@ -1173,18 +1175,54 @@ GxChunks gx_f32_chunks(long T, int NP, int ldb, int cus) {
     const long by_mem = std::max(1L, (256L << 20) / ((long)ldb * NP * 8));
     const long want = std::max(1L, (long)cus / (NP / (16 * gx_f32_ct(NP))));
     const long n = std::max(1L, std::min(by_len, std::max(want, by_mem)));
+    const int CT = gx_f32_ct(NP), slabs = NP / (16 * CT), rw = std::min(ldb, 512) / 64;
     GxChunks c;
     c.chunk = gx_chunk(T, (int)n, 4);
-    /* other widths below 512 columns: S such ranges in one workgroup, whose
-     * totals meet in LDS: S times fewer partials */
-    if (!shared && S > 1) c.chunk *= S;
     c.n = (int)((T + c.chunk - 1) / c.chunk);
+    c.spread = 1;
+    c.grouped = S > 1;
+    c.depth = CT == 8 || c.n >= 256 ? 2 : 4;
+    if (S > 1 && !shared) {
+        /* other widths below 512 columns: S such ranges in one workgroup of 8
+         * waves, whose totals meet in LDS: S times fewer partials.  But a range
+         * to a workgroup of its own where those leave every CU one at most
+         * (128 ch x 75k x 2 models, GEMM and reductions: 215 -> 167 us), or
+         * where the ranges' waves fit the GPU at once with one step of loads in
+         * flight and its fewer registers, and not with two: the workgroups of 8
+         * would start a second time for a few of them (128 ch x 300k x 2 models
+         * 444 -> 337 us, 100 ch x 600k 434 -> 341, 64 ch x 600k x 4 models
+         * 348 -> 307).  The decision is the device's, not the budget's, so that
+         * a budget never asks for more partials than the whole device. */
+        const long waves = (long)c.n * rw * slabs, simds = 4L * all;
+        const bool once = waves > simds * gx_f32_waves(CT, 2) && waves <= simds * gx_f32_waves(CT, 1);
+        const long grouped = (c.n + S - 1) / S;
+        if (grouped >= 64 && (once || (CT == 8 && (long)c.n * slabs <= all))) {
+            c.grouped = 0;
+            c.depth = once ? 1 : 2;
+            return c;
+        }
+        c.chunk *= S;
+        c.n = (int)((T + c.chunk - 1) / c.chunk);
+        c.depth = CT == 8 || c.n >= 256 ? 2 : 4;
+    }
     /* Where that leaves most of the GPU idle, a chunk's ranges go to
      * workgroups of their own, 16 columns of x to each (the sums inside a range
      * are the same): 16 ch x 20k samples ran 10 workgroups of 8 waves, 62 us;
      * 316 of one wave take 16 us. */
     c.spread = S > 1 && c.n < 64 ? S : 1;
     c.n *= c.spread;
+    /* Widths that do not divide 8: more steps in flight pay while the waves they
+     * leave room for (12, 16 or 20 a CU) hold every workgroup at once.  Three
+     * waves: four steps hold four workgroups a CU, two steps five, one step six
+     * (64 ch x 300k x 3 models, GEMM and reductions 198 -> 177 us, 700k 326 ->
+     * 293); past four, one step where that saves a round.  Five waves put two on one SIMD, so that four steps hold one
+     * workgroup a CU, two steps two and one step three: 320 ch x 300k 1043 ->
+     * 986 us, 64 ch x 500k x 5 models 434 -> 372. */
+    if (CT == 4 && S == 1 && (rw == 3 || rw == 5)) {
+        const long per_cu = ((long)c.n * slabs + all - 1) / all;
+        if (rw == 3) c.depth = per_cu <= 4 ? 4 : (per_cu + 5) / 6 < (per_cu + 4) / 5 ? 1 : 2;
+        else c.depth = per_cu <= 1 ? 4 : per_cu == 2 ? 2 : 1;
+    }
     return c;
 }
 
@@ -1198,15 +1236,19 @@ int launch_gx_f32(const float* g, const float* x, double* part, long T, int NP, 
     }
     const int CT = gx_f32_ct(NP);
     dim3 grid(c.n, NP / (16 * CT), (ldb + 511) / 512), block(std::min(ldb, 512));
-    const bool split = gx_f32_split(ldb);
-    if (split) block = dim3(512);
-    const size_t shm = split ? gx_f32_split_lds(NP, ldb) : 0;
-    if (CT == 8)
-        hipLaunchKernelGGL((gx_f32_slab_kernel<8, 2>), grid, block, shm, st, g, x, part, T, NP, ldb, c.chunk, 1);
-    else if (c.n < 256)   /* less than a workgroup per CU: more of a wave's loads in flight */
-        hipLaunchKernelGGL((gx_f32_slab_kernel<4, 4>), grid, block, shm, st, g, x, part, T, NP, ldb, c.chunk, 1);
-    else
-        hipLaunchKernelGGL((gx_f32_slab_kernel<4, 2>), grid, block, shm, st, g, x, part, T, NP, ldb, c.chunk, 1);
+    if (c.grouped && !gx_f32_split(ldb)) return -1;
+    if (c.grouped) block = dim3(512);
+    const size_t shm = c.grouped ? gx_f32_split_lds(NP, ldb) : 0;
+#define AMICA_GX_CASE(CT_, D_)                                                                              \
+    if (CT == CT_ && c.depth == D_)                                                                         \
+        hipLaunchKernelGGL((gx_f32_slab_kernel<CT_, D_>), grid, block, shm, st, g, x, part, T, NP, ldb, c.chunk, 1);
+    AMICA_GX_CASE(8, 2)
+    else AMICA_GX_CASE(8, 1)
+    else AMICA_GX_CASE(4, 4)
+    else AMICA_GX_CASE(4, 2)
+    else AMICA_GX_CASE(4, 1)
+    else return -1;
+#undef AMICA_GX_CASE
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
