@@ -143,10 +143,10 @@ template <> struct Base<double> {
 
 /* Samples per tile, held in registers between the densities and the gradient
  * sums (4 values per component and sample on the adjoint), about what 256 VGPRs
- * hold.  The adjoint goes past them into scratch memory at m = 3, 5, 7 and 8 in
- * FP64 (several models: 80 to 224 bytes a lane; one: 36 to 96 at m = 3, 5, 8)
- * and m = 5, 7 and 8 in FP32 (56 to 196; one: 92 at m = 8, where the split pass
- * takes 20).  In FP32 at m = 3, which fits, tiles of two took 14.9 ms a call
+ * hold.  The adjoint goes past them into scratch memory in FP64 at m = 3, 5, 7
+ * and 8 (several models: 84 to 216 bytes a lane; one: 52 and 60 at m = 5 and 8)
+ * and in FP32 at m = 5, 7 and 8 (56 to 196; one: 92 at m = 8, where the split
+ * pass takes 20).  In FP32 at m = 3, which fits, tiles of two took 14.9 ms a call
  * where these take 13.4 (128 ch x 2M x 4 models); smaller tiles where it spills
  * have not been timed. */
 template <typename Real, int MJ, bool ADJ> constexpr int tile_samples() {

@@ -179,9 +179,11 @@ constexpr bool estep_keeps(int MJ, bool B64, int mode, bool GB, bool mid) {
  *   kEstepStats  split launch, last pass: the densities again, the model
  *                posteriors read from vq (written between the passes by
  *                estep_post_kernel), then the statistics and g. */
-template <int MJ, bool B64, int MODE, bool GB, int kS, bool kKeep>
+template <int MJ, bool B64, int MODE, bool GB, int kS, bool kKeep, bool kThree>
 __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
     static_assert(8 % kS == 0 && 7 + kS <= kEstepRowPad, "the unchecked loads past a range stay in the padding rows");
+    /* a register past the 128 that four waves per SIMD leave: three then */
+    if constexpr (kThree) __asm__ volatile("" ::: "v130");
     static_assert(!kKeep || kS == 1, "larger tiles have no registers to keep more");
     constexpr bool kRecY = !B64 && !kKeep;
     /* a tile of four samples is long enough for its own x to arrive behind its
@@ -698,10 +700,16 @@ __global__ __launch_bounds__(512) void estep_kernel(EstepArgs a) {
     }
 }
 
-/* the kernel of a launch, by the workgroup's waves (fused: up to kSmallWaves; 5 to 7) */
-template <int MJ, bool B64, int MODE, bool GB, bool SMALL = false, bool MID = false>
+/* the kernel of a launch, by the workgroup's waves (fused: 2; up to
+ * kSmallWaves; 5 to 7).  With FP64 b at m = 4 it takes 126 VGPRs, four waves per
+ * SIMD, but the sample ranges are cut for three (estep_blocks_per_cu).  Workgroups
+ * of two waves then crowd some SIMDs; held to three they spread evenly (E-step
+ * of 64 ch x 2 models 1.10 times the time otherwise); larger ones use the room
+ * (64 ch x 3 models 0.75 times). */
+template <int MJ, bool B64, int MODE, bool GB, bool SMALL = false, bool MID = false, bool TWO = false>
 constexpr auto estep_variant() {
-    return &estep_kernel<MJ, B64, MODE, GB, estep_tile_samples(MJ, B64, SMALL), estep_keeps(MJ, B64, MODE, GB, MID)>;
+    return &estep_kernel<MJ, B64, MODE, GB, estep_tile_samples(MJ, B64, SMALL), estep_keeps(MJ, B64, MODE, GB, MID),
+                         TWO && MJ == 4 && B64>;
 }
 
 /* 4 x 4 transpose between the registers r[0..3] and the four rows of 16 lanes */
@@ -1157,7 +1165,8 @@ int estep_configure(int MJ, size_t lds_bytes) {
     hipError_t r = hipSuccess;
 #define AMICA_ESTEP_ATTR(J)                                                                       \
     case J:                                                                                       \
-        for (const void* fn : {(const void*)estep_variant<J, true, kEstepFused, false, true>(),   \
+        for (const void* fn : {(const void*)estep_variant<J, true, kEstepFused, false, true, false, true>(), \
+                               (const void*)estep_variant<J, true, kEstepFused, false, true>(),   \
                                (const void*)estep_variant<J, true, kEstepFused, false>(),         \
                                (const void*)estep_variant<J, false, kEstepFused, false, false, true>(), \
                                (const void*)estep_variant<J, false, kEstepFused, false>(),        \
@@ -1338,7 +1347,8 @@ int launch_estep(const EstepArgs& a, int MJ, int nblocks, int cus, hipStream_t s
             if (b64) hipLaunchKernelGGL((estep_m1_kernel<J, true>), grid, block, shm, st, a); \
             else hipLaunchKernelGGL((estep_m1_kernel<J, false>), grid, block, shm, st, a);    \
         } else {                                                                              \
-            hipLaunchKernelGGL((b64 && small ? estep_variant<J, true, kEstepFused, false, true>()             \
+            hipLaunchKernelGGL((b64 && waves == 2 ? estep_variant<J, true, kEstepFused, false, true, false, true>() \
+                                : b64 && small ? estep_variant<J, true, kEstepFused, false, true>()           \
                                 : b64        ? estep_variant<J, true, kEstepFused, false>()                   \
                                 : a.g_bf16   ? estep_variant<J, false, kEstepFused, true>()                   \
                                 : mid        ? estep_variant<J, false, kEstepFused, false, false, true>()     \
