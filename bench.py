@@ -13,14 +13,15 @@ Prints one JSON line.  Fields beyond the driver's contract:
                 around it on the engine stream during the timed steps; also
                 against the bandwidth of this library's own streaming copy
                 kernel (amica_hbm_probe)
-  valu          the E-step's VALU-issue bound (the one it runs against): SIMD
-                cycles its VALU instructions occupy per launch (rocprofv3
-                SQ_ACTIVE_INST_VALU x 4, from profiles/valu_<workload>_<prec>.json)
-                over the SIMD cycles of 1024 SIMDs at the 2400 MHz maximum engine
-                clock during the live average launch time; frac_under_counters
-                uses the cycles the counter run itself counted (GRBM_GUI_ACTIVE)
+  valu          the E-step's vector-ALU load: VALU instructions per launch (and
+                the transcendentals among them) from rocprofv3 counters of the
+                same kernel kept in profiles/sq_<workload>_<prec>.json, their
+                rate over the live average launch time, and the SIMD cycles that
+                1024 SIMDs offer per instruction in that time at the 2400 MHz
+                maximum engine clock; null where the profile is of another kernel
   gemm          algorithmic GEMM FLOPs (4 M n^2 T) over the two GEMMs' time,
-                against the dense MFMA peak of their operand type
+                against the dense MFMA peak of their operand type; where the
+                E-step forms b itself, the statistic GEMM alone (2 M n^2 T, FP32)
   cpu_baseline  the FP64 CPU oracle (C++, OpenMP on all host cores) on the
                 whole recording, 2 iterations (median), with its FP32
                 variant beside it
@@ -347,22 +348,54 @@ def copy_probe(mib):
     log(f"copy probe: memset + copy of {mib} MiB")
 
 
-def measured_traffic(workload, prec):
-    """HBM bytes per E-step launch measured with rocprofv3 --pmc FETCH_SIZE and
-    WRITE_SIZE passes (scaled by the copy probe), kept in profiles/ as JSON."""
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
-                        f"traffic_{workload}_{PREC_NAME[prec]}.json")
+def estep_kernel(n, M, m, prec):
+    """The start of the name of the E-step kernel an engine of these shapes launches."""
+    blocks = M * ((n + 63) // 64)
+    if M == 1 and blocks <= 8:
+        if prec == 32 and n <= 64 and m <= 3:
+            return f"estep_m1_unmix_kernel<{m}>"
+        return f"estep_m1_kernel<{m}, {str(prec == 32).lower()}>"
+    return f"estep_kernel<{m}, {str(prec == 32).lower()}, {0 if blocks <= 8 else 2}, {str(prec in (16, 8)).lower()}, "
+
+
+def _profile(kind, workload, prec, kernel):
+    """profiles/<kind>_<workload>_<prec>.json, or None where there is none or it is of another kernel."""
+    path = os.path.join(ROOT, "profiles", f"{kind}_{workload}_{PREC_NAME[prec]}.json")
     if not os.path.exists(path):
         return None
     with open(path) as f:
-        return json.load(f).get("traffic_bytes")
+        d = json.load(f)
+    return d if d["kernel"].startswith(kernel) else None
+
+
+def measured_traffic(workload, prec, kernel):
+    """HBM bytes per E-step launch measured with rocprofv3 --pmc FETCH_SIZE and
+    WRITE_SIZE passes (scaled by the copy probe), kept in profiles/ as JSON."""
+    d = _profile("traffic", workload, prec, kernel)
+    return d and d["traffic_bytes"]
+
+
+def valu_rate(workload, prec, kernel, avg_ms):
+    """VALU instructions per launch of the profiled E-step kernel, and their rate
+    over the live average launch time."""
+    d = _profile("sq", workload, prec, kernel)
+    if d is None:
+        return None
+    c = d["counters"]
+    insts = c["SQ_INSTS_VALU"]
+    cycles = d["simds"] * d["max_engine_clock_mhz"] * 1e3 * avg_ms
+    return {"kernel": d["kernel"], "valu_insts_per_launch": insts,
+            "transcendental_insts_per_launch": c.get("SQ_INSTS_VALU_TRANS_F32"),
+            "achieved": insts / avg_ms / 1e6, "unit": "G instructions/s",
+            "simd_cycles_per_inst": cycles / insts}
 
 
 def valu_roofline(workload, prec, avg_ms):
-    """The E-step's VALU-issue bound: the SIMD cycles its VALU instructions
-    occupy per launch (rocprofv3 SQ_ACTIVE_INST_VALU quad-cycles x 4, kept in
-    profiles/ as JSON) over the SIMD cycles the GPU offers at its maximum
-    engine clock during the live average launch time."""
+    """SQ_ACTIVE_INST_VALU quad-cycles x 4 of the counters in profiles/valu_*.json
+    over the SIMD cycles the GPU offers at its maximum engine clock during a
+    launch of avg_ms.  Those are of the E-step with two-sample tiles; the
+    factor of 4 is too large for FP32 instructions (the present kernel's counters
+    give 102 %), so the printed line states instructions instead (valu_rate)."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
                         f"valu_{workload}_{PREC_NAME[prec]}.json")
     if not os.path.exists(path):
@@ -526,9 +559,12 @@ def main():
     nbytes = estep_bytes(n, T, M, prec)
     achieved = nbytes / (kms[2] * 1e-3) / 1e9
     hbm, hbm_read = measured_hbm_gbs()
+    kernel = estep_kernel(n, M, m, prec)
     gemm_flop = 4.0 * M * n * n * T          # GEMM1 + GEMM2, algorithmic
     gemm_s = (kms[1] + kms[3]) * 1e-3
     gemm_peak = GEMM_PEAK_TFLOPS[prec]
+    if kernel.startswith("estep_m1_unmix"):  # GEMM1 is part of the E-step
+        gemm_flop, gemm_s, gemm_peak = gemm_flop / 2, kms[3] * 1e-3, GEMM_PEAK_TFLOPS[33]
     out = {
         "metric": METRIC,
         "value": its,
@@ -546,12 +582,12 @@ def main():
                    "precision": PREC_NAME[prec], "parallelism": "single-gpu",
                    **({"cu_budget": args.cu_budget} if args.cu_budget else {})},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(w.name, prec),
-                     "kernel": "estep_kernel", "bytes_per_launch": nbytes,
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(w.name, prec, kernel),
+                     "kernel": kernel.split("<")[0], "bytes_per_launch": nbytes,
                      "avg_ms": kms[2], "launches": cnt,
                      "measured_copy_gbs": hbm, "measured_read_gbs": hbm_read,
                      "frac_of_measured": achieved / hbm if hbm else None},
-        "valu": valu_roofline(w.name, prec, kms[2]),
+        "valu": valu_rate(w.name, prec, kernel, kms[2]),
         "gemm": {"flop_per_iter": gemm_flop, "ms": gemm_s * 1e3,
                  "tflops": gemm_flop / gemm_s / 1e12,
                  "peak_tflops": gemm_peak, "mfma_frac": gemm_flop / gemm_s / 1e12 / gemm_peak},
