@@ -1025,9 +1025,9 @@ __global__ __launch_bounds__(512) void estep_m1_kernel(EstepArgs a) {
  * separate unmixing and E-step (x read and b written; b and x read, g
  * written), which are bound by HBM at 4.3-5 TB/s.  W's fragments and the FP64
  * constants are in LDS, once for the workgroup's waves, which share nothing else
- * (a range of samples each).  What bounds it is issue on the SIMDs: 59 % of
- * the cycles the vector ALU (101 instructions a sample at m = 3), 32 % the FP64
- * MFMAs, which do not run beside it; the next tile's x loaded ahead and wave
+ * (a range of samples each).  What bounds it is issue on the SIMDs: up to 55 %
+ * of the cycles the vector ALU (99 instructions a sample at m = 3), 31 % the FP64
+ * MFMAs, one after the other in a wave; the next tile's x loaded ahead and wave
  * priorities by phase changed nothing.  64 ch x 1M, us, unmixing and E-step
  * together: m = 1 436 -> 355, m = 2 440 -> 332, m = 3 482 -> 400; 16 ch x 20k 35
  * -> 32; 40 ch x 5k 28 and 28.  For m > 3 the kernel needs more than 128 VGPRs,
